@@ -230,6 +230,10 @@ struct PathQueues {
   // queues
   uint32_t *queue_a, *queue_b, *shadow_queue;
   uint32_t *counters;   // [0] queue_a count, [1] queue_b count, [2] shadow count, [3..] stats
+  // Lengths of the shadow queue: of the rays the previous shade launch queued (which the trace
+  // launch takes) and of those this iteration's shade launch queues.  Slot-ordered queues
+  // alternate between two counters, so that none is cleared between two launches.
+  uint32_t *shadow_in, *shadow_out;
   // path regeneration: slots of the paths finished in the current iteration, and the pass's
   // progress ([0] camera paths issued so far, [1] paths queued for the next iteration)
   uint32_t *free_slots;
@@ -273,7 +277,24 @@ enum FlagBits : uint32_t {
 
 enum Counter {
   kCountA = 0, kCountB = 1, kCountShadow = 2, kCountRecords = 3, kStatClosest = 4, kStatShadow = 5, kStatPaths = 6,
-  kStatRecordsDropped = 7, kWorkTrace = 8, kCountFree = 9, kIdentA = 10, kIdentB = 11, kNumCounters = 16
+  kStatRecordsDropped = 7, kWorkTrace = 8, kCountFree = 9, kIdentA = 10, kIdentB = 11, kCountShadow2 = 12, kSlotTicket = 13,
+  kNumCounters = 16
+};
+// What the slot selection of an iteration hands to the regeneration: how many freed slots take the
+// next camera paths of the pass, and the pixel and sample of the first of them.
+struct SlotPlan {
+  unsigned long long sample0;
+  uint32_t pixel0, refill;
+};
+// Progress record of an iteration, written by the device into page-locked host memory: camera
+// paths issued, work queued for the next iteration, and the iteration's number (written last).
+struct PassProgress {
+  unsigned long long issued, queued, seq;
+};
+// End of a pass, written by the device into page-locked host memory.
+struct PassReport {
+  uint32_t counters[kNumCounters];
+  uint32_t stack_overflow;
 };
 // Queues A and B carry a flag beside their length (counters[kIdentA], counters[kIdentB]): 1 when the
 // queue holds every slot of the wavefront, so that entry k may be taken as slot k.

@@ -56,8 +56,8 @@ __device__ __forceinline__ uint32_t gtid() { return blockIdx.x * blockDim.x + th
 __global__ void k_reset_counter(uint32_t *counters, int which) {
   if (threadIdx.x == 0 && blockIdx.x == 0) counters[which] = 0;
 }
-__global__ void k_fill_f64(double *p, size_t n, double v) {
-  for (size_t i = gtid(); i < n; i += grid_stride()) p[i] = v;
+__global__ void k_fill_f64(double *p, double *p2, size_t n, double v) {
+  for (size_t i = gtid(); i < n; i += grid_stride()) p[i] = p2[i] = v;
 }
 
 // ---- camera (src/camera.hxx:105-124, 176-210) ----------------------------
@@ -89,12 +89,10 @@ __device__ __forceinline__ bool camera_ray(const DevCamera &c, int px, int py, f
   return false;
 }
 
-// Camera path number g of the pass in path slot `slot`: pixel = g % npix, sample = spp_base + g / npix.
+// Camera path of (pixel, sample) in path slot i.
 // Lambda selection: LambdaSelectionStrategy::WithWeights (src/shader_util.hxx:83-91) with 4 strata.
-__device__ __forceinline__ void init_camera_path(const DeviceScene &sc, const PathQueues &q, uint32_t i, uint64_t g, uint32_t npix,
-                                                 uint32_t spp_base, uint64_t seed) {
-  const uint32_t pixel = (uint32_t)(g % npix);
-  const uint64_t sample = spp_base + g / npix;
+__device__ __forceinline__ void init_camera_path(const DeviceScene &sc, const PathQueues &q, uint32_t i, uint32_t pixel, uint64_t sample,
+                                                 uint32_t npix, uint64_t seed) {
   Pcg rng;
   rng.seed(seed, sample * npix + pixel);
   int main_idx = (int)rng.bounded(kStrata);
@@ -133,11 +131,29 @@ __device__ __forceinline__ void init_camera_path(const DeviceScene &sc, const Pa
   }
 }
 
-// The first `count` camera paths of a pass fill slots [0, count).
+// The first `count` camera paths of a pass fill slots [0, count): path g is sample
+// spp_base + g / npix of pixel g % npix.  Also sets up the pass's counters (which this kernel does
+// not read): queue A is 0, 1, .., count - 1.
 __global__ void __launch_bounds__(256) k_raygen(DeviceScene sc, PathQueues q, uint32_t count, uint32_t npix, uint32_t spp_base,
                                                 uint64_t seed) {
+  if (gtid() == 0) {
+    q.counters[kCountA] = count;
+    q.counters[kCountB] = 0;
+    q.counters[kCountShadow] = 0;
+    q.counters[kCountShadow2] = 0;
+    q.counters[kCountFree] = 0;
+    q.counters[kSlotTicket] = 0;
+    q.counters[kIdentA] = 1;
+    q.counters[kIdentB] = 0;
+    if (sc.guide_record) {
+      q.counters[kCountRecords] = 0;
+      q.counters[kStatRecordsDropped] = 0;
+    }
+    q.progress[0] = count;
+    q.progress[1] = count;
+  }
   for (uint32_t i = gtid(); i < count; i += grid_stride()) {
-    init_camera_path(sc, q, i, i, npix, spp_base, seed);
+    init_camera_path(sc, q, i, i % npix, (uint64_t)spp_base + i / npix, npix, seed);
     q.queue_a[i] = i;
     if (q.alive) {
       q.alive[i] = 1;
@@ -146,113 +162,168 @@ __global__ void __launch_bounds__(256) k_raygen(DeviceScene sc, PathQueues q, ui
   }
 }
 
-// Sets up the counters of a pass whose first `count` paths are in queue A.
-__global__ void k_begin_pass(PathQueues q, uint32_t count) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    q.counters[kCountA] = count;
-    q.counters[kCountB] = 0;
-    q.counters[kCountShadow] = 0;
-    q.counters[kCountFree] = 0;
-    q.counters[kIdentA] = 1;  // queue A is 0, 1, .., count - 1
-    q.counters[kIdentB] = 0;
-    q.progress[0] = count;
-    q.progress[1] = count;
-  }
+// Waits until this wave's stores have arrived where their scope is coherent, and keeps the compiler
+// from moving memory accesses across.  Together with relaxed atomics of that scope it orders two
+// accesses without a fence, which would write the whole L2 back (buffer_wbl2): one such fence per
+// wave made k_slot_select 74 us instead of 12.
+__device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+__device__ __forceinline__ void report_progress(PassProgress *host, unsigned long long issued, unsigned long long queued,
+                                                unsigned long long seq) {
+  __hip_atomic_store(&host->issued, issued, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&host->queued, queued, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  wait_stores();
+  __hip_atomic_store(&host->seq, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Path regeneration: the slots freed in this iteration take the next camera paths of the pass (up
-// to `limit` paths in total), queued after the surviving paths for the next trace.
-__device__ __forceinline__ uint32_t regen_count(const PathQueues &q, uint64_t limit, uint64_t issued) {
+// Path regeneration (appended queues): the slots freed in this iteration take the next camera
+// paths of the pass (up to `limit` paths in total), queued after the surviving paths.
+__device__ __forceinline__ uint32_t regen_count(uint32_t freed, uint64_t limit, uint64_t issued) {
   const uint64_t left = limit > issued ? limit - issued : 0;
-  return (uint32_t)min((uint64_t)q.counters[kCountFree], left);
+  return (uint32_t)min((uint64_t)freed, left);
 }
 __global__ void __launch_bounds__(256) k_regen(DeviceScene sc, PathQueues q, uint32_t *__restrict__ queue_out,
                                                const uint32_t *__restrict__ count_out, uint64_t limit, uint32_t npix,
                                                uint32_t spp_base, uint64_t seed) {
   const uint64_t issued = q.progress[0];
-  const uint32_t n = regen_count(q, limit, issued);
+  const uint32_t n = regen_count(q.counters[kCountFree], limit, issued);
   const uint32_t out0 = *count_out;
   for (uint32_t k = gtid(); k < n; k += grid_stride()) {
     const uint32_t slot = q.free_slots[k];
-    init_camera_path(sc, q, slot, issued + k, npix, spp_base, seed);
-    if (q.alive) {
-      q.alive[slot] = 1;
-      q.freed[slot] = 0;
-    } else {
-      queue_out[out0 + k] = slot;
-    }
+    const uint64_t g = issued + k;
+    init_camera_path(sc, q, slot, (uint32_t)(g % npix), spp_base + g / npix, npix, seed);
+    queue_out[out0 + k] = slot;
   }
 }
+// Runs after k_regen (same stream): commits the issued paths and the queue length.  progress[1],
+// which the host polls to end the pass, is the work of the next trace launch: the queue, plus the
+// shadow rays queued for it when it takes them (with_shadow).
+__global__ void k_regen_commit(PathQueues q, uint32_t *count_out, uint64_t limit, int with_shadow, PassProgress *host,
+                               unsigned long long seq) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) {
+    const uint64_t issued = q.progress[0];
+    const uint32_t n = regen_count(q.counters[kCountFree], limit, issued);
+    const uint32_t total = *count_out + n;
+    *count_out = total;
+    // A queue of every slot is read as slot k = entry k (coalesced path-state accesses).
+    count_out[kIdentOffset] = total == (uint32_t)q.capacity ? 1u : 0u;
+    q.progress[0] = issued + n;
+    q.progress[1] = total + (with_shadow ? *q.shadow_out : 0u);
+    q.counters[kCountFree] = 0;
+    report_progress(host, q.progress[0], q.progress[1], seq);
+  }
+}
+
 // ---- slot-ordered queues -------------------------------------------------------------
 // The next queue lists, in ascending slot order, the alive slots (paths that continue) and the
 // freed slots the regeneration refills (the first min(freed, paths left) of the freed slots in
-// ascending order, which free_slots lists for k_regen): slot k lands at (alive slots before k) +
-// min(freed slots before k, refilled).  One thread per slot, kSlotBlock slots per block (large
-// blocks keep the single-block scan over the block counts short: 4096 counts for 4 M slots).
+// ascending order): slot k lands at (alive slots before k) + min(freed slots before k, refilled).
+// Two launches per iteration.  k_slot_select counts the flags of each chunk of kSlotBlock slots
+// (one wave per chunk, 16 flags of each kind per lane in two 16-byte loads); its last block turns
+// the counts into prefix sums, commits the pass's progress and reports it to the host.
+// k_slot_scatter writes the queue and starts the new camera paths in their slots.  Both are bound
+// by launch latency below a million slots (6 + 5 us); over 4 M slots they take 12 + 46 us, where
+// separate count, scan, scatter, regeneration and commit kernels, the clears of the counters and
+// the progress copy took 13 + 8 + 17 + 37 + 5 + 9 + 4 us in nine launches (1080p benchmark, average
+// launch).
 constexpr int kSlotBlock = 1024;
 
-__global__ void __launch_bounds__(kSlotBlock) k_slot_count(PathQueues q, uint32_t n, uint32_t *__restrict__ bc) {
-  __shared__ uint32_t s[2][kSlotBlock / 64];
-  const uint32_t k = blockIdx.x * kSlotBlock + threadIdx.x;
-  const bool a = k < n && q.alive[k] != 0, f = k < n && q.freed[k] != 0;
-  const uint64_t ma = __ballot(a), mf = __ballot(f);
-  const int w = (int)(threadIdx.x >> 6);
-  if ((threadIdx.x & 63) == 0) {
-    s[0][w] = (uint32_t)__popcll(ma);
-    s[1][w] = (uint32_t)__popcll(mf);
+// Storage of the selection: the plan, the chunks' packed counts, and their prefix sums.
+struct SlotTemp {
+  SlotPlan plan;
+  uint32_t counts[1];  // nb packed counts (alive | freed << 16), then nb alive and nb freed prefix sums
+};
+
+__global__ void __launch_bounds__(kSlotBlock) k_slot_select(PathQueues q, uint32_t n, uint32_t nb, SlotTemp *__restrict__ tmp,
+                                                            uint32_t *count_out, uint64_t limit, uint32_t npix, uint32_t spp_base,
+                                                            int with_shadow, PassProgress *host, unsigned long long seq) {
+  constexpr int kWaves = kSlotBlock / 64;
+  __shared__ uint32_t s_part[2][kWaves];
+  __shared__ int s_last;
+  const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6);
+  uint32_t *counts = tmp->counts;
+  const uint32_t chunk = blockIdx.x * kWaves + wave;
+  if (chunk < nb) {
+    const uint32_t base = chunk * kSlotBlock + 16u * lane;
+    uint32_t c = 0;
+    if (base + 16u <= n) {
+      const uint4 a = *reinterpret_cast<const uint4 *>(q.alive + base), f = *reinterpret_cast<const uint4 *>(q.freed + base);
+      c = (uint32_t)(__popc(a.x) + __popc(a.y) + __popc(a.z) + __popc(a.w)) +
+          ((uint32_t)(__popc(f.x) + __popc(f.y) + __popc(f.z) + __popc(f.w)) << 16);
+    } else {
+      for (uint32_t k = base; k < n; ++k) c += (uint32_t)q.alive[k] + ((uint32_t)q.freed[k] << 16);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
+    if (lane == 0) {
+      __hip_atomic_store(counts + chunk, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      wait_stores();
+    }
   }
   __syncthreads();
+  if (threadIdx.x == 0) s_last = atomicAdd(q.counters + kSlotTicket, 1u) == gridDim.x - 1u;
+  __syncthreads();
+  if (!s_last) return;
+  // The last block to arrive: every chunk's count is in memory.
+  const uint32_t per = (nb + kSlotBlock - 1) / kSlotBlock, b0 = min(threadIdx.x * per, nb), b1 = min(b0 + per, nb);
+  uint32_t *pa = counts + nb, *pf = counts + 2 * (size_t)nb;
+  uint32_t ta = 0, tf = 0;
+  for (uint32_t b = b0; b < b1; ++b) {
+    const uint32_t c = __hip_atomic_load(counts + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    ta += c & 0xffffu;
+    tf += c >> 16;
+  }
+  uint32_t ia = ta, jf = tf;  // inclusive sums over the wave's threads
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t va = __shfl_up(ia, o), vf = __shfl_up(jf, o);
+    ia += lane >= o ? va : 0u;
+    jf += lane >= o ? vf : 0u;
+  }
+  if (lane == 63) {
+    s_part[0][wave] = ia;
+    s_part[1][wave] = jf;
+  }
+  __syncthreads();
+  uint32_t before_a = 0, before_f = 0, all_a = 0, all_f = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    if (w < wave) {
+      before_a += s_part[0][w];
+      before_f += s_part[1][w];
+    }
+    all_a += s_part[0][w];
+    all_f += s_part[1][w];
+  }
+  uint32_t ra = before_a + ia - ta, rf = before_f + jf - tf;
+  for (uint32_t b = b0; b < b1; ++b) {
+    const uint32_t c = __hip_atomic_load(counts + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    pa[b] = ra;
+    pf[b] = rf;
+    ra += c & 0xffffu;
+    rf += c >> 16;
+  }
   if (threadIdx.x == 0) {
-    uint32_t ta = 0, tf = 0;
-#pragma unroll
-    for (int i = 0; i < kSlotBlock / 64; ++i) {
-      ta += s[0][i];
-      tf += s[1][i];
-    }
-    bc[blockIdx.x] = ta;
-    bc[gridDim.x + blockIdx.x] = tf;
+    const uint64_t issued = q.progress[0];
+    const uint32_t refill = regen_count(all_f, limit, issued);
+    const uint32_t total = all_a + refill;
+    tmp->plan = SlotPlan{spp_base + issued / npix, (uint32_t)(issued % npix), refill};
+    *count_out = total;
+    // A queue of every slot of the pass is read as slot k = entry k (coalesced path-state accesses).
+    count_out[kIdentOffset] = total == n ? 1u : 0u;
+    q.progress[0] = issued + refill;
+    q.progress[1] = total + (with_shadow ? *q.shadow_out : 0u);
+    *q.shadow_in = 0;  // read by this iteration's trace launch; the next shade launch appends there
+    q.counters[kSlotTicket] = 0;
+    report_progress(host, q.progress[0], q.progress[1], seq);
   }
 }
 
-// One block of 1024 threads: exclusive prefix sums of the nb per-block counts of each flag, in
-// place; the next queue's length (alive + refilled) and the number of freed slots.
-__global__ void __launch_bounds__(1024) k_slot_scan(PathQueues q, uint32_t nb, uint32_t *__restrict__ bc, uint32_t *count_out,
-                                                    uint64_t limit) {
-  __shared__ uint32_t part[2][1024];
-  const uint32_t t = threadIdx.x, per = (nb + 1023) / 1024, b0 = t * per, b1 = min(b0 + per, nb);
-#pragma unroll
-  for (int f = 0; f < 2; ++f) {
-    uint32_t sum = 0;
-    for (uint32_t b = b0; b < b1; ++b) sum += bc[(size_t)f * nb + b];
-    part[f][t] = sum;
-  }
-  __syncthreads();
-  for (uint32_t off = 1; off < 1024; off <<= 1) {
-    const uint32_t v0 = t >= off ? part[0][t - off] : 0u, v1 = t >= off ? part[1][t - off] : 0u;
-    __syncthreads();
-    part[0][t] += v0;
-    part[1][t] += v1;
-    __syncthreads();
-  }
-#pragma unroll
-  for (int f = 0; f < 2; ++f) {
-    uint32_t run = t > 0 ? part[f][t - 1] : 0u;
-    for (uint32_t b = b0; b < b1; ++b) {
-      const uint32_t v = bc[(size_t)f * nb + b];
-      bc[(size_t)f * nb + b] = run;
-      run += v;
-    }
-  }
-  if (t == 0) {
-    const uint32_t freed = part[1][1023];
-    q.counters[kCountFree] = freed;
-    *count_out = part[0][1023] + regen_count(q, limit, q.progress[0]);
-  }
-}
-
-__global__ void __launch_bounds__(kSlotBlock) k_slot_scatter(PathQueues q, uint32_t n, const uint32_t *__restrict__ bc, uint64_t limit,
+__global__ void __launch_bounds__(kSlotBlock) k_slot_scatter(DeviceScene sc, PathQueues q, uint32_t n, uint32_t nb,
+                                                             const SlotTemp *__restrict__ tmp, uint32_t npix, uint64_t seed,
                                                              uint32_t *__restrict__ queue_out) {
   __shared__ uint32_t s[2][kSlotBlock / 64];
+  if (tmp->counts[blockIdx.x] == 0) return;  // no slot of the chunk is alive or freed
   const uint32_t k = blockIdx.x * kSlotBlock + threadIdx.x;
   const bool a = k < n && q.alive[k] != 0, f = k < n && q.freed[k] != 0;
   const uint64_t ma = __ballot(a), mf = __ballot(f);
@@ -262,7 +333,7 @@ __global__ void __launch_bounds__(kSlotBlock) k_slot_scatter(PathQueues q, uint3
     s[1][w] = (uint32_t)__popcll(mf);
   }
   __syncthreads();
-  uint32_t ra = bc[blockIdx.x], rf = bc[gridDim.x + blockIdx.x];
+  uint32_t ra = tmp->counts[nb + blockIdx.x], rf = tmp->counts[2 * (size_t)nb + blockIdx.x];
   for (int i = 0; i < w; ++i) {
     ra += s[0][i];
     rf += s[1][i];
@@ -270,26 +341,24 @@ __global__ void __launch_bounds__(kSlotBlock) k_slot_scatter(PathQueues q, uint3
   const uint64_t below = (1ull << lane) - 1ull;
   ra += (uint32_t)__popcll(ma & below);
   rf += (uint32_t)__popcll(mf & below);
-  const uint32_t refill = regen_count(q, limit, q.progress[0]);
-  if (f) q.free_slots[rf] = k;
-  if (a || (f && rf < refill)) queue_out[ra + min(rf, refill)] = k;
+  const SlotPlan plan = tmp->plan;
+  const bool refilled = f && rf < plan.refill;
+  if (a || refilled) queue_out[ra + min(rf, plan.refill)] = k;
+  if (refilled) {
+    // pixel0 + rf stays below 2^32: fewer than 2^31 pixels, at most 2^26 slots.
+    const uint32_t g = plan.pixel0 + rf;
+    init_camera_path(sc, q, k, g % npix, plan.sample0 + g / npix, npix, seed);
+    q.alive[k] = 1;
+    q.freed[k] = 0;
+  }
 }
 
-// Runs after k_regen (same stream): commits the issued paths and the queue length.  progress[1],
-// which the host polls to end the pass, is the work of the next trace launch: the queue, plus the
-// shadow rays queued for it when it takes them (with_shadow).
-__global__ void k_regen_commit(PathQueues q, uint32_t *count_out, uint64_t limit, int with_shadow) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    const uint64_t issued = q.progress[0];
-    const uint32_t n = regen_count(q, limit, issued);
-    // Slot-ordered queues: the selection of the alive slots (after k_regen) already counted them.
-    const uint32_t total = q.alive ? *count_out : *count_out + n;
-    *count_out = total;
-    // A queue of every slot is read as slot k = entry k (coalesced path-state accesses).
-    count_out[kIdentOffset] = total == (uint32_t)q.capacity ? 1u : 0u;
-    q.progress[0] = issued + n;
-    q.progress[1] = total + (with_shadow ? q.counters[kCountShadow] : 0u);
-    q.counters[kCountFree] = 0;
+__global__ void k_report(PathQueues q, PassReport *host) {
+  if (threadIdx.x < kNumCounters) host->counters[threadIdx.x] = q.counters[threadIdx.x];
+  if (threadIdx.x == 0) {
+    const unsigned int v = g_stack_overflow;
+    host->stack_overflow = v;
+    if (v) g_stack_overflow = 0;
   }
 }
 
@@ -345,7 +414,7 @@ __global__ void __launch_bounds__(kTraceBlock, TTGPU_TRACE_WAVES) k_trace(Device
   int *stack = lds_stack + threadIdx.x;
   int spill[kSpillStack];
   const uint32_t ccount = *count_ptr;
-  const uint32_t scount = kShadow ? q.counters[kCountShadow] : 0u;
+  const uint32_t scount = kShadow ? *q.shadow_in : 0u;
   const uint32_t count = ccount + scount;
   const bool ident = count_ptr[kIdentOffset] != 0;
   for (uint32_t k = gtid(); k < count; k += grid_stride()) {
@@ -384,7 +453,7 @@ __global__ void __launch_bounds__(kTraceBlock, TTGPU_TRACE_WAVES) k_trace_dyn(De
   int *stack = lds_stack + threadIdx.x;
   int spill[kSpillStack];
   const uint32_t ccount = *count_ptr;
-  const uint32_t scount = kShadow ? q.counters[kCountShadow] : 0u;
+  const uint32_t scount = kShadow ? *q.shadow_in : 0u;
   const uint32_t count = ccount + scount;
   const bool ident = count_ptr[kIdentOffset] != 0;
   Trav t;
@@ -900,7 +969,7 @@ __global__ void __launch_bounds__(256, TTGPU_SHADE_WAVES) k_shade(DeviceScene sc
       }
     }
     uint32_t slot, sslot;
-    block_append2<4>(count_out, push && !q.alive, q.counters + kCountShadow, push_shadow, s_cnt, slot, sslot);
+    block_append2<4>(count_out, push && !q.alive, q.shadow_out, push_shadow, s_cnt, slot, sslot);
     if (q.alive) {
       if (active) q.alive[i] = push ? 1 : 0;
     } else if (push) {
@@ -913,7 +982,7 @@ __global__ void __launch_bounds__(256, TTGPU_SHADE_WAVES) k_shade(DeviceScene sc
 // ---- shadow rays: any hit + accumulate + finalize -----------------------------------
 __global__ void __launch_bounds__(kTraceBlock, TTGPU_TRACE_WAVES) k_shadow(DeviceScene sc, PathQueues q, double *fb, double *fb_sq, uint32_t *stats) {
   __shared__ int lds_stack[kLdsStack * kTraceBlock];
-  const uint32_t count = q.counters[kCountShadow];
+  const uint32_t count = *q.shadow_out;
   for (uint32_t k = gtid(); k < count; k += grid_stride()) {
     const uint32_t i = q.shadow_queue[k];
     const float4 o = q.sh_org[i];
@@ -1192,7 +1261,7 @@ __global__ void __launch_bounds__(kTraceBlock) k_shade_media(DeviceScene sc, Pat
       }
     }
     uint32_t slot, sslot;
-    block_append2<kTraceBlock / 64>(count_out, push && !q.alive, q.counters + kCountShadow, push_shadow, s_cnt, slot, sslot);
+    block_append2<kTraceBlock / 64>(count_out, push && !q.alive, q.shadow_out, push_shadow, s_cnt, slot, sslot);
     if (q.alive) {
       if (active) q.alive[i] = push ? 1 : 0;
     } else if (push) {
@@ -1205,7 +1274,7 @@ __global__ void __launch_bounds__(kTraceBlock) k_shade_media(DeviceScene sc, Pat
 // ---- media: shadow rays with occlusion + null-path transmission + MIS -----------------------
 __global__ void __launch_bounds__(kTraceBlock) k_shadow_media(DeviceScene sc, PathQueues q, double *fb, double *fb_sq, uint32_t *stats) {
   __shared__ int lds_stack[kLdsStack * kTraceBlock];
-  const uint32_t count = q.counters[kCountShadow];
+  const uint32_t count = *q.shadow_out;
   const bool mis = sc.sample_mode == TTGPU_SAMPLE_BOTH;
   const bool rec = sc.guide_record != 0 && q.vt != nullptr;
   for (uint32_t k = gtid(); k < count; k += grid_stride()) {
@@ -1510,7 +1579,7 @@ __global__ void __launch_bounds__(kTraceBlock) k_shade_media_guided(DeviceScene 
       }
     }
     uint32_t slot, sslot;
-    block_append2<kTraceBlock / 64>(count_out, push && !q.alive, q.counters + kCountShadow, push_shadow, s_cnt, slot, sslot);
+    block_append2<kTraceBlock / 64>(count_out, push && !q.alive, q.shadow_out, push_shadow, s_cnt, slot, sslot);
     if (q.alive) {
       if (active) q.alive[i] = push ? 1 : 0;
     } else if (push) {
@@ -1667,7 +1736,7 @@ __global__ void __launch_bounds__(256) k_shade_guided(DeviceScene sc, PathQueues
       }
     }
     uint32_t slot, sslot;
-    block_append2<4>(count_out, push && !q.alive, q.counters + kCountShadow, push_shadow, s_cnt, slot, sslot);
+    block_append2<4>(count_out, push && !q.alive, q.shadow_out, push_shadow, s_cnt, slot, sslot);
     if (q.alive) {
       if (active) q.alive[i] = push ? 1 : 0;
     } else if (push) {
@@ -1705,7 +1774,7 @@ __device__ void shadow_done_guided(const DeviceScene &sc, const PathQueues &q, u
 
 __global__ void __launch_bounds__(kTraceBlock) k_shadow_guided(DeviceScene sc, PathQueues q, double *fb, double *fb_sq, uint32_t *stats) {
   __shared__ int lds_stack[kLdsStack * kTraceBlock];
-  const uint32_t count = q.counters[kCountShadow];
+  const uint32_t count = *q.shadow_out;
   for (uint32_t k = gtid(); k < count; k += grid_stride()) {
     const uint32_t i = q.shadow_queue[k];
     const float4 o = q.sh_org[i];
@@ -2463,33 +2532,32 @@ static int Blocks(uint64_t n, int block, int cap) {
 void LaunchResetCounter(uint32_t *counters, int which, hipStream_t st) {
   hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(64), 0, st, counters, which);
 }
-void LaunchFill(double *p, size_t n, double v, hipStream_t st) {
-  hipLaunchKernelGGL(k_fill_f64, dim3(Blocks(n, 256, 4096)), dim3(256), 0, st, p, n, v);
+void LaunchFill(double *p, double *p2, size_t n, double v, hipStream_t st) {
+  hipLaunchKernelGGL(k_fill_f64, dim3(Blocks(n, 256, 4096)), dim3(256), 0, st, p, p2, n, v);
 }
 void LaunchRaygen(const DeviceScene &sc, const PathQueues &q, uint32_t count, uint32_t npix, uint32_t spp_base, uint64_t seed,
                   hipStream_t st) {
   hipLaunchKernelGGL(k_raygen, dim3(Blocks(count, 256, 65535)), dim3(256), 0, st, sc, q, count, npix, spp_base, seed);
-  hipLaunchKernelGGL(k_begin_pass, dim3(1), dim3(64), 0, st, q, count);
 }
-size_t SelectTempBytes(uint32_t capacity) { return 2 * (size_t)((capacity + kSlotBlock - 1) / kSlotBlock) * sizeof(uint32_t); }
+size_t SelectTempBytes(uint32_t capacity) {
+  return sizeof(SlotTemp) + 3 * (size_t)((capacity + kSlotBlock - 1) / kSlotBlock) * sizeof(uint32_t);
+}
 
-void LaunchRegen(const DeviceScene &sc, const PathQueues &q, uint32_t *queue_out, uint32_t *count_out, uint32_t max_count,
-                 uint64_t limit, uint32_t npix, uint32_t spp_base, uint64_t seed, bool with_shadow, uint32_t slots, void *select_temp,
-                 size_t select_bytes, hipStream_t st) {
+void LaunchRegen(const DeviceScene &sc, const PathQueues &q, const RegenArgs &a, hipStream_t st) {
   if (q.alive) {
-    // Slot-ordered queues over the pass's slots [0, slots): per-block counts of the alive and
-    // freed flags, their prefix sums, then the next queue (alive slots and the freed slots the
-    // regeneration takes, ascending) and the freed slots in ascending order.
-    const uint32_t nb = (slots + kSlotBlock - 1) / kSlotBlock;
-    if (2 * (size_t)nb * sizeof(uint32_t) > select_bytes) throw std::runtime_error("slot selection storage too small");
-    uint32_t *bc = static_cast<uint32_t *>(select_temp);
-    hipLaunchKernelGGL(k_slot_count, dim3(nb), dim3(kSlotBlock), 0, st, q, slots, bc);
-    hipLaunchKernelGGL(k_slot_scan, dim3(1), dim3(1024), 0, st, q, nb, bc, count_out, limit);
-    hipLaunchKernelGGL(k_slot_scatter, dim3(nb), dim3(kSlotBlock), 0, st, q, slots, bc, limit, queue_out);
+    const uint32_t nb = (a.slots + kSlotBlock - 1) / kSlotBlock, per_block = kSlotBlock / 64;
+    SlotTemp *tmp = static_cast<SlotTemp *>(a.select_temp);
+    hipLaunchKernelGGL(k_slot_select, dim3((nb + per_block - 1) / per_block), dim3(kSlotBlock), 0, st, q, a.slots, nb, tmp, a.count_out,
+                       a.limit, a.npix, a.spp_base, a.with_shadow ? 1 : 0, a.host, a.seq);
+    hipLaunchKernelGGL(k_slot_scatter, dim3(nb), dim3(kSlotBlock), 0, st, sc, q, a.slots, nb, tmp, a.npix, a.seed, a.queue_out);
+    return;
   }
-  hipLaunchKernelGGL(k_regen, dim3(Blocks(max_count, 256, 8192)), dim3(256), 0, st, sc, q, queue_out, count_out, limit, npix, spp_base,
-                     seed);
-  hipLaunchKernelGGL(k_regen_commit, dim3(1), dim3(64), 0, st, q, count_out, limit, with_shadow ? 1 : 0);
+  hipLaunchKernelGGL(k_regen, dim3(Blocks(a.slots, 256, 8192)), dim3(256), 0, st, sc, q, a.queue_out, a.count_out, a.limit, a.npix,
+                     a.spp_base, a.seed);
+  hipLaunchKernelGGL(k_regen_commit, dim3(1), dim3(64), 0, st, q, a.count_out, a.limit, a.with_shadow ? 1 : 0, a.host, a.seq);
+}
+void LaunchReport(const PathQueues &q, PassReport *host, hipStream_t st) {
+  hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, st, q, host);
 }
 // Workgroups that fit on the device at once for a persistent kernel (computed on first use).
 template <class K>

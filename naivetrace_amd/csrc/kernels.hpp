@@ -8,19 +8,27 @@ namespace ttgpu {
 
 hipError_t UploadSpectralTables(const float *to_rgb, const float *smits);
 void LaunchResetCounter(uint32_t *counters, int which, hipStream_t st);
-void LaunchFill(double *p, size_t n, double v, hipStream_t st);
+void LaunchFill(double *p, double *p2, size_t n, double v, hipStream_t st);  // two arrays of n values
 // First `count` camera paths of a pass into slots [0, count) of queue A; resets the pass counters.
 void LaunchRaygen(const DeviceScene &sc, const PathQueues &q, uint32_t count, uint32_t npix, uint32_t spp_base, uint64_t seed,
                   hipStream_t st);
-// Path regeneration after an iteration's shadow rays: freed slots take the pass's next camera paths
-// (at most `limit` issued in total) and are queued after the survivors in queue_out.
-// Slot-ordered queues (q.alive): before the regeneration, the freed slots of [0, slots) are listed
-// in ascending order and the next queue is built from the alive flags and the slots the
-// regeneration refills, with `select_temp` (SelectTempBytes(capacity) bytes) for the per-block
-// counts.
-void LaunchRegen(const DeviceScene &sc, const PathQueues &q, uint32_t *queue_out, uint32_t *count_out, uint32_t max_count,
-                 uint64_t limit, uint32_t npix, uint32_t spp_base, uint64_t seed, bool with_shadow, uint32_t slots, void *select_temp,
-                 size_t select_bytes, hipStream_t st);
+// Path regeneration of an iteration: freed slots take the pass's next camera paths (at most `limit`
+// issued in total) and the next queue is built in queue_out, its length (and identity flag) in
+// count_out; the iteration's progress goes to `host` with sequence number `seq`.
+struct RegenArgs {
+  uint32_t *queue_out, *count_out;
+  uint32_t slots;           // slots the pass uses: [0, slots)
+  uint64_t limit;
+  uint32_t npix, spp_base;
+  uint64_t seed;
+  bool with_shadow;         // the queued shadow rays are work of the next trace launch
+  PassProgress *host;       // device address of the page-locked record
+  unsigned long long seq;
+  void *select_temp;        // SelectTempBytes(capacity) bytes (slot-ordered queues)
+};
+void LaunchRegen(const DeviceScene &sc, const PathQueues &q, const RegenArgs &a, hipStream_t st);
+// Counters and the stack-overflow flag (then cleared) to the page-locked report.
+void LaunchReport(const PathQueues &q, PassReport *host, hipStream_t st);
 size_t SelectTempBytes(uint32_t capacity);
 // with_shadow: the persistent traversal also takes the shadow rays of the previous shade launch
 // (ShadowInTrace), and LaunchShadow is not called.

@@ -89,7 +89,6 @@ struct ttgpu_handle {
   std::vector<void *> allocs;
   double *fb = nullptr, *fb_sq = nullptr;
   void *select_temp = nullptr;  // storage of the slot-ordered queue selection
-  size_t select_bytes = 0;
   InferSort infer_sort{};       // learned guide: sort of the inference queue by hit point
   bool infer_sorted = false;
   std::vector<uint64_t> pixel_spp;
@@ -109,9 +108,12 @@ struct ttgpu_handle {
   std::vector<std::pair<std::string, std::pair<hipEvent_t, hipEvent_t>>> pending_events;
   std::vector<hipEvent_t> event_pool;
   size_t event_next = 0;
-  // path-regeneration progress read-back: two pinned slots of {issued, queued} and their events
-  unsigned long long *poll = nullptr;
-  hipEvent_t poll_ev[2] = {nullptr, nullptr};
+  // page-locked records the device writes: the progress of even and odd iterations, and the
+  // counters at the end of a pass
+  struct Pinned {
+    PassProgress poll[2];
+    PassReport report;
+  } *pinned = nullptr, *pinned_dev = nullptr;
   int npix = 0;
   uint32_t capacity = 0;
   // host copies needed later
@@ -192,9 +194,7 @@ struct ttgpu_handle {
   ~ttgpu_handle() {
     if (stream) (void)hipStreamSynchronize(stream);
     for (auto e : event_pool) (void)hipEventDestroy(e);
-    for (auto e : poll_ev)
-      if (e) (void)hipEventDestroy(e);
-    if (poll) (void)hipHostFree(poll);
+    if (pinned) (void)hipHostFree(pinned);
     for (void *p : allocs) (void)hipFree(p);
     if (d_guide_nodes) (void)hipFree(d_guide_nodes);
     if (d_guide_cells) (void)hipFree(d_guide_cells);
@@ -807,13 +807,14 @@ void AllocateQueues(ttgpu_handle *h) {
     q.freed = h->Alloc<uint8_t>(N);
     Check(hipMemset(q.alive, 0, N), "hipMemset alive flags");
     Check(hipMemset(q.freed, 0, N), "hipMemset freed flags");
-    h->select_bytes = std::max<size_t>(SelectTempBytes(N), 16);
-    h->select_temp = h->Alloc<uint8_t>(h->select_bytes);
+    h->select_temp = h->Alloc<uint8_t>(SelectTempBytes(N));
   }
   q.progress = h->Alloc<unsigned long long>(2);
   Check(hipMemset(q.progress, 0, 2 * sizeof(unsigned long long)), "hipMemset progress");
-  Check(hipHostMalloc((void **)&h->poll, 4 * sizeof(unsigned long long)), "hipHostMalloc");
-  for (auto &e : h->poll_ev) Check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+  Check(hipHostMalloc((void **)&h->pinned, sizeof(*h->pinned)), "hipHostMalloc");
+  Check(hipHostGetDevicePointer((void **)&h->pinned_dev, h->pinned, 0), "hipHostGetDevicePointer");
+  *h->pinned = {};
+  q.shadow_in = q.shadow_out = q.counters + kCountShadow;
   if (h->dsc.has_media) {
     q.wt_r = h->Alloc<float4>(N);
     q.wt_c = h->Alloc<float4>(N);
@@ -870,8 +871,7 @@ void AllocateQueues(ttgpu_handle *h) {
   const size_t npix = (size_t)h->npix;
   h->fb = h->Alloc<double>(3 * npix);
   h->fb_sq = h->Alloc<double>(3 * npix);
-  LaunchFill(h->fb, 3 * npix, 0.0, h->stream);
-  LaunchFill(h->fb_sq, 3 * npix, 0.0, h->stream);
+  LaunchFill(h->fb, h->fb_sq, 3 * npix, 0.0, h->stream);
   Check(hipGetLastError(), "fill framebuffer");
   Check(hipStreamSynchronize(h->stream), "sync");
 }
@@ -1165,8 +1165,7 @@ void DownloadFit(ttgpu_handle *h) {
 // The fit of the pass just rendered, on the device: entries, sort by cell, per-cell fit.
 void GpuFitPass(ttgpu_handle *h) {
   auto &F = h->fit;
-  uint32_t counters[kNumCounters];
-  Check(hipMemcpy(counters, h->q.counters, sizeof(counters), hipMemcpyDeviceToHost), "read counters");
+  const uint32_t *counters = h->pinned->report.counters;  // of the pass just rendered
   const int64_t n = std::min(counters[kCountRecords], h->q.rec_capacity);
   h->records_last_pass = n;
   h->records_dropped += counters[kStatRecordsDropped];
@@ -1209,8 +1208,7 @@ void GpuFitPass(ttgpu_handle *h) {
 
 // Downloads the records of the pass just rendered and hands them to the recorder.
 void CollectRecords(ttgpu_handle *h) {
-  uint32_t counters[kNumCounters];
-  Check(hipMemcpy(counters, h->q.counters, sizeof(counters), hipMemcpyDeviceToHost), "read counters");
+  const uint32_t *counters = h->pinned->report.counters;  // of the pass just rendered
   const uint32_t n = std::min(counters[kCountRecords], h->q.rec_capacity);
   h->records_last_pass = n;
   h->records_dropped += counters[kStatRecordsDropped];
@@ -1241,8 +1239,7 @@ void LearnFromPass(ttgpu_handle *h) {
     else GpuFitPass(h);
     return;
   }
-  uint32_t counters[kNumCounters];
-  Check(hipMemcpy(counters, h->q.counters, sizeof(counters), hipMemcpyDeviceToHost), "read counters");
+  const uint32_t *counters = h->pinned->report.counters;  // of the pass just rendered
   const int64_t n = std::min(counters[kCountRecords], h->q.rec_capacity);
   h->records_last_pass = n;
   h->records_dropped += counters[kStatRecordsDropped];
@@ -1281,11 +1278,36 @@ int Fail(ttgpu_handle *h, int code, const std::string &msg) {
     return Fail(h, TTGPU_ERR_RUNTIME, e.what());                          \
   }
 
+// Ends a pass: the counters and the traversal's overflow flag come back with the wait for the stream.
+void FinishPass(ttgpu_handle *h, hipEvent_t ev1) {
+  LaunchReport(h->q, &h->pinned_dev->report, h->stream);
+  Check(hipGetLastError(), "kernel launch");
+  Check(hipEventRecord(ev1, h->stream), "hipEventRecord");
+  Check(hipStreamSynchronize(h->stream), "hipStreamSynchronize");
+}
+void CheckReport(const ttgpu_handle *h) {
+  if (h->pinned->report.stack_overflow)
+    throw std::runtime_error("BVH traversal stack overflow: the tree is deeper than the traversal stack allows");
+}
+
+// Waits until iteration `seq` has reported its progress.  The stream's state bounds the wait: once
+// it has run dry (or failed) no report is on its way.
+const PassProgress &WaitProgress(ttgpu_handle *h, int slot, unsigned long long seq) {
+  const PassProgress &r = h->pinned->poll[slot];
+  for (unsigned spins = 1; __atomic_load_n(&r.seq, __ATOMIC_ACQUIRE) != seq; ++spins) {
+    __builtin_ia32_pause();
+    if (spins % 8192 != 0) continue;
+    const hipError_t e = hipStreamQuery(h->stream);
+    if (e == hipErrorNotReady) continue;
+    Check(e, "hipStreamQuery");
+    if (__atomic_load_n(&r.seq, __ATOMIC_ACQUIRE) != seq) throw std::runtime_error("no progress report from the device (internal error)");
+  }
+  return r;
+}
+
 void ResetFramebuffer(ttgpu_handle *h) {
-  LaunchFill(h->fb, 3 * (size_t)h->npix, 0.0, h->stream);
-  LaunchFill(h->fb_sq, 3 * (size_t)h->npix, 0.0, h->stream);
+  LaunchFill(h->fb, h->fb_sq, 3 * (size_t)h->npix, 0.0, h->stream);
   Check(hipGetLastError(), "fill");
-  Check(hipStreamSynchronize(h->stream), "sync");
   std::fill(h->pixel_spp.begin(), h->pixel_spp.end(), 0);
 }
 
@@ -1312,8 +1334,7 @@ bool RenderPassBdpt(ttgpu_handle *h, int spp) {
     issued += n;
     if (h->interrupt.exchange(false) && h->cb) h->cb(h->cb_user, 0);
   }
-  Check(hipEventRecord(ev1, h->stream), "hipEventRecord");
-  Check(hipStreamSynchronize(h->stream), "hipStreamSynchronize");
+  FinishPass(h, ev1);
   const bool complete = issued == total;
   {
     const uint64_t full = issued / npix, rem = issued % npix;
@@ -1327,11 +1348,9 @@ bool RenderPassBdpt(ttgpu_handle *h, int spp) {
   h->stats.render_ms = ms;
   h->CollectTimers();
   h->event_next = 0;
-  CheckTraversal(h->stream);
-  uint32_t counters[kNumCounters];
-  Check(hipMemcpy(counters, h->q.counters, sizeof(counters), hipMemcpyDeviceToHost), "read counters");
-  h->stats.rays_closest = counters[kStatClosest];
-  h->stats.rays_shadow = counters[kStatShadow];
+  CheckReport(h);
+  h->stats.rays_closest = h->pinned->report.counters[kStatClosest];
+  h->stats.rays_shadow = h->pinned->report.counters[kStatShadow];
   if (complete) {
     h->total_spp += spp;
     h->sched_total += spp;
@@ -1350,10 +1369,6 @@ bool RenderPass(ttgpu_handle *h, int spp) {
   PathQueues &q = h->q;
   hipEvent_t ev0 = h->NextEvent(), ev1 = h->NextEvent();
   Check(hipEventRecord(ev0, h->stream), "hipEventRecord");
-  if (h->dsc.guide_record) {
-    LaunchResetCounter(q.counters, kCountRecords, h->stream);
-    LaunchResetCounter(q.counters, kStatRecordsDropped, h->stream);
-  }
   const uint32_t n0 = (uint32_t)std::min<uint64_t>(cap, total);
   const uint32_t spp_base = (uint32_t)h->total_spp;
   h->Timed("raygen", [&] { LaunchRaygen(h->dsc, q, n0, (uint32_t)npix, spp_base, h->params.seed, h->stream); });
@@ -1363,40 +1378,48 @@ bool RenderPass(ttgpu_handle *h, int spp) {
   uint64_t limit = total;
   uint32_t *cur_q = q.queue_a, *nxt_q = q.queue_b;
   uint32_t *cur_c = q.counters + kCountA, *nxt_c = q.counters + kCountB;
-  int nxt_idx = kCountB;
+  uint32_t *shadow_in = q.counters + kCountShadow2, *shadow_out = q.counters + kCountShadow;
   bool stopped = false;
   // Plain surface passes trace each iteration's shadow rays in the next closest-hit launch.
   const bool shadow_in_trace = ShadowInTrace(h->dsc, q);
-  if (shadow_in_trace) LaunchResetCounter(q.counters, kCountShadow, h->stream);
+  const bool slot_order = q.alive != nullptr;
+  if (!slot_order) shadow_in = shadow_out;
+  h->pinned->poll[0] = h->pinned->poll[1] = PassProgress{n0, n0, 0};
+  // Every queue holds at most the pass's n0 slots; once all paths are issued, at most the work
+  // the last known iteration left (the launches' grids; their kernels stride over any count).
+  uint32_t bound = n0;
   for (uint64_t it = 0;; ++it) {
     if (it > max_iter) throw std::runtime_error("path regeneration did not drain (internal error)");
     if (!stopped && h->stop.load()) {
       stopped = true;
       limit = 0;  // issue no further camera paths; the paths in flight finish
     }
-    h->Timed("trace", [&] { LaunchTrace(h->dsc, q, cur_q, cur_c, cap, h->fb, h->fb_sq, shadow_in_trace, h->stream); });
-    if (q.vt) h->Timed("media", [&] { LaunchTrackMedia(h->dsc, q, cur_q, cur_c, cap, h->stream); });
+    q.shadow_in = shadow_in;
+    q.shadow_out = shadow_out;
+    h->Timed("trace", [&] { LaunchTrace(h->dsc, q, cur_q, cur_c, bound, h->fb, h->fb_sq, shadow_in_trace, h->stream); });
+    if (q.vt) h->Timed("media", [&] { LaunchTrackMedia(h->dsc, q, cur_q, cur_c, bound, h->stream); });
     if (h->learned)
       h->Timed("guide", [&] {
-        LaunchGuideInfer(h->dsc, q, cur_q, cur_c, h->infer_sorted ? n0 : cap, h->net->View(), h->infer_sorted ? &h->infer_sort : nullptr,
-                         h->stream);
+        LaunchGuideInfer(h->dsc, q, cur_q, cur_c, h->infer_sorted ? n0 : bound, h->net->View(),
+                         h->infer_sorted ? &h->infer_sort : nullptr, h->stream);
       });
-    LaunchResetCounter(q.counters, nxt_idx, h->stream);
-    LaunchResetCounter(q.counters, kCountShadow, h->stream);
-    h->Timed("shade", [&] { LaunchShade(h->dsc, q, cur_q, cur_c, nxt_q, nxt_c, cap, h->fb, h->fb_sq, h->stream); });
-    if (!shadow_in_trace) h->Timed("shadow", [&] { LaunchShadow(h->dsc, q, cap, h->fb, h->fb_sq, h->stream); });
+    if (!slot_order) {
+      LaunchResetCounter(q.counters, (int)(nxt_c - q.counters), h->stream);
+      LaunchResetCounter(q.counters, kCountShadow, h->stream);
+    }
+    h->Timed("shade", [&] { LaunchShade(h->dsc, q, cur_q, cur_c, nxt_q, nxt_c, bound, h->fb, h->fb_sq, h->stream); });
+    if (!shadow_in_trace) h->Timed("shadow", [&] { LaunchShadow(h->dsc, q, bound, h->fb, h->fb_sq, h->stream); });
+    const int slot = (int)(it & 1);
     h->Timed("raygen", [&] {
-      LaunchRegen(h->dsc, q, nxt_q, nxt_c, cap, limit, (uint32_t)npix, spp_base, h->params.seed, shadow_in_trace, n0, h->select_temp,
-                  h->select_bytes, h->stream);
+      LaunchRegen(h->dsc, q,
+                  RegenArgs{nxt_q, nxt_c, n0, limit, (uint32_t)npix, spp_base, h->params.seed, shadow_in_trace, &h->pinned_dev->poll[slot], it + 1,
+                            h->select_temp},
+                  h->stream);
     });
     Check(hipGetLastError(), "kernel launch");
-    const int slot = (int)(it & 1);
-    Check(hipMemcpyAsync(h->poll + 2 * slot, q.progress, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, h->stream),
-          "progress read-back");
-    Check(hipEventRecord(h->poll_ev[slot], h->stream), "hipEventRecord");
     std::swap(cur_q, nxt_q);
     std::swap(cur_c, nxt_c);
-    nxt_idx = nxt_idx == kCountA ? kCountB : kCountA;
+    if (slot_order) std::swap(shadow_in, shadow_out);
     if (h->interrupt.exchange(false)) {
       Check(hipStreamSynchronize(h->stream), "sync");
       if (h->cb) h->cb(h->cb_user, 0);
@@ -1404,22 +1427,19 @@ bool RenderPass(ttgpu_handle *h, int spp) {
     // Wait for the previous iteration (this one is already queued behind it): an empty queue after
     // regeneration means every issued path has finished and none is left to issue.
     if (it > 0) {
-      const int prev = 1 - slot;
-      Check(hipEventSynchronize(h->poll_ev[prev]), "hipEventSynchronize");
-      if (h->poll[2 * prev + 1] == 0) break;
+      const PassProgress &r = WaitProgress(h, 1 - slot, it);
+      if (r.queued == 0) break;
+      if (r.issued >= limit) bound = (uint32_t)std::min<uint64_t>(n0, r.queued);
     }
   }
-  Check(hipStreamSynchronize(h->stream), "hipStreamSynchronize");
-  const uint64_t issued = std::max(h->poll[0], h->poll[2]);
+  const uint64_t issued = std::max(h->pinned->poll[0].issued, h->pinned->poll[1].issued);
   const bool complete = issued == total;
   // pt: the light connection at the camera node of every issued camera sample.
   if (h->dsc.algo_pt && h->dsc.sample_mode != TTGPU_SAMPLE_BSDF && h->dsc.cam.kind == TTGPU_CAMERA_PINHOLE)
     h->Timed("camera", [&] {
       LaunchCameraConnect(h->dsc, 0, issued, (uint32_t)npix, spp_base, h->params.seed, h->fb, h->fb_sq, q.counters, h->stream);
     });
-  Check(hipGetLastError(), "kernel launch");
-  Check(hipEventRecord(ev1, h->stream), "hipEventRecord");
-  Check(hipStreamSynchronize(h->stream), "hipStreamSynchronize");
+  FinishPass(h, ev1);
   // Per-pixel sample counts: path g of the pass belongs to pixel g % npix.
   {
     const uint64_t full = issued / npix, rem = issued % npix;
@@ -1433,11 +1453,9 @@ bool RenderPass(ttgpu_handle *h, int spp) {
   h->stats.render_ms = ms;
   h->CollectTimers();
   h->event_next = 0;
-  CheckTraversal(h->stream);
-  uint32_t counters[kNumCounters];
-  Check(hipMemcpy(counters, q.counters, sizeof(counters), hipMemcpyDeviceToHost), "read counters");
-  h->stats.rays_closest = counters[kStatClosest];
-  h->stats.rays_shadow = counters[kStatShadow];
+  CheckReport(h);
+  h->stats.rays_closest = h->pinned->report.counters[kStatClosest];
+  h->stats.rays_shadow = h->pinned->report.counters[kStatShadow];
   if (complete) {
     h->total_spp += spp;
     h->sched_total += spp;
