@@ -542,8 +542,8 @@ def main():
     dom = max(("trace", "shade", "shadow"), key=lambda k: times[k][0])
     ms_tot, launches = times[dom]
     avg_ms = ms_tot / max(launches, 1)
-    # With persistent traversal the closest-hit launches also trace the shadow rays (no shadow
-    # launches of their own): their bytes count toward the traversal kernel.
+    # The closest-hit launches also trace the shadow rays (no shadow launches of their own): their
+    # bytes count toward the traversal kernel.
     shadow_in_trace = times["shadow"][1] == 0
     if dom == "trace":
         alg_bytes = (TRACE_BYTES_PER_RAY * rays_closest + (SHADOW_BYTES_PER_RAY * rays_shadow if shadow_in_trace else 0)) / max(launches, 1)
@@ -552,10 +552,8 @@ def main():
     else:
         alg_bytes = SHADE_BYTES_PER_PATH * rays_closest / max(launches, 1)
     achieved = alg_bytes / (avg_ms * 1e-3) / 1e9
-    # Closest-hit rays run in the persistent traversal kernel only with TTGPU_PERSISTENT_TRAVERSAL=1.
-    persistent = os.environ.get("TTGPU_PERSISTENT_TRAVERSAL", "0")[:1] == "1"
     # The trace kernels are templates on how they take shadow rays: <1> also traces them.
-    kname = (f"{'k_trace_dyn' if persistent else 'k_trace'}<{1 if shadow_in_trace else 0}>" if dom == "trace"
+    kname = (f"k_trace<{1 if shadow_in_trace else 0}>" if dom == "trace"
              else "k_shade<false>" if dom == "shade" else f"k_{dom}")
     roofline = {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": load_traffic(kname), "kernel": kname,

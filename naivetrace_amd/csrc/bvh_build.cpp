@@ -351,4 +351,86 @@ std::vector<uint32_t> QuantizeBvh4(const BuiltBvh4 &b4) {
   return out;
 }
 
+PackedBvh PackTraversal(const BuiltBvh4 &b4) {
+  PackedBvh out;
+  if (b4.num_nodes == 0) return out;
+  out.nodes.assign(16 * (size_t)b4.num_nodes, 0u);
+  out.num_nodes = 1;
+  // (node of b4, packed index), depth first; a node's children get their indices when it is packed.
+  std::vector<std::pair<int, int>> stack{{0, 0}};
+  while (!stack.empty()) {
+    const auto [src, dst] = stack.back();
+    stack.pop_back();
+    const float *n = &b4.nodes[32 * (size_t)src];
+    int child[4], count[4], slot[4], num_inner = 0, num = 0;
+    std::memcpy(child, n + 24, sizeof(child));
+    std::memcpy(count, n + 28, sizeof(count));
+    for (int c = 0; c < 4; ++c)
+      if (child[c] >= 0) slot[num++] = c;
+    num_inner = num;
+    for (int c = 0; c < 4; ++c)
+      if (child[c] < 0 && count[c] > 0) slot[num++] = c;
+    uint32_t *o = &out.nodes[16 * (size_t)dst];
+    uint32_t rows[6] = {0, 0, 0, 0, 0, 0}, exps = 0;
+    for (int k = 0; k < 3; ++k) {
+      const float *lo = n + 4 * (2 * k), *hi = n + 4 * (2 * k + 1);
+      double bot = kInf, top = -kInf;
+      for (int i = 0; i < num; ++i) {
+        bot = std::min(bot, (double)lo[slot[i]]);
+        top = std::max(top, (double)hi[slot[i]]);
+      }
+      if (!(bot <= top)) bot = top = 0.;  // no child at all (empty tree)
+      const double big = std::max(std::fabs(bot), std::fabs(top));
+      const double ulp = std::ldexp(1.0, std::max(-126, big > 0. ? std::ilogb(big) : -126) - 23);
+      int e = -100;
+      if (top > bot) e = std::max(e, (int)std::ceil(std::log2((top - bot) / 255.0)));
+      float org = 0.f;
+      for (;; ++e) {
+        if (e > 127) throw std::runtime_error("BVH node extent too large for 8-bit planes");
+        const double step = std::ldexp(1.0, e), margin = step * 0x1p-12 + 4. * ulp;
+        org = (float)(bot - margin);
+        while ((double)org > bot - margin) org = std::nextafter(org, -kInf);
+        bool ok = true;
+        uint32_t rlo = 0, rhi = 0;
+        for (int i = 0; i < 4; ++i) {
+          if (i >= num) {  // empty slot: an inverted box (and no primitives) misses every ray
+            rlo |= 255u << (8 * i);
+            continue;
+          }
+          const double ql = std::floor(((double)lo[slot[i]] - margin - org) / step), qh = std::ceil(((double)hi[slot[i]] + margin - org) / step);
+          ok = ok && ql >= 0. && qh <= 255.;
+          rlo |= (uint32_t)std::max(0., std::min(255., ql)) << (8 * i);
+          rhi |= (uint32_t)std::max(0., std::min(255., qh)) << (8 * i);
+        }
+        if (!ok) continue;
+        rows[2 * k] = rlo;
+        rows[2 * k + 1] = rhi;
+        break;
+      }
+      std::memcpy(&o[k], &org, 4);
+      exps |= ((uint32_t)e & 0xffu) << (8 * k);
+    }
+    o[3] = exps;
+    for (int r = 0; r < 6; ++r) o[4 + r] = rows[r];
+    const int child_base = out.num_nodes, prim_base = (int)out.prims.size();
+    std::memcpy(&o[10], &child_base, 4);
+    std::memcpy(&o[11], &prim_base, 4);
+    out.num_nodes += num_inner;
+    int first = 0;
+    for (int i = 0; i < 4; ++i) {
+      uint32_t word = i < num_inner ? 0u : 0x80000000u;
+      if (i >= num_inner && i < num) {
+        const int c = slot[i];
+        if (first + count[c] > 31) throw std::runtime_error("BVH node with more than 31 leaf primitives");
+        word |= ((1u << count[c]) - 1u) << first;
+        first += count[c];
+        for (int j = 0; j < count[c]; ++j) out.prims.push_back((uint32_t)(~child[c] + j));
+      }
+      o[12 + i] = word;
+    }
+    for (int i = num_inner - 1; i >= 0; --i) stack.push_back({child[slot[i]], child_base + i});
+  }
+  return out;
+}
+
 }  // namespace ttgpu

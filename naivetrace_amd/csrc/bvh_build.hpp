@@ -40,4 +40,19 @@ BuiltBvh4 CollapseToBvh4(const BuiltBvh &b2);
 // get q = 0.  Throws if a leaf holds more than 255 primitives or an extent exceeds 255 x 2^127.
 std::vector<uint32_t> QuantizeBvh4(const BuiltBvh4 &b4);
 
+// The tree as the device traverses it (device layout TravNode, 16 words per node): inner children of
+// a node consecutive and in its first slots, the primitives of its leaves consecutive.  Planes are
+// quantized anew: each lies outside the child's box by a margin of 2^-12 of the grid step plus 4
+// units in the last place of the coordinates.  The slab test evaluates plane * inv - org * inv as
+// q * (step * inv) + (origin * inv - org * inv): against exact arithmetic that is off by the
+// rounding of the second term, at most 2^-24 (|t| + 255 step |inv|), so by less than 2^-16 step in
+// the plane beside the relative error that the decoded form has too.
+struct PackedBvh {
+  std::vector<uint32_t> nodes;   // 16 * num_nodes
+  std::vector<uint32_t> prims;   // traversal order -> leaf-order index of BuiltBvh
+  int num_nodes = 0;
+};
+// Throws if a node's leaves hold more than 31 primitives or an extent exceeds 255 x 2^127.
+PackedBvh PackTraversal(const BuiltBvh4 &b4);
+
 }  // namespace ttgpu

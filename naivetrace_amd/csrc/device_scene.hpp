@@ -52,14 +52,24 @@ struct alignas(64) QBvh4Node {
   int4 child;
 };
 
-#ifndef TTGPU_QBVH
-#define TTGPU_QBVH 1
-#endif
-#if TTGPU_QBVH
-using SurfNode = QBvh4Node;
-#else
-using SurfNode = Bvh4Node;
-#endif
+// Traversal node of the surface BVH, 64 bytes: the quantized BVH4 laid out for few instructions per
+// visit.  A node's inner children are consecutive nodes and take its first slots, so that child
+// slot c is node child_base + c; the primitives of its leaves are consecutive too, so that the
+// leaves a ray enters are one bit mask.
+//   origin : xyz = grid origin, w = the grid steps' exponents (signed bytes x, y, z)
+//   qxy    : lo.x, hi.x, lo.y, hi.y rows, byte c = child c; qlz, qhz: the z rows.  Planes are
+//            origin + q * 2^e in exact arithmetic, outside the child's box by a margin that covers
+//            the slab test's rounding (PackTraversal)
+//   leaf   : per slot 0 for an inner child, else bit 31 and the leaf's primitives as bits of the
+//            node's primitives (bit k: prim_base + k; none for an empty slot)
+struct alignas(64) TravNode {
+  float4 origin;
+  uint4 qxy;
+  uint32_t qlz, qhz;
+  int child_base, prim_base;
+  uint4 leaf;
+};
+using SurfNode = TravNode;
 
 constexpr int kStackEntries = 96;                   // traversal stack entries per lane
 // A BVH4 node pushes at most three children, so a tree of depth D needs 3 (D + 1) entries.
@@ -161,11 +171,12 @@ struct QuadCell {
 };
 
 struct DeviceScene {
-  const SurfNode *nodes;             // surface BVH (QBvh4Node, or Bvh4Node when built with TTGPU_QBVH=0)
+  const SurfNode *nodes;           // surface BVH
   const PrimRecord *prims;         // leaf order
-  // Three copies of prims for traversal: copy k holds each triangle's vertex coordinates in
-  // the order ((k+1) mod 3, (k+2) mod 3, k), the frame of the watertight test for rays whose
-  // largest direction component is k (spheres are stored unchanged).
+  // Three copies of prims for traversal, in the order of the nodes' primitive ranges: copy k holds
+  // each triangle's vertex coordinates in the order ((k+1) mod 3, (k+2) mod 3, k), the frame of the
+  // watertight test for rays whose largest direction component is k (spheres are stored
+  // unchanged).  a.w holds the primitive's index in the leaf-order arrays.
   const PrimRecord *prims_kz;
   const int *prim_material;        // leaf order
   const float4 *prim_normals;      // leaf order, 3 per triangle (vertex normals), or null
@@ -196,8 +207,7 @@ struct DeviceScene {
   DevCamera cam;
   int sample_mode, mis_mode, max_depth;
   int algo_pt;                     // 1: pt semantics (power heuristic, Russian roulette, camera connections)
-  int persistent;                  // 1: persistent traversal kernels with dynamic ray fetch
-  int shadow_in_trace;             // 1: surface passes trace shadow rays in the next persistent closest-hit launch
+  int shadow_in_trace;             // 1: surface passes trace shadow rays in the next closest-hit launch
   int sort_shade;                  // 1: the surface shade kernel sorts each block's paths by shader class
   // guiding (guided integrator only)
   const GuideNode *guide_nodes;
@@ -277,7 +287,7 @@ enum FlagBits : uint32_t {
 
 enum Counter {
   kCountA = 0, kCountB = 1, kCountShadow = 2, kCountRecords = 3, kStatClosest = 4, kStatShadow = 5, kStatPaths = 6,
-  kStatRecordsDropped = 7, kWorkTrace = 8, kCountFree = 9, kIdentA = 10, kIdentB = 11, kCountShadow2 = 12, kSlotTicket = 13,
+  kStatRecordsDropped = 7, kCountFree = 9, kIdentA = 10, kIdentB = 11, kCountShadow2 = 12, kSlotTicket = 13,
   kNumCounters = 16
 };
 // What the slot selection of an iteration hands to the regeneration: how many freed slots take the

@@ -403,9 +403,18 @@ __device__ __forceinline__ Ray trace_entry(const PathQueues &q, const uint32_t *
   return r;
 }
 
-// One ray per thread.  With kShadow (1: plain, 2: guided) the launch also traces the shadow rays
-// of the previous shade launch (entries after the closest-hit queue), so that they need no launch
-// of their own.
+// Rays of a trace launch: each wave owns a run of consecutive entries and takes new ones from it
+// into its idle lanes whenever at most kRefill lanes still have a ray, so that long rays do not
+// leave the wave nearly empty (a model of the benchmark scene's rays: 35 % of the lanes busy in node
+// steps with one ray per lane, 47-54 % with runs of 256 rays).  Runs need no counter (a returning
+// atomic per refill cost more than the idle lanes), and finished rays' results are written together
+// at the next refill.  1080p benchmark, trace per 8-spp pass: one ray per lane with the decoded
+// quantized nodes 20.6 ms; this kernel 17.0 / 16.4 / 16.4 / 16.5 / 17.0 ms refilling at 24 / 32 /
+// 40 / 48 / 56 lanes; Cornell box 64 spp 2.76 ms, then 2.34 / 2.40 / 2.48 / 2.59 / 2.76.
+constexpr int kRefill = 32;
+
+// With kShadow (1: plain, 2: guided) the launch also traces the shadow rays of the previous shade
+// launch (entries after the closest-hit queue), so that they need no launch of their own.
 template <int kShadow>
 __global__ void __launch_bounds__(kTraceBlock, TTGPU_TRACE_WAVES) k_trace(DeviceScene sc, PathQueues q, const uint32_t *__restrict__ queue,
                                                        const uint32_t *__restrict__ count_ptr, uint32_t *stats, double *fb,
@@ -417,72 +426,37 @@ __global__ void __launch_bounds__(kTraceBlock, TTGPU_TRACE_WAVES) k_trace(Device
   const uint32_t scount = kShadow ? *q.shadow_in : 0u;
   const uint32_t count = ccount + scount;
   const bool ident = count_ptr[kIdentOffset] != 0;
-  for (uint32_t k = gtid(); k < count; k += grid_stride()) {
-    uint32_t i;
-    bool shadow;
-    const Ray r = trace_entry<kShadow>(q, queue, ident, ccount, k, i, shadow);
-    Trav t;
-    trav_init(t, r, sc.nodes, sc.num_prims, shadow);
-    while (trav_step<false>(t, sc.nodes, sc.prims_kz, stack, spill)) {}
-    if (kShadow && shadow) shadow_done<kShadow>(sc, q, i, t.hit.prim >= 0, fb, fb_sq);
-    else q.hit[i] = t.hit.prim >= 0 ? make_float4(t.hit.t, t.hit.u, t.hit.v, as_float(t.hit.prim)) : make_float4(0.f, 0.f, 0.f, as_float(-1));
-  }
-  if (gtid() == 0) {
-    atomicAdd(stats + kStatClosest, ccount);
-    if (kShadow) atomicAdd(stats + kStatShadow, scount);
-  }
-}
-
-// ---- persistent closest-hit traversal with dynamic ray fetch -------------------------------
-#ifndef TTGPU_STEPS_PER_FETCH
-#define TTGPU_STEPS_PER_FETCH 32
-#endif
-constexpr int kStepsPerFetch = TTGPU_STEPS_PER_FETCH;  // traversal steps between refills of idle lanes
-
-// With kShadow (1: plain, 2: guided), the same waves also take the shadow rays the previous shade
-// launch queued (entries count .. count + shadow count - 1 of the work counter): any-hit
-// traversal, then what k_shadow / k_shadow_guided do with the result.  Those rays then fill the
-// lanes the closest-hit rays leave idle in the launch's tail instead of running as a short launch
-// of their own.  The closest-hit and the shadow entry of one path touch disjoint state (hit
-// record; radiance, or the whole path when it ends).
-template <int kShadow>
-__global__ void __launch_bounds__(kTraceBlock, TTGPU_TRACE_WAVES) k_trace_dyn(DeviceScene sc, PathQueues q, const uint32_t *__restrict__ queue,
-                                                           const uint32_t *__restrict__ count_ptr, uint32_t *work,
-                                                           uint32_t *stats, double *fb, double *fb_sq) {
-  __shared__ int lds_stack[kLdsStack * kTraceBlock];
-  int *stack = lds_stack + threadIdx.x;
-  int spill[kSpillStack];
-  const uint32_t ccount = *count_ptr;
-  const uint32_t scount = kShadow ? *q.shadow_in : 0u;
-  const uint32_t count = ccount + scount;
-  const bool ident = count_ptr[kIdentOffset] != 0;
+  const uint32_t waves = gridDim.x * (kTraceBlock / 64), wave = blockIdx.x * (kTraceBlock / 64) + (threadIdx.x >> 6);
+  const uint32_t run = max(64u, ((count + waves - 1) / waves + 63u) & ~63u);
+  uint32_t next = __builtin_amdgcn_readfirstlane((uint32_t)min((uint64_t)wave * run, (uint64_t)count));
+  const uint32_t end = min(next + run, count);
+  const uint64_t below = (1ull << __lane_id()) - 1ull;
   Trav t;
-  bool active = false, shadow = false;
-  // Set (wave-uniform) once a fetch came back past the end: the counter only grows, so the wave
-  // fetches no more and only finishes the rays it holds.
-  bool drained = false;
+  t.node = -1;
+  t.pmask = 0;
+  bool loaded = false, shadow = false;  // loaded: the lane has a ray whose result is not written yet
   uint32_t i = 0;
   for (;;) {
-    const bool need = !active && !drained;
-    const uint32_t got = drained ? count : wave_append(work, need);
-    drained = drained || __ballot(need && got >= count) != 0;
-    if (need && got < count) {
-      const Ray r = trace_entry<kShadow>(q, queue, ident, ccount, got, i, shadow);
-      trav_init(t, r, sc.nodes, sc.num_prims, shadow);
-      active = true;
+    const bool idle = !t.active();
+    if (idle && loaded) {
+      if (kShadow && shadow) shadow_done<kShadow>(sc, q, i, t.hit.prim >= 0, fb, fb_sq);
+      else q.hit[i] = t.hit.prim >= 0 ? make_float4(t.hit.t, t.hit.u, t.hit.v, as_float(t.hit.prim)) : make_float4(0.f, 0.f, 0.f, as_float(-1));
+      loaded = false;
     }
-    if (__ballot(active) == 0) break;
-    for (int it = 0; it < kStepsPerFetch && active; ++it) {
-      if (!trav_step<false>(t, sc.nodes, sc.prims_kz, stack, spill)) {
-        if (kShadow && shadow) {
-          shadow_done<kShadow>(sc, q, i, t.hit.prim >= 0, fb, fb_sq);
-        } else {
-          q.hit[i] = t.hit.prim >= 0 ? make_float4(t.hit.t, t.hit.u, t.hit.v, as_float(t.hit.prim))
-                                     : make_float4(0.f, 0.f, 0.f, as_float(-1));
-        }
-        active = false;
+    const uint64_t free_lanes = __ballot(idle);
+    if (next < end) {
+      const uint32_t k = next + (uint32_t)__popcll(free_lanes & below);
+      if (idle && k < end) {
+        const Ray r = trace_entry<kShadow>(q, queue, ident, ccount, k, i, shadow);
+        trav_init(t, r, sc.num_prims, shadow, stack);
+        loaded = true;
       }
+      next = min(next + (uint32_t)__popcll(free_lanes), end);
+    } else if (free_lanes == ~0ull) {
+      break;
     }
+    const int stop = next < end ? kRefill : 0;
+    while ((int)__popcll(__builtin_amdgcn_ballot_w64(t.active())) > stop) trav_advance(t, sc.nodes, sc.prims_kz, stack, spill);
   }
   if (gtid() == 0) {
     atomicAdd(stats + kStatClosest, ccount);
@@ -2515,8 +2489,6 @@ __global__ void __launch_bounds__(kTraceBlock) k_bdpt(DeviceScene sc, uint64_t f
 }
 
 // ---- host-side launchers ------------------------------------------------------------------
-static int g_trace_blocks = 0;
-
 hipError_t UploadSpectralTables(const float *to_rgb, const float *smits) {
   hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(c_spec_to_rgb), to_rgb, sizeof(float) * 3 * kNBins);
   if (e != hipSuccess) return e;
@@ -2559,38 +2531,16 @@ void LaunchRegen(const DeviceScene &sc, const PathQueues &q, const RegenArgs &a,
 void LaunchReport(const PathQueues &q, PassReport *host, hipStream_t st) {
   hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, st, q, host);
 }
-// Workgroups that fit on the device at once for a persistent kernel (computed on first use).
-template <class K>
-static int ResidentBlocks(K kernel, int block) {
-  int dev = 0, per_cu = 0;
-  hipDeviceProp_t prop;
-  if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, 0) != hipSuccess || per_cu < 1)
-    return 1024;
-  return per_cu * prop.multiProcessorCount;
-}
+// Blocks of a trace launch: four times what is resident at five waves per SIMD, so that short runs
+// (about 100-200 rays of a 4 M-path wavefront) even out at the launch's end; or one wave per 64
+// rays when there are fewer.  1080p benchmark with 2560 / 4096 / 5120 / 7680 / 10240 / 16384 blocks:
+// 16.8 / 17.7 / 16.5 / 16.1 / 15.9 / 16.0 ms per pass.
+constexpr int kTraceGrid = 10240;
 
 void LaunchTrace(const DeviceScene &sc, const PathQueues &q, const uint32_t *queue, const uint32_t *count, uint32_t max_count,
                  double *fb, double *fb_sq, bool with_shadow, hipStream_t st) {
-  if (sc.persistent) {
-    hipLaunchKernelGGL(k_reset_counter, dim3(1), dim3(64), 0, st, q.counters, (int)kWorkTrace);
-    const bool guided = sc.guide_cells || sc.guide_qcells || q.gmix;
-    if (with_shadow && guided) {
-      static const int resident = ResidentBlocks(k_trace_dyn<2>, kTraceBlock);
-      hipLaunchKernelGGL(k_trace_dyn<2>, dim3(Blocks(max_count, kTraceBlock, resident)), dim3(kTraceBlock), 0, st, sc, q, queue,
-                         count, q.counters + kWorkTrace, q.counters, fb, fb_sq);
-    } else if (with_shadow) {
-      static const int resident = ResidentBlocks(k_trace_dyn<1>, kTraceBlock);
-      hipLaunchKernelGGL(k_trace_dyn<1>, dim3(Blocks(max_count, kTraceBlock, resident)), dim3(kTraceBlock), 0, st, sc, q, queue,
-                         count, q.counters + kWorkTrace, q.counters, fb, fb_sq);
-    } else {
-      static const int resident = ResidentBlocks(k_trace_dyn<0>, kTraceBlock);
-      hipLaunchKernelGGL(k_trace_dyn<0>, dim3(Blocks(max_count, kTraceBlock, resident)), dim3(kTraceBlock), 0, st, sc, q, queue,
-                         count, q.counters + kWorkTrace, q.counters, fb, fb_sq);
-    }
-    return;
-  }
-  const dim3 grid(Blocks(max_count, kTraceBlock, 16384)), block(kTraceBlock);
+  // With shadow rays, up to max_count of each kind.
+  const dim3 grid(Blocks((with_shadow ? 2ull : 1ull) * max_count, kTraceBlock, kTraceGrid)), block(kTraceBlock);
   const bool guided = sc.guide_cells || sc.guide_qcells || q.gmix;
   if (with_shadow && guided) hipLaunchKernelGGL(k_trace<2>, grid, block, 0, st, sc, q, queue, count, q.counters, fb, fb_sq);
   else if (with_shadow) hipLaunchKernelGGL(k_trace<1>, grid, block, 0, st, sc, q, queue, count, q.counters, fb, fb_sq);

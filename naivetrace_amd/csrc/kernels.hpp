@@ -30,7 +30,7 @@ void LaunchRegen(const DeviceScene &sc, const PathQueues &q, const RegenArgs &a,
 // Counters and the stack-overflow flag (then cleared) to the page-locked report.
 void LaunchReport(const PathQueues &q, PassReport *host, hipStream_t st);
 size_t SelectTempBytes(uint32_t capacity);
-// with_shadow: the persistent traversal also takes the shadow rays of the previous shade launch
+// with_shadow: the launch also takes the shadow rays of the previous shade launch
 // (ShadowInTrace), and LaunchShadow is not called.
 void LaunchTrace(const DeviceScene &sc, const PathQueues &q, const uint32_t *queue, const uint32_t *count, uint32_t max_count,
                  double *fb, double *fb_sq, bool with_shadow, hipStream_t st);

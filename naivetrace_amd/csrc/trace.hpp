@@ -99,12 +99,14 @@ TT_HD bool intersect_triangle_k(const RayPre &p, float3 A, float3 B, float3 C, f
   float U = Cx * By - Cy * Bx;
   float V = Ax * Cy - Ay * Cx;
   float W = Bx * Ay - By * Ax;
-  if (U == 0.f || V == 0.f || W == 0.f) {
+  // Comparisons through minima and maxima (exact; NaNs end at the determinant): a third of the
+  // instructions of one compare per edge and sign.
+  if (fminf(fminf(fabsf(U), fabsf(V)), fabsf(W)) == 0.f) {
     U = (float)((double)Cx * (double)By - (double)Cy * (double)Bx);
     V = (float)((double)Ax * (double)Cy - (double)Ay * (double)Cx);
     W = (float)((double)Bx * (double)Ay - (double)By * (double)Ax);
   }
-  if ((U < 0.f || V < 0.f || W < 0.f) && (U > 0.f || V > 0.f || W > 0.f)) return false;
+  if (fminf(fminf(U, V), W) < 0.f && fmaxf(fmaxf(U, V), W) > 0.f) return false;
   const float det = U + V + W;
   if (det == 0.f) return false;
   const float Az = p.Sz * Akz, Bz = p.Sz * Bkz, Cz = p.Sz * Ckz;
@@ -202,7 +204,7 @@ TT_HD void box2(const BvhNode &n, const RayPre &p, float tmax, float &tl, float 
   tr = rmin <= rmax ? rmin : as_float(0x7f800000);
 }
 
-// ---- BVH4 traversal ----------------------------------------------------------------------
+// ---- BVH4 traversal of the intermediate layouts (run on the host by the checks of the BVH build) --
 // A ray's traversal state; one step is one node visit or one primitive test, so the loop below
 // and the persistent kernels with dynamic ray fetch (Aila & Laine 2009) share the same code.
 // `cur` holds the node to visit next and `rec` the primitive to test next, both already fetched:
@@ -224,7 +226,6 @@ struct TravT {
   int kofs;             // p.kz x the number of primitives: this ray's copy of the records
   bool any;             // any-hit query: finished at the first hit
 };
-using Trav = TravT<SurfNode>;
 
 template <class Node>
 TT_HD void trav_init(TravT<Node> &t, const Ray &r, const Node *__restrict__ nodes, int num_prims, bool any_hit = false) {
@@ -427,6 +428,185 @@ TT_HD bool traverse(const Node *__restrict__ nodes, const PrimRecord *__restrict
   TravT<Node> t;
   trav_init(t, r, nodes, num_prims);
   while (trav_step<kAnyHit>(t, nodes, prims, stack, spill)) {}
+  hit = t.hit;
+  return t.hit.prim >= 0;
+}
+
+// ---- traversal of the packed nodes ------------------------------------------------------------
+// Issue-bound as one ray per lane with the intermediate layout (VALU work in 95-100 % of SIMD cycles,
+// 5.4e8 instructions per launch of the 1080p benchmark): what counted was instructions per step times
+// the steps a wave makes, which its busiest lanes set.  Now 2.7e8 instructions, VALU busy 61 % and the
+// vector-memory return path 80 % (a scattered 16-byte load of 32 lanes takes 30 cycles of it, so a
+// node step's four take 120 of the 173 x 4 its arithmetic takes on each of the four SIMDs).  Three
+// things keep both low:
+//  * the packed layout.  Child boxes take two instructions per plane (byte to float, fma onto
+//    per-node constants); entry distances carry the slot in their low two bits, so sorting the four
+//    is five integer min / max pairs and a child's index one addition; entered leaves are bits of
+//    one mask.  A node step is 173 VALU instructions, with the decoded planes, compare-and-swap pairs
+//    and leaf list of the intermediate layout it was 233.
+//  * one kind of step per iteration.  Lanes with primitives to test and lanes with a node to visit
+//    do not advance together: the wave takes the kind of step that more of its lanes wait for, and
+//    the others wait (their fetch is on its way meanwhile).  A model of 64-lane waves over the
+//    benchmark scene's rays counted 146 issued instructions per ray for this, 173 for both kinds in
+//    every iteration.
+//  * waves take new rays as theirs end (k_trace).
+// `node` is the node to visit next and `pmask` the primitives to test before.  A step loads what it
+// works on when it starts: with four or five waves per SIMD the others' arithmetic covers the
+// latency.  Fetching a step ahead kept 28 more registers alive across the loop, and the copies that
+// merged them between the two kinds of step waited for the fetch anyway.
+struct Trav {
+  RayPre p;
+  float3 org, dir;
+  float tmax;
+  HitRec hit;
+  int sp;            // stack top, in entries x kTraceBlock
+  int node;          // -1: none
+  uint32_t pmask;
+  int pbase;         // record of pmask's bit 0
+  int kofs;          // p.kz x the number of primitives: this ray's copy of the records
+  bool any;          // any-hit query: finished at the first hit
+  TT_HD bool wants_prim() const { return pmask != 0; }
+  TT_HD bool wants_node() const { return pmask == 0 && node >= 0; }
+  TT_HD bool active() const { return pmask != 0 || node >= 0; }
+};
+
+TT_HD int first_bit(uint32_t m) { return __builtin_ctz(m); }
+TT_HD void sort2(uint32_t &a, uint32_t &b) {
+  const uint32_t lo = a < b ? a : b, hi = a < b ? b : a;
+  a = lo;
+  b = hi;
+}
+
+TT_HD void trav_init(Trav &t, const Ray &r, int num_prims, bool any_hit, int *stack) {
+  t.any = any_hit;
+  t.p = precompute(r);
+  t.kofs = t.p.kz * num_prims;
+  t.org = r.org;
+  t.dir = r.dir;
+  t.tmax = r.tmax;
+  t.hit.prim = -1;
+  stack[0] = -1;  // popped when the tree is exhausted
+  t.sp = kTraceBlock;
+  t.node = 0;
+  t.pmask = 0;
+  t.pbase = 0;
+}
+
+// Primitive step: tests the first primitive of the mask.
+TT_HD void trav_prim(Trav &t, const PrimRecord *prims) {
+  PrimRecord cur = prims[t.pbase + first_bit(t.pmask)];
+  t.pmask &= t.pmask - 1u;
+#if defined(__HIP_DEVICE_COMPILE__)
+  // The whole record in three wide loads at once, rather than its kind first and the rest in pieces
+  // behind the branch on it.
+  asm volatile("" : "+v"(cur.a.x), "+v"(cur.a.y), "+v"(cur.a.z), "+v"(cur.a.w), "+v"(cur.b.x), "+v"(cur.b.y), "+v"(cur.b.z),
+                    "+v"(cur.b.w), "+v"(cur.c.x), "+v"(cur.c.y), "+v"(cur.c.z), "+v"(cur.c.w));
+#endif
+  Ray r;
+  r.org = t.org;
+  r.dir = t.dir;
+  float th, u, v;
+  if (intersect_prim_k(cur, t.p, r, t.tmax, th, u, v)) {
+    t.tmax = th;
+    t.hit.t = th; t.hit.u = u; t.hit.v = v; t.hit.prim = as_int(cur.a.w);
+    if (t.any) {
+      t.pmask = 0;
+      t.node = -1;
+    }
+  }
+}
+
+// Node step: slab test of the four children; inner children sorted by entry distance, the nearest
+// visited next and the others pushed far to near; the mask of the entered leaves' primitives.
+TT_HD void trav_node(Trav &t, const TravNode *nodes, int *stack, int *spill) {
+  const TravNode n = nodes[t.node];
+  const uint32_t e = as_uint(n.origin.w);
+  const float ax = ldexpf(t.p.inv.x, (int)(int8_t)e), ay = ldexpf(t.p.inv.y, (int)(int8_t)(e >> 8)),
+              az = ldexpf(t.p.inv.z, (int)(int8_t)(e >> 16));
+  const float bnx = fmaf(n.origin.x, t.p.inv.x, -t.p.onear.x), bfx = fmaf(n.origin.x, t.p.inv.x, -t.p.ofar.x);
+  const float bny = fmaf(n.origin.y, t.p.inv.y, -t.p.onear.y), bfy = fmaf(n.origin.y, t.p.inv.y, -t.p.ofar.y);
+  const float bnz = fmaf(n.origin.z, t.p.inv.z, -t.p.onear.z), bfz = fmaf(n.origin.z, t.p.inv.z, -t.p.ofar.z);
+  // Rows of the planes the ray enters and leaves by, per axis.
+  const uint32_t nx = t.p.negx ? n.qxy.y : n.qxy.x, fx = t.p.negx ? n.qxy.x : n.qxy.y;
+  const uint32_t ny = t.p.negy ? n.qxy.w : n.qxy.z, fy = t.p.negy ? n.qxy.z : n.qxy.w;
+  const uint32_t nz = t.p.negz ? n.qhz : n.qlz, fz = t.p.negz ? n.qlz : n.qhz;
+  const uint32_t leaf[4] = {n.leaf.x, n.leaf.y, n.leaf.z, n.leaf.w};
+  const float pad = 1.0000004f;  // conservative far bound, 1 + 2 gamma(3) (Ize 2013)
+  uint32_t key[4], mask = 0;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    auto q = [c](uint32_t row) { return (float)((row >> (8 * c)) & 0xffu); };
+    const float tn = fmaxf(fmaxf(fmaf(q(nx), ax, bnx), fmaf(q(ny), ay, bny)), fmaxf(fmaf(q(nz), az, bnz), 0.f));
+    const float tf = fminf(fminf(fmaf(q(fx), ax, bfx), fmaf(q(fy), ay, bfy)), fminf(fmaf(q(fz), az, bfz), t.tmax)) * pad;
+    const bool ok = tn <= tf;
+    // Distance with the slot in its low bits; leaf and empty slots (bit 31 of their word) and
+    // missed children sort behind every inner one, as negative integers.
+    const uint32_t k = (as_uint(tn) & ~3u) | (uint32_t)c;
+    key[c] = ok ? (k > leaf[c] ? k : leaf[c]) : 0xffffffffu;
+    mask |= ok ? leaf[c] : 0u;
+  }
+  sort2(key[0], key[1]);
+  sort2(key[2], key[3]);
+  sort2(key[0], key[2]);
+  sort2(key[1], key[3]);
+  sort2(key[1], key[2]);
+  const int base = n.child_base;
+  if (t.sp + 3 * kTraceBlock <= kLdsStack * kTraceBlock) {
+    // All three writes land in the LDS part: each writes at the top and only a child moves it, so
+    // an absent child's write is overwritten or left above the top.
+#pragma unroll
+    for (int c = 3; c >= 1; --c) {
+      stack[t.sp] = base + (int)(key[c] & 3u);
+      t.sp += (int)key[c] >= 0 ? kTraceBlock : 0;
+    }
+  } else {
+#pragma unroll
+    for (int c = 3; c >= 1; --c) {
+      if ((int)key[c] < 0) continue;
+      const int id = base + (int)(key[c] & 3u), k = t.sp / kTraceBlock;
+      if (k < kLdsStack) stack[t.sp] = id;
+      else if (k < kStackEntries) spill[k - kLdsStack] = id;
+      if (k < kStackEntries) t.sp += kTraceBlock;
+      else TTGPU_STACK_OVERFLOW();
+    }
+  }
+  int next = base + (int)(key[0] & 3u);
+  if ((int)key[0] < 0) {
+    t.sp -= kTraceBlock;
+    // An LDS read (the top's entry, or the last LDS entry when the top lies in the spill part)
+    // rather than one generic load through a selected address space.
+    const int top = t.sp;
+    next = stack[top < (kLdsStack - 1) * kTraceBlock ? top : (kLdsStack - 1) * kTraceBlock];
+    if (top >= kLdsStack * kTraceBlock) next = spill[top / kTraceBlock - kLdsStack];
+  }
+  t.pmask = mask & 0x7fffffffu;
+  t.pbase = t.kofs + n.prim_base;
+  t.node = next;
+}
+
+// One iteration of the wave: the kind of step more of its lanes wait for.
+TT_HD void trav_advance(Trav &t, const TravNode *nodes, const PrimRecord *prims, int *stack, int *spill) {
+  const bool wp = t.wants_prim(), wn = t.wants_node();
+#if defined(__HIP_DEVICE_COMPILE__)
+  const bool take_node = (int)__popcll(__builtin_amdgcn_ballot_w64(wn)) >= (int)__popcll(__builtin_amdgcn_ballot_w64(wp));
+#else
+  const bool take_node = wn;
+#endif
+  if (take_node) {
+    if (wn) trav_node(t, nodes, stack, spill);
+  } else {
+    if (wp) trav_prim(t, prims);
+  }
+}
+
+// Whole traversal of one ray (closest hit, or any hit with kAnyHit); true if something was hit.
+template <bool kAnyHit>
+TT_HD bool traverse(const TravNode *__restrict__ nodes, const PrimRecord *__restrict__ prims, int num_prims, const Ray &r, int *stack,
+                    HitRec &hit) {
+  int spill[kSpillStack];
+  Trav t;
+  trav_init(t, r, num_prims, kAnyHit, stack);
+  while (t.active()) trav_advance(t, nodes, prims, stack, spill);
   hit = t.hit;
   return t.hit.prim >= 0;
 }

@@ -387,14 +387,9 @@ void BuildGeometry(ttgpu_handle *h, const ttgpu_scene &s, const std::vector<int6
     const BuiltBvh4 b4 = CollapseToBvh4(bvh);
     if (b4.max_depth > kMaxBvh4Depth)
       throw std::runtime_error("BVH4 deeper than the traversal stack (" + std::to_string(kMaxBvh4Depth) + " levels)");
-#if TTGPU_QBVH
-    const std::vector<uint32_t> qnodes = QuantizeBvh4(b4);
-    h->dsc.nodes = h->Upload((const QBvh4Node *)qnodes.data(), b4.num_nodes);
-    h->stats.scene_bytes += qnodes.size() * 4;
-#else
-    h->dsc.nodes = h->Upload((const Bvh4Node *)b4.nodes.data(), b4.num_nodes);
-    h->stats.scene_bytes += b4.nodes.size() * 4;
-#endif
+    const PackedBvh packed = PackTraversal(b4);
+    h->dsc.nodes = h->Upload((const TravNode *)packed.nodes.data(), packed.num_nodes);
+    h->stats.scene_bytes += packed.nodes.size() * 4;
     h->stats.bvh_nodes = b4.num_nodes;
     h->dsc.prims = h->Upload(recs.data(), recs.size());
     {
@@ -405,12 +400,14 @@ void BuildGeometry(ttgpu_handle *h, const ttgpu_scene &s, const std::vector<int6
           const float c[3] = {v.x, v.y, v.z};
           return make_float4(c[kx], c[ky], c[k], v.w);
         };
-        for (size_t i = 0; i < recs.size(); ++i) {
-          PrimRecord r = recs[i];
+        for (size_t i = 0; i < packed.prims.size(); ++i) {
+          PrimRecord r = recs[packed.prims[i]];
+          const int index = (int)packed.prims[i];
+          std::memcpy(&r.a.w, &index, 4);
           int kind;
           std::memcpy(&kind, &r.b.w, 4);
           if (kind == 0) {
-            r.a = perm(r.a);
+            r.a = perm(r.a);  // keeps w
             r.b = perm(r.b);
             r.c = perm(r.c);
           }
@@ -763,11 +760,6 @@ void BuildTables(ttgpu_handle *h, const ttgpu_scene &s, double bb_diag) {
   dc.xmin = (float)-a; dc.ymin = (float)-b; dc.xper = (float)(2. * a / W); dc.yper = (float)(2. * b / H);
   dc.fish_delta = (float)(2. / std::min(W, H));
   dc.width = W; dc.height = H;
-  // Closest-hit traversal: one ray per thread, or persistent waves with dynamic ray fetch when
-  // TTGPU_PERSISTENT_TRAVERSAL=1.  Once the shadow rays share the closest-hit launch, one ray per
-  // thread is the faster of the two on every scene measured (36 to 1 M triangles).
-  const char *pt = std::getenv("TTGPU_PERSISTENT_TRAVERSAL");
-  h->dsc.persistent = (pt && pt[0] == '1') ? 1 : 0;
   // Surface passes trace each iteration's shadow rays in the next closest-hit launch unless
   // TTGPU_SHADOW_IN_TRACE=0.
   const char *sit = std::getenv("TTGPU_SHADOW_IN_TRACE");
