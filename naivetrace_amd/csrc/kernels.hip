@@ -2011,18 +2011,22 @@ __global__ void k_guide_pdf_at(DeviceScene sc, int64_t n, const float *pos, cons
 }
 
 // ---- bdpt: bidirectional path tracing (renderingalgorithms_pathtracing.hxx:341-700) ----------
-// One thread per camera sample: eye and light subpaths on the random-walk framework in private
-// arrays, then every strategy of BdptWorker::RenderPixel: each camera / scatter vertex of the eye
-// subpath connects to a fresh light sample and to the light subpath's vertices 1..; eye vertices on
-// emitters count as light hits; connections from the camera are splatted to their pixel.  MIS: the
-// power heuristic over all strategies of the full path, strategies with >= 2 eye vertices weighted
-// by 1 / pixel count, strategies next to a delta vertex excluded; the densities of every strategy
-// are computed afresh per connection (FP64 products).  Surfaces in vacuum, pinhole camera.
-#ifndef TTGPU_BDPT_MAX_VERTS
-#define TTGPU_BDPT_MAX_VERTS 17
-#endif
-constexpr int kBdptMaxVerts = TTGPU_BDPT_MAX_VERTS;  // max_ray_depth + 1 <= this (checked on the host)
-static_assert(kBdptMaxVerts == kBdptMaxVertices, "the host check and the kernel's arrays must agree");
+// Eye and light subpaths on the random-walk framework, then every strategy of
+// BdptWorker::RenderPixel: each camera / scatter vertex of the eye subpath connects to a fresh light
+// sample and to the light subpath's vertices 1..; eye vertices on emitters count as light hits;
+// connections from the camera are splatted to their pixel.  MIS: the power heuristic over all
+// strategies of the full path, strategies with >= 2 eye vertices weighted by 1 / pixel count,
+// strategies next to a delta vertex excluded; every density is that of the connection at hand (FP64
+// products).  Surfaces in vacuum, pinhole camera.
+//
+// Three kernels per chunk of samples.  k_bdpt_walk (one thread per sample) walks both subpaths,
+// writes their vertices, counts the light hits and lists the connections; k_bdpt_connect takes one
+// connection per thread, so that the few samples with many connections do not hold a wave;
+// k_bdpt_finish adds the samples to their pixels.  Each vertex carries the products of the densities
+// before it and the summed squares of the strategies that connect earlier on its subpath, so a
+// connection's MIS weight takes a dozen FP64 operations instead of a product per strategy.  As one
+// kernel with private arrays (5.9 KB of scratch per lane, 232 registers, 23 % of the lanes active, 72
+// % of the wave cycles waiting) 262,144 samples of the Cornell box took 4.75 ms.
 enum { kBvCamera = 0, kBvSurf = 1, kBvArea = 2, kBvEnv = 3, kBvPoint = 4 };
 
 struct BdptVertex {
@@ -2031,10 +2035,68 @@ struct BdptVertex {
   float4 beta;   // path weight
   float4 Le;     // kBvArea / kBvEnv radiance, kBvPoint intensity
   float pdf_walk;   // density of this vertex from its own subpath's side
-  float pdf_other;  // density from the opposite side (inner vertices, set by the walk)
   int type;
   int delta;     // the walk left this vertex through a delta lobe
+  // MIS over the strategies that connect within the subpath 0 .. this vertex (index n):
+  double prod;   // product of the subpath's densities pdf_walk[0 .. n]
+  double sum;    // sum over j <= n - 1 of (w_j prod[j - 1] x the opposite side's densities of j .. n - 2)^2,
+                 // j vertices on the subpath's own side, skipping j next to a delta vertex
 };
+
+// A vertex in memory: six float4 in the order of BdptVertex's parts.
+constexpr int kBdptRows = 6;
+enum { kBdptEye = 0, kBdptLight = 1, kBdptDirect = 2 };
+__device__ __forceinline__ float4 *bdpt_row(const BdptWork &w, int kind, int k, uint32_t s) {
+  return w.verts + ((size_t)(kind * w.max_nodes + k) * w.capacity + s) * kBdptRows;
+}
+// type in bits 0-2, delta bit 3, n = -ng bit 4, material from bit 5.
+__device__ __forceinline__ int bdpt_meta(const BdptVertex &v) {
+  const bool flip = (v.type == kBvSurf) && (v.h.n.x != v.h.ng.x || v.h.n.y != v.h.ng.y || v.h.n.z != v.h.ng.z);
+  return v.type | (v.delta << 3) | ((flip ? 1 : 0) << 4) | (v.type == kBvSurf ? v.h.material << 5 : 0);
+}
+__device__ __forceinline__ float4 pack_doubles(double a, double b) {
+  return make_float4(as_float(__double2loint(a)), as_float(__double2hiint(a)), as_float(__double2loint(b)), as_float(__double2hiint(b)));
+}
+__device__ __forceinline__ double unpack_double(float lo, float hi) { return __hiloint2double(as_int(hi), as_int(lo)); }
+__device__ __forceinline__ void bdpt_store(const BdptWork &w, int kind, int k, uint32_t s, const BdptVertex &v) {
+  float4 *r = bdpt_row(w, kind, k, s);
+  r[0] = make_float4(v.h.pos.x, v.h.pos.y, v.h.pos.z, v.h.offset);
+  r[1] = make_float4(v.h.ng.x, v.h.ng.y, v.h.ng.z, as_float(bdpt_meta(v)));
+  if (kind == kBdptDirect) {
+    r[2] = v.Le;
+  } else {
+    r[2] = make_float4(v.h.ns.x, v.h.ns.y, v.h.ns.z, 0.f);
+    r[3] = make_float4(v.wi.x, v.wi.y, v.wi.z, 0.f);
+  }
+  r[4] = v.beta;
+  r[5] = pack_doubles(v.prod, v.sum);
+}
+__device__ __forceinline__ void bdpt_unpack_geometry(const float4 *r, BdptVertex &v) {
+  const float4 a = r[0], b = r[1];
+  const int meta = as_int(b.w);
+  v.h.pos = xyz(a);
+  v.h.offset = a.w;
+  v.h.ng = xyz(b);
+  v.type = meta & 7;
+  v.delta = (meta >> 3) & 1;
+  v.h.n = (meta >> 4) & 1 ? -v.h.ng : v.h.ng;
+  v.h.material = meta >> 5;
+}
+__device__ __forceinline__ void bdpt_load(const BdptWork &w, int kind, int k, uint32_t s, BdptVertex &v) {
+  const float4 *r = bdpt_row(w, kind, k, s);
+  bdpt_unpack_geometry(r, v);
+  const float4 c = r[2], d = r[3], f = r[5];
+  if (kind == kBdptDirect) {
+    v.Le = c;
+    v.h.ns = v.h.ng;
+  } else {
+    v.h.ns = xyz(c);
+    v.wi = xyz(d);
+  }
+  v.beta = r[4];
+  v.prod = unpack_double(f.x, f.y);
+  v.sum = unpack_double(f.z, f.w);
+}
 
 struct BdptCtx {
   const DeviceScene &sc;
@@ -2161,14 +2223,30 @@ __device__ __forceinline__ float bv_scatter_pdf(const BdptCtx &c, const BdptVert
   return pdf;
 }
 
-// BdptForwardTrace (:598-646) from the last vertex of `path` with the sampled direction `dir`.
-__device__ void bv_walk(const BdptCtx &c, BdptVertex *path, int &n, float3 org, float3 dir, float pdf, bool pdf_delta, float4 factor,
-                        bool importance, Pcg &rng, int *lds_stack, uint32_t &rays) {
+__device__ __forceinline__ double sq(double x) { return x * x; }
+
+// Adds every lane's count with one atomic per wave (called by whole waves).
+__device__ __forceinline__ void wave_stat(uint32_t *counter, uint32_t n) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+  if ((threadIdx.x & 63) == 0 && n) atomicAdd(counter, n);
+}
+
+// BdptForwardTrace (:598-646) from `cur`, the subpath's first vertex (index 0, already stored), with
+// the sampled direction `dir`; stores the vertices and returns their number.  Eye subpaths add their
+// light hits (HandleLightHit, :526-556) to `acc`.
+template <bool kLight>
+__device__ int bv_walk(const BdptCtx &c, const BdptWork &w, uint32_t s, BdptVertex cur, float3 org, float3 dir, float pdf, float4 factor,
+                       bool light_delta, Pcg &rng, int *lds_stack, uint32_t &rays, float4 &acc) {
   const DeviceScene &sc = c.sc;
-  const int max_nodes = min(sc.max_depth + 1, kBdptMaxVerts);
+  constexpr int kKind = kLight ? kBdptLight : kBdptEye;
+  BdptVertex prev;
+  int n = 1;
   float carry = 1.f;
+  bool pdf_delta = false;
+  const double inv = c.inv_npix;
   for (;;) {
-    if (all_zero(factor) || !(pdf > 0.f) || !isfinite(factor.x + factor.y + factor.z + factor.w)) return;
+    if (all_zero(factor) || !(pdf > 0.f) || !isfinite(factor.x + factor.y + factor.z + factor.w)) return n;
     Ray r;
     r.org = org;
     r.dir = dir;
@@ -2176,27 +2254,28 @@ __device__ void bv_walk(const BdptCtx &c, BdptVertex *path, int &n, float3 org, 
     HitRec hr;
     ++rays;
     const bool hit = traverse<false>(sc.nodes, sc.prims_kz, sc.num_prims, r, lds_stack, hr);
-    if (!hit && (importance || sc.num_envs == 0)) return;  // light subpaths end at the environment
-    BdptVertex &cur = path[n - 1];
-    cur.delta = pdf_delta ? 1 : 0;
+    if (!hit && (kLight || sc.num_envs == 0)) return n;  // light subpaths end at the environment
+    if (pdf_delta) {
+      cur.delta = 1;
+      bdpt_row(w, kKind, n - 1, s)[1].w = as_float(bdpt_meta(cur));
+    }
     factor = carry * factor;
     carry = 1.f;
-    bool survive = n + 1 < max_nodes;
+    bool survive = n + 1 < w.max_nodes;
     if (survive && n + 1 > 5) {
       const float ps = fminf(0.9f, fmaxf(fmaxf(factor.x, factor.y), fmaxf(factor.z, factor.w)));
       if (rng.uniform() > ps) survive = false;
       else if (c.consistent_rr) carry = 1.f / ps;
       else factor = factor * (1.f / ps);
     }
-    BdptVertex &v = path[n];
+    BdptVertex v;
     v.beta = cur.beta * factor;
     v.delta = 0;
-    v.pdf_other = 0.f;
+    float penv = 0.f;
     if (!hit) {
       v.type = kBvEnv;
       v.h.pos = -dir;
-      float pe;
-      v.Le = env_eval(sc, -dir, c.bins, &pe);
+      v.Le = env_eval(sc, -dir, c.bins, &penv);
       v.pdf_walk = pdf;
     } else {
       v.type = kBvSurf;
@@ -2204,288 +2283,308 @@ __device__ void bv_walk(const BdptCtx &c, BdptVertex *path, int &n, float3 org, 
       v.wi = dir;
       v.pdf_walk = pdf * bv_conv(cur, v, dir, hr.t);
     }
-    if (n >= 2 && cur.type == kBvSurf) {
-      BdptVertex &prev = path[n - 2];
-      const float rp = pdf_delta ? pdf : bv_scatter_pdf(c, cur, dir, -cur.wi, importance);
+    // The opposite side's density of vertex n - 2, now that the scatter at n - 1 is known, and the
+    // sums of the strategies that connect earlier.
+    if (n >= 2) {
+      const float rp = pdf_delta ? pdf : bv_scatter_pdf(c, cur, dir, -cur.wi, kLight);
       float3 o, d;
       float len;
       bv_segment(c, cur, prev, o, d, len);
-      prev.pdf_other = rp * bv_conv(cur, prev, d, len);
+      const double other = rp * bv_conv(cur, prev, d, len);
+      v.sum = cur.sum * sq(other);
+      if (!prev.delta && !cur.delta) v.sum += sq((!kLight && n - 1 >= 2 ? inv : 1.) * prev.prod);
+    } else {
+      v.sum = kLight && !light_delta && !cur.delta ? 1. : 0.;
+    }
+    v.prod = cur.prod * v.pdf_walk;
+    if (v.type == kBvSurf) bdpt_store(w, kKind, n, s, v);
+    if constexpr (!kLight) {
+      float4 Le = f4(0.f);
+      float p_start = 0.f, p_emit = 0.f;
+      BdptVertex as_light = v;
+      if (v.type == kBvEnv) {
+        Le = v.Le;
+        p_start = penv * sc.type_probs[0];
+        p_emit = bv_emission_pdf(c, v, v.h.pos);
+      } else if (sc.materials[v.h.material].emitter >= 0) {
+        const DevEmitter &em = sc.emitters[sc.materials[v.h.material].emitter];
+        const bool facing = dot(v.h.ng, -v.wi) > 0.f;
+        if (em.kind == TTGPU_AREA_UNIFORM && facing) Le = take(em.radiance, c.bins);
+        p_start = sc.area_pick_prob / sc.prim_area[v.h.prim];
+        as_light.type = kBvArea;
+        p_emit = facing ? 1.f / (2.f * kPi) : 0.f;
+      }
+      if (!all_zero(Le)) {
+        float3 o2, d2;
+        float l2;
+        bv_segment(c, as_light, cur, o2, d2, l2);
+        const double pl_prev = (double)p_emit * bv_conv(as_light, cur, d2, l2);
+        const double p_hit = sq((n + 1 >= 2 ? inv : 1.) * v.prod);  // all n + 1 vertices from the eye
+        double den = p_hit + v.sum * sq(pl_prev * p_start);
+        if (!cur.delta) den += sq((n >= 2 ? inv : 1.) * cur.prod * p_start);
+        if (den > 0.) acc = acc + (float)(p_hit / den) * (v.beta * Le);
+      }
     }
     ++n;
-    if (!survive || v.type == kBvEnv) return;
+    if (!survive || v.type == kBvEnv) return v.type == kBvEnv ? n - 1 : n;
     const DevShader &shd = sc.shaders[sc.materials[v.h.material].shader];
-    const Scatter s = sample_bsdf(shd, v.h, -v.wi, c.bins, 0.f, c.lambda0, rng, importance);
-    factor = (bv_corr(v, s.dir, importance) / s.pdf) * s.value;
-    pdf = s.pdf;
-    pdf_delta = s.delta;
-    dir = s.dir;
-    org = offset_origin(v.h, s.dir);
+    const Scatter sct = sample_bsdf(shd, v.h, -v.wi, c.bins, 0.f, c.lambda0, rng, kLight);
+    factor = (bv_corr(v, sct.dir, kLight) / sct.pdf) * sct.value;
+    pdf = sct.pdf;
+    pdf_delta = sct.delta;
+    dir = sct.dir;
+    org = offset_origin(v.h, sct.dir);
+    prev = cur;
+    cur = v;
   }
 }
 
-// MIS weight of the strategy with s eye vertices over the full path of N vertices.
-__device__ float bv_mis(const double *pe, const double *pl, const bool *spec, int N, bool light_delta, int s, double inv_npix) {
-  double den = 0., ps = 0.;
-  for (int j = 0; j <= N; ++j) {
-    const bool a = j == 0 ? true : spec[j - 1];
-    const bool b = j == N ? light_delta : spec[j];
-    if ((a || b) && j != s) continue;
-    double p = j >= 2 ? inv_npix : 1.;
-    for (int k = 0; k < j; ++k) p *= pe[k];
-    for (int k = j; k < N; ++k) p *= pl[k];
-    if (j == s) ps = p;
-    if (!(a || b)) den += p * p;
-  }
-  return den > 0. ? (float)(ps * ps / den) : 0.f;
+// Wavelengths and random numbers of a camera sample (as init_camera_path).
+__device__ __forceinline__ BdptCtx bdpt_context(const DeviceScene &sc, Pcg &rng, uint32_t npix) {
+  const int main_idx = (int)rng.bounded(kStrata);
+  int idx[4] = {main_idx, main_idx + kStrata, main_idx + 2 * kStrata, main_idx + 3 * kStrata};
+  const int rot = (int)rng.bounded(4);
+  const int t = idx[0]; idx[0] = idx[rot]; idx[rot] = t;
+  const float lambda0 = 370.f + 10.f * idx[0] + 10.f * rng.uniform();
+  rng.uniform(); rng.uniform(); rng.uniform();
+  const uint32_t bins = (uint32_t)idx[0] | ((uint32_t)idx[1] << 8) | ((uint32_t)idx[2] << 16) | ((uint32_t)idx[3] << 24);
+  return BdptCtx{sc, bins, lambda0, sc.mis_mode == TTGPU_MIS_CONSISTENT, 1.f / (float)npix};
 }
 
-// Connection of eye vertex e with light vertex l of `light`; the contribution (MIS weighted) and
-// the splat pixel (camera connections) or -1.
-__device__ bool bv_connect(const BdptCtx &c, const BdptVertex *eye, int e, const BdptVertex *light, int l, bool light_delta,
-                           int *lds_stack, uint32_t &rays, float4 &contrib, int &pixel) {
-  const DeviceScene &sc = c.sc;
-  const BdptVertex &a = eye[e], &b = light[l];
-  float3 org, dir;
-  float len;
-  bv_segment(c, a, b, org, dir, len);
-  float4 fa;
-  float pa_fwd = 0.f, pa_rev = 0.f;
-  pixel = -1;
-  if (a.type == kBvCamera) {
-    const DevCamera &cam = sc.cam;
-    const float z = dot(dir, cam.dir);
-    if (!(z > 0.f)) return false;
-    const float x = dot(dir, cam.right) / z, y = dot(dir, cam.up) / z;
-    const float fx = (x - cam.xmin) / cam.xper, fy = (y - cam.ymin) / cam.yper;
-    const bool trunc = sc.mis_mode != TTGPU_MIS_CONSISTENT;
-    const float ix = trunc ? truncf(fx) : floorf(fx), iy = trunc ? truncf(fy) : floorf(fy);
-    if (!(ix >= 0.f && ix < (float)cam.width && iy >= 0.f && iy < (float)cam.height)) return false;
-    pixel = (int)iy * cam.width + (int)ix;
-    pa_fwd = camera_pdf(cam, x, y);
-    fa = f4(pa_fwd);
-  } else {
-    const DevShader &shd = sc.shaders[sc.materials[a.h.material].shader];
-    fa = bv_corr(a, dir, false) * eval_bsdf(shd, a.h, -a.wi, c.bins, 0.f, c.lambda0, dir, &pa_fwd);
-    pa_rev = bv_scatter_pdf(c, a, dir, -a.wi, false);
-  }
-  float4 fb;
-  float pb_fwd = 0.f, pb_rev = 0.f;
-  if (b.type == kBvSurf) {
-    const DevShader &shd = sc.shaders[sc.materials[b.h.material].shader];
-    fb = bv_corr(b, -dir, true) * eval_bsdf(shd, b.h, -b.wi, c.bins, 0.f, c.lambda0, -dir, &pb_fwd, true);
-    pb_rev = bv_scatter_pdf(c, b, -dir, -b.wi, true);
-  } else {
-    pb_fwd = bv_emission_pdf(c, b, -dir);
-    fb = b.type == kBvArea ? (dot(b.h.ng, -dir) > 0.f ? fabsf(dot(b.h.ng, dir)) : 0.f) * b.Le : b.Le;
-  }
-  const float4 f = fa * fb;
-  if (all_zero(f)) return false;
-  const float G = b.type == kBvEnv ? 1.f : 1.f / (len * len);
-  Ray r;
-  r.org = org;
-  r.dir = dir;
-  r.tmax = len * 0.9999f;
-  HitRec hr;
-  ++rays;
-  if (traverse<true>(sc.nodes, sc.prims_kz, sc.num_prims, r, lds_stack, hr)) return false;
-  const int N = e + 1 + l + 1;
-  double pe[2 * kBdptMaxVerts], pl[2 * kBdptMaxVerts];
-  bool spec[2 * kBdptMaxVerts];
-  for (int k = 0; k <= e; ++k) {
-    pe[k] = k == 0 ? 1. : (double)eye[k].pdf_walk;
-    pl[k] = eye[k].pdf_other;
-    spec[k] = k < e && eye[k].delta;
-  }
-  for (int j = 0; j <= l; ++j) {
-    const int k = N - 1 - j;
-    pl[k] = light[j].pdf_walk;
-    pe[k] = light[j].pdf_other;
-    spec[k] = j < l && light[j].delta;
-  }
-  pe[e + 1] = (double)pa_fwd * bv_conv(a, b, dir, len);
-  pl[e] = (double)pb_fwd * bv_conv(b, a, -dir, len);
-  if (e >= 1) {
-    float3 o2, d2;
-    float l2;
-    bv_segment(c, a, eye[e - 1], o2, d2, l2);
-    pl[e - 1] = (double)pa_rev * bv_conv(a, eye[e - 1], d2, l2);
-  }
-  if (l >= 1) {
-    float3 o2, d2;
-    float l2;
-    bv_segment(c, b, light[l - 1], o2, d2, l2);
-    pe[e + 2] = (double)pb_rev * bv_conv(b, light[l - 1], d2, l2);
-  }
-  const float w = bv_mis(pe, pl, spec, N, light_delta, e + 1, c.inv_npix);
-  contrib = (w * G) * (a.beta * b.beta * f);
-  return true;
-}
-
-__global__ void __launch_bounds__(kTraceBlock) k_bdpt(DeviceScene sc, uint64_t first, uint64_t count, uint32_t npix,
-                                                       uint32_t spp_base, uint64_t seed, double *fb, double *fb_sq, uint32_t *stats) {
+// Sample `first + s` of the pass for every s < count (at most w.capacity).
+__global__ void __launch_bounds__(kTraceBlock) k_bdpt_walk(DeviceScene sc, BdptWork w, uint64_t first, uint32_t count, uint32_t npix,
+                                                            uint32_t spp_base, uint64_t seed, uint32_t *stats) {
   __shared__ int lds_stack[kLdsStack * kTraceBlock];
-  uint32_t rays = 0;
-  for (uint64_t g = first + gtid(); g < first + count; g += grid_stride()) {
+  const uint32_t s = gtid();
+  uint32_t rays = 0, num = 0;
+  int ne = 0, nl = 0;
+  uint32_t directs = 0;  // bit e: eye vertex e has a light sample to connect to
+  if (s < count) {
+    const uint64_t g = first + s;
     const uint32_t pixel = (uint32_t)(g % npix);
-    const uint64_t sample = spp_base + g / npix;
     Pcg rng;
-    rng.seed(seed, sample * npix + pixel);
-    const int main_idx = (int)rng.bounded(kStrata);
-    int idx[4] = {main_idx, main_idx + kStrata, main_idx + 2 * kStrata, main_idx + 3 * kStrata};
-    const int rot = (int)rng.bounded(4);
-    const int t = idx[0]; idx[0] = idx[rot]; idx[rot] = t;
-    const float lambda0 = 370.f + 10.f * idx[0] + 10.f * rng.uniform();
-    rng.uniform(); rng.uniform(); rng.uniform();
-    const uint32_t bins = (uint32_t)idx[0] | ((uint32_t)idx[1] << 8) | ((uint32_t)idx[2] << 16) | ((uint32_t)idx[3] << 24);
-    const BdptCtx c{sc, bins, lambda0, sc.mis_mode == TTGPU_MIS_CONSISTENT, 1.f / (float)npix};
-    const int max_nodes = min(sc.max_depth + 1, kBdptMaxVerts);
+    rng.seed(seed, (spp_base + g / npix) * npix + pixel);
+    const BdptCtx c = bdpt_context(sc, rng, npix);
+    float4 acc = f4(0.f);
     // eye subpath
-    BdptVertex eye[kBdptMaxVerts];
-    int ne = 1;
-    eye[0].type = kBvCamera;
-    eye[0].h.pos = sc.cam.pos;
-    eye[0].beta = f4((float)kStrata);
-    eye[0].pdf_walk = 1.f;
-    eye[0].pdf_other = 0.f;
-    eye[0].delta = 0;
     {
+      BdptVertex v{};
+      v.type = kBvCamera;
+      v.h.pos = sc.cam.pos;
+      v.beta = f4((float)kStrata);
+      v.pdf_walk = 1.f;
+      v.prod = 1.;
+      bdpt_store(w, kBdptEye, 0, s, v);
       const int px = pixel % sc.cam.width, py = pixel / sc.cam.width;
       const float r0 = rng.uniform(), r1 = rng.uniform();
       float3 dir;
       float pdf_cam;
       camera_ray(sc.cam, px, py, r0, r1, dir, &pdf_cam);
-      if (max_nodes > 1) bv_walk(c, eye, ne, sc.cam.pos, dir, pdf_cam, false, f4(1.f), false, rng, lds_stack + threadIdx.x, rays);
+      ne = 1;
+      if (w.max_nodes > 1)
+        ne = bv_walk<false>(c, w, s, v, sc.cam.pos, dir, pdf_cam, f4(1.f), false, rng, lds_stack + threadIdx.x, rays, acc);
     }
     // light subpath
-    BdptVertex light[kBdptMaxVerts];
-    int nl = 0;
     bool light_delta = false;
-    if (bv_sample_light(c, rng, light[0], light_delta)) {
-      light[0].beta = f4(1.f / light[0].pdf_walk);
-      light[0].pdf_other = 0.f;
+    BdptVertex v{};
+    if (bv_sample_light(c, rng, v, light_delta)) {
+      v.beta = f4(1.f / v.pdf_walk);
+      v.prod = v.pdf_walk;
+      v.sum = 0.;
+      bdpt_store(w, kBdptLight, 0, s, v);
       nl = 1;
       const float r0 = rng.uniform(), r1 = rng.uniform();
       float3 org, dir;
       float pdf;
       float4 factor;
-      if (light[0].type == kBvArea) {
+      if (v.type == kBvArea) {
         const float3 l = to_uniform_hemisphere(r0, r1);
-        const Frame fr = make_frame(light[0].h.ng);
+        const Frame fr = make_frame(v.h.ng);
         dir = fr.to_world(l);
         pdf = 1.f / (2.f * kPi);
-        factor = (fabsf(dot(light[0].h.ng, dir)) * 2.f * kPi) * light[0].Le;
-        org = offset_origin(light[0].h, dir);
-      } else if (light[0].type == kBvPoint) {
+        factor = (fabsf(dot(v.h.ng, dir)) * 2.f * kPi) * v.Le;
+        org = offset_origin(v.h, dir);
+      } else if (v.type == kBvPoint) {
         dir = to_uniform_sphere(r0, r1);
         pdf = 1.f / (4.f * kPi);
-        factor = (4.f * kPi) * light[0].Le;
-        org = light[0].h.pos;
+        factor = (4.f * kPi) * v.Le;
+        org = v.h.pos;
       } else {
         // EnvLightPointSamplingBeyondScene (light.cxx:201-219): a disc across the scene's box.
-        dir = light[0].h.pos;
+        dir = v.h.pos;
         const float rr = sqrtf(r0), ph = 2.f * kPi * r1;
         float sn, cs;
         fast_sincos(ph, &sn, &cs);
         const Frame fr = make_frame(dir);
         org = sc.bb_center - dir * (10.f * sc.bb_diag) + fr.to_world(mk(rr * cs, rr * sn, 0.f)) * (0.5f * sc.bb_diag);
-        pdf = bv_emission_pdf(c, light[0], dir);
-        factor = (1.f / pdf) * light[0].Le;
+        pdf = bv_emission_pdf(c, v, dir);
+        factor = (1.f / pdf) * v.Le;
       }
-      if (max_nodes > 1) bv_walk(c, light, nl, org, dir, pdf, false, factor, true, rng, lds_stack + threadIdx.x, rays);
+      if (w.max_nodes > 1)
+        nl = bv_walk<true>(c, w, s, v, org, dir, pdf, factor, light_delta, rng, lds_stack + threadIdx.x, rays, acc);
     }
-    // strategies
-    float4 acc = f4(0.f);
-    for (int e = 0; e < ne; ++e) {
-      const BdptVertex &ev = eye[e];
-      if (e == 0 || ev.type == kBvSurf) {
-        if (e + 1 < max_nodes) {
-          BdptVertex direct[1];
-          bool dl_delta;
-          if (bv_sample_light(c, rng, direct[0], dl_delta)) {
-            direct[0].beta = f4(1.f / direct[0].pdf_walk);
-            direct[0].pdf_other = 0.f;
-            float4 contrib;
-            int pix;
-            if (bv_connect(c, eye, e, direct, 0, dl_delta, lds_stack + threadIdx.x, rays, contrib, pix)) {
-              if (e == 0) {
-                const float3 rgb = spectral_to_rgb(c.inv_npix * contrib, bins);
-                atomicAdd(fb + 3 * (size_t)pix + 0, (double)rgb.x);
-                atomicAdd(fb + 3 * (size_t)pix + 1, (double)rgb.y);
-                atomicAdd(fb + 3 * (size_t)pix + 2, (double)rgb.z);
-              } else {
-                acc = acc + contrib;
-              }
-            }
-          }
-        }
-        const int lmax = min(nl, max_nodes - e - 1);
-        for (int l = 1; l < lmax; ++l) {
-          float4 contrib;
-          int pix;
-          if (!bv_connect(c, eye, e, light, l, light_delta, lds_stack + threadIdx.x, rays, contrib, pix)) continue;
-          if (e == 0) {
-            const float3 rgb = spectral_to_rgb(c.inv_npix * contrib, bins);
-            atomicAdd(fb + 3 * (size_t)pix + 0, (double)rgb.x);
-            atomicAdd(fb + 3 * (size_t)pix + 1, (double)rgb.y);
-            atomicAdd(fb + 3 * (size_t)pix + 2, (double)rgb.z);
-          } else {
-            acc = acc + contrib;
-          }
-        }
+    // A fresh light sample per eye vertex, and the number of connections.
+    for (int e = 0; e < ne && e + 1 < w.max_nodes; ++e) {
+      BdptVertex d{};
+      bool dl_delta;
+      if (bv_sample_light(c, rng, d, dl_delta)) {
+        d.beta = f4(1.f / d.pdf_walk);
+        d.prod = d.pdf_walk;
+        d.sum = 0.;
+        d.delta = dl_delta ? 1 : 0;
+        bdpt_store(w, kBdptDirect, e, s, d);
+        directs |= 1u << e;
+        ++num;
       }
-      // HandleLightHit (:526-556)
-      if (e > 0) {
-        float4 Le = f4(0.f);
-        float p_start = 0.f, p_emit = 0.f;
-        bool is_light = false;
-        BdptVertex as_light = ev;
-        if (ev.type == kBvEnv) {
-          float pe;
-          env_eval(sc, ev.h.pos, bins, &pe);
-          Le = ev.Le;
-          p_start = pe * sc.type_probs[0];
-          p_emit = bv_emission_pdf(c, ev, ev.h.pos);
-          is_light = true;
-        } else if (ev.type == kBvSurf && sc.materials[ev.h.material].emitter >= 0) {
-          const DevEmitter &em = sc.emitters[sc.materials[ev.h.material].emitter];
-          const bool facing = dot(ev.h.ng, -ev.wi) > 0.f;
-          Le = (em.kind == TTGPU_AREA_UNIFORM && facing) ? take(em.radiance, bins) : f4(0.f);
-          p_start = sc.area_pick_prob / sc.prim_area[ev.h.prim];
-          as_light.type = kBvArea;
-          p_emit = facing ? 1.f / (2.f * kPi) : 0.f;
-          is_light = true;
-        }
-        if (is_light && !all_zero(Le)) {
-          const int N = e + 1;
-          double pe[kBdptMaxVerts], pl[kBdptMaxVerts];
-          bool spec[kBdptMaxVerts];
-          for (int k = 0; k <= e; ++k) {
-            pe[k] = k == 0 ? 1. : (double)eye[k].pdf_walk;
-            pl[k] = eye[k].pdf_other;
-            spec[k] = k < e && eye[k].delta;
-          }
-          pl[e] = p_start;
-          float3 o2, d2;
-          float l2;
-          bv_segment(c, as_light, eye[e - 1], o2, d2, l2);
-          pl[e - 1] = (double)p_emit * bv_conv(as_light, eye[e - 1], d2, l2);
-          const float w = bv_mis(pe, pl, spec, N, false, N, c.inv_npix);
-          acc = acc + w * (ev.beta * Le);
-        }
-      }
+      num += (uint32_t)max(0, min(nl, w.max_nodes - e - 1) - 1);
     }
-    const float3 rgb = spectral_to_rgb(acc, bins);
-    atomicAdd(fb + 3 * (size_t)pixel + 0, (double)rgb.x);
-    atomicAdd(fb + 3 * (size_t)pixel + 1, (double)rgb.y);
-    atomicAdd(fb + 3 * (size_t)pixel + 2, (double)rgb.z);
-    if (fb_sq) {
-      atomicAdd(fb_sq + 3 * (size_t)pixel + 0, (double)rgb.x * rgb.x);
-      atomicAdd(fb_sq + 3 * (size_t)pixel + 1, (double)rgb.y * rgb.y);
-      atomicAdd(fb_sq + 3 * (size_t)pixel + 2, (double)rgb.z * rgb.z);
+    w.info[s] = make_uint2(c.bins, (uint32_t)as_int(c.lambda0));
+    const float3 rgb = spectral_to_rgb(acc, c.bins);
+    w.acc[3 * (size_t)s + 0] = rgb.x;
+    w.acc[3 * (size_t)s + 1] = rgb.y;
+    w.acc[3 * (size_t)s + 2] = rgb.z;
+  }
+  // The wave's connections, listed with one atomic.
+  uint32_t at = num;
+  const int lane = (int)(threadIdx.x & 63);
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t x = __shfl_up(at, o);
+    at += lane >= o ? x : 0u;
+  }
+  uint32_t base = 0;
+  if (lane == 63 && at) base = atomicAdd(w.count, at);
+  at = __shfl(base, 63) + at - num;
+  if (s < count) {
+    for (int e = 0; e < ne && e + 1 < w.max_nodes; ++e) {
+      if ((directs >> e) & 1u) w.pairs[at++] = s | ((uint32_t)e << 20) | 0u;
+      const int lmax = min(nl, w.max_nodes - e - 1);
+      for (int l = 1; l < lmax; ++l) w.pairs[at++] = s | ((uint32_t)e << 20) | ((uint32_t)l << 25);
     }
   }
-  if (rays) atomicAdd(stats + kStatClosest, rays);
+  wave_stat(stats + kStatClosest, rays);
+}
+
+// Connection of an eye vertex with a light vertex (index l >= 1) or with its light sample (l = 0).
+__global__ void __launch_bounds__(kTraceBlock) k_bdpt_connect(DeviceScene sc, BdptWork w, uint32_t npix, double *fb, uint32_t *stats) {
+  __shared__ int lds_stack[kLdsStack * kTraceBlock];
+  const uint32_t count = *w.count;
+  const double inv = 1.f / (float)npix;
+  uint32_t rays = 0;
+  for (uint32_t k = gtid(); k < count; k += grid_stride()) {
+    const uint32_t id = w.pairs[k], s = id & 0xfffffu;
+    const int e = (int)((id >> 20) & 31u), l = (int)(id >> 25);
+    const uint2 info = w.info[s];
+    const BdptCtx c{sc, info.x, as_float((int)info.y), false, 1.f / (float)npix};
+    BdptVertex a, b;
+    bdpt_load(w, kBdptEye, e, s, a);
+    if (l == 0) bdpt_load(w, kBdptDirect, e, s, b);
+    else bdpt_load(w, kBdptLight, l, s, b);
+    float3 org, dir;
+    float len;
+    bv_segment(c, a, b, org, dir, len);
+    float4 fa;
+    float pa_fwd = 0.f, pa_rev = 0.f;
+    int pixel = -1;
+    if (a.type == kBvCamera) {
+      const DevCamera &cam = sc.cam;
+      const float z = dot(dir, cam.dir);
+      if (!(z > 0.f)) continue;
+      const float x = dot(dir, cam.right) / z, y = dot(dir, cam.up) / z;
+      const float fx = (x - cam.xmin) / cam.xper, fy = (y - cam.ymin) / cam.yper;
+      const bool trunc = sc.mis_mode != TTGPU_MIS_CONSISTENT;
+      const float ix = trunc ? truncf(fx) : floorf(fx), iy = trunc ? truncf(fy) : floorf(fy);
+      if (!(ix >= 0.f && ix < (float)cam.width && iy >= 0.f && iy < (float)cam.height)) continue;
+      pixel = (int)iy * cam.width + (int)ix;
+      pa_fwd = camera_pdf(cam, x, y);
+      fa = f4(pa_fwd);
+    } else {
+      const DevShader &shd = sc.shaders[sc.materials[a.h.material].shader];
+      fa = bv_corr(a, dir, false) * eval_bsdf(shd, a.h, -a.wi, c.bins, 0.f, c.lambda0, dir, &pa_fwd);
+    }
+    float4 fl;
+    float pb_fwd = 0.f, pb_rev = 0.f;
+    if (b.type == kBvSurf) {
+      const DevShader &shd = sc.shaders[sc.materials[b.h.material].shader];
+      fl = bv_corr(b, -dir, true) * eval_bsdf(shd, b.h, -b.wi, c.bins, 0.f, c.lambda0, -dir, &pb_fwd, true);
+    } else {
+      pb_fwd = bv_emission_pdf(c, b, -dir);
+      fl = b.type == kBvArea ? (dot(b.h.ng, -dir) > 0.f ? fabsf(dot(b.h.ng, dir)) : 0.f) * b.Le : b.Le;
+    }
+    const float4 f = fa * fl;
+    if (all_zero(f)) continue;
+    const float G = b.type == kBvEnv ? 1.f : 1.f / (len * len);
+    Ray r;
+    r.org = org;
+    r.dir = dir;
+    r.tmax = len * 0.9999f;
+    HitRec hr;
+    ++rays;
+    if (traverse<true>(sc.nodes, sc.prims_kz, sc.num_prims, r, lds_stack + threadIdx.x, hr)) continue;
+    // Strategies of the full path by their number of eye vertices j: up to e - 1 (a.sum), e, this one
+    // (e + 1), e + 2, and more (b.sum).
+    const double pe_b = (double)pa_fwd * bv_conv(a, b, dir, len), pl_a = (double)pb_fwd * bv_conv(b, a, -dir, len);
+    const double mine = sq((e >= 1 ? inv : 1.) * a.prod * b.prod);
+    double den = mine;
+    if (e >= 1) {
+      BdptVertex p;
+      const float4 *row = bdpt_row(w, kBdptEye, e - 1, s);
+      bdpt_unpack_geometry(row, p);
+      const float4 m = row[5];
+      if (e >= 2) {
+        // a.sum is zero for e < 2: no strategy connects before the first scatter vertex.
+        pa_rev = bv_scatter_pdf(c, a, dir, -a.wi, false);
+        float3 o2, d2;
+        float l2;
+        bv_segment(c, a, p, o2, d2, l2);
+        den += a.sum * sq((double)pa_rev * bv_conv(a, p, d2, l2) * pl_a * b.prod);
+      }
+      if (!p.delta) den += sq((e >= 2 ? inv : 1.) * unpack_double(m.x, m.y) * pl_a * b.prod);
+    }
+    if (l >= 1) {
+      BdptVertex p;
+      const float4 *row = bdpt_row(w, kBdptLight, l - 1, s);
+      bdpt_unpack_geometry(row, p);
+      const float4 m = row[5];
+      if (!p.delta) den += sq(inv * a.prod * pe_b * unpack_double(m.x, m.y));
+      if (b.sum > 0.) {
+        pb_rev = bv_scatter_pdf(c, b, -dir, -b.wi, true);
+        float3 o2, d2;
+        float l2;
+        bv_segment(c, b, p, o2, d2, l2);
+        den += b.sum * sq(inv * a.prod * pe_b * (double)pb_rev * bv_conv(b, p, d2, l2));
+      }
+    } else if (!b.delta) {
+      den += sq(inv * a.prod * pe_b);
+    }
+    const float wgt = den > 0. ? (float)(mine / den) : 0.f;
+    const float4 contrib = (wgt * G) * (a.beta * b.beta * f);
+    if (e == 0) {
+      const float3 rgb = spectral_to_rgb(c.inv_npix * contrib, c.bins);
+      atomicAdd(fb + 3 * (size_t)pixel + 0, (double)rgb.x);
+      atomicAdd(fb + 3 * (size_t)pixel + 1, (double)rgb.y);
+      atomicAdd(fb + 3 * (size_t)pixel + 2, (double)rgb.z);
+    } else {
+      const float3 rgb = spectral_to_rgb(contrib, c.bins);
+      atomicAdd(w.acc + 3 * (size_t)s + 0, (double)rgb.x);
+      atomicAdd(w.acc + 3 * (size_t)s + 1, (double)rgb.y);
+      atomicAdd(w.acc + 3 * (size_t)s + 2, (double)rgb.z);
+    }
+  }
+  wave_stat(stats + kStatClosest, rays);
+}
+
+__global__ void __launch_bounds__(256) k_bdpt_finish(BdptWork w, uint64_t first, uint32_t count, uint32_t npix, double *fb, double *fb_sq) {
+  const uint32_t s = gtid();
+  if (s == 0) *w.count = 0;
+  if (s >= count) return;
+  const uint32_t pixel = (uint32_t)((first + s) % npix);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const double v = (double)(float)w.acc[3 * (size_t)s + k];
+    atomicAdd(fb + 3 * (size_t)pixel + k, v);
+    if (fb_sq) atomicAdd(fb_sq + 3 * (size_t)pixel + k, v * v);
+  }
 }
 
 // ---- host-side launchers ------------------------------------------------------------------
@@ -2578,11 +2677,14 @@ void LaunchShade(const DeviceScene &sc, const PathQueues &q, const uint32_t *que
     hipLaunchKernelGGL(k_shade<false>, dim3(Blocks(max_count, 256, 8192)), dim3(256), 0, st, sc, q, queue_in, count_in, queue_out, count_out,
                        fb, fb_sq);
 }
-void LaunchBdpt(const DeviceScene &sc, uint64_t first, uint64_t count, uint32_t npix, uint32_t spp_base, uint64_t seed, double *fb,
-                double *fb_sq, uint32_t *stats, hipStream_t st) {
+size_t BdptVertexBytes(int max_nodes) { return (size_t)3 * max_nodes * kBdptRows * sizeof(float4); }
+void LaunchBdpt(const DeviceScene &sc, const BdptWork &w, uint64_t first, uint32_t count, uint32_t npix, uint32_t spp_base, uint64_t seed,
+                double *fb, double *fb_sq, uint32_t *stats, hipStream_t st) {
   if (count == 0) return;
-  hipLaunchKernelGGL(k_bdpt, dim3(Blocks(count, kTraceBlock, 16384)), dim3(kTraceBlock), 0, st, sc, first, count, npix, spp_base,
-                     seed, fb, fb_sq, stats);
+  hipLaunchKernelGGL(k_bdpt_walk, dim3((count + kTraceBlock - 1) / kTraceBlock), dim3(kTraceBlock), 0, st, sc, w, first, count, npix, spp_base,
+                     seed, stats);
+  hipLaunchKernelGGL(k_bdpt_connect, dim3(Blocks((uint64_t)count * 8, kTraceBlock, 16384)), dim3(kTraceBlock), 0, st, sc, w, npix, fb, stats);
+  hipLaunchKernelGGL(k_bdpt_finish, dim3((count + 255) / 256), dim3(256), 0, st, w, first, count, npix, fb, fb_sq);
 }
 void LaunchCameraConnect(const DeviceScene &sc, uint64_t first, uint64_t count, uint32_t npix, uint32_t spp_base, uint64_t seed,
                          double *fb, double *fb_sq, uint32_t *stats, hipStream_t st) {

@@ -40,8 +40,23 @@ void LaunchTrackMedia(const DeviceScene &sc, const PathQueues &q, const uint32_t
 void LaunchShade(const DeviceScene &sc, const PathQueues &q, const uint32_t *queue_in, const uint32_t *count_in, uint32_t *queue_out,
                  uint32_t *count_out, uint32_t max_count, double *fb, double *fb_sq, hipStream_t st);
 constexpr int kBdptMaxVertices = 17;  // BDPT subpath vertices per thread: max_ray_depth <= 16
-void LaunchBdpt(const DeviceScene &sc, uint64_t first, uint64_t count, uint32_t npix, uint32_t spp_base, uint64_t seed, double *fb,
-                double *fb_sq, uint32_t *stats, hipStream_t st);
+// Workspace of a chunk of at most `capacity` (<= 2^20) BDPT samples.
+struct BdptWork {
+  float4 *verts;     // eye, light and light-sample vertices: capacity x BdptVertexBytes(max_nodes)
+  uint32_t *pairs;   // connections: sample | eye vertex << 20 | light vertex << 25 (0: light sample)
+  uint32_t *count;   // number of connections; zero between chunks
+  uint2 *info;       // per sample: wavelength bins, lambda of the hero wavelength
+  double *acc;       // per sample: rgb
+  int max_nodes;     // vertices per subpath
+  uint32_t capacity;
+};
+size_t BdptVertexBytes(int max_nodes);
+// Connections of a sample at most: eye vertex e < max_nodes - 1 with its light sample and the light
+// vertices 1 .. max_nodes - e - 2.
+constexpr size_t BdptMaxPairs(int max_nodes) { return max_nodes > 1 ? (size_t)max_nodes * (max_nodes - 1) / 2 : 1; }
+// Samples [first, first + count) of the pass, count <= capacity.
+void LaunchBdpt(const DeviceScene &sc, const BdptWork &w, uint64_t first, uint32_t count, uint32_t npix, uint32_t spp_base, uint64_t seed,
+                double *fb, double *fb_sq, uint32_t *stats, hipStream_t st);
 void LaunchCameraConnect(const DeviceScene &sc, uint64_t first, uint64_t count, uint32_t npix, uint32_t spp_base, uint64_t seed,
                          double *fb, double *fb_sq, uint32_t *stats, hipStream_t st);
 void LaunchShadow(const DeviceScene &sc, const PathQueues &q, uint32_t max_count, double *fb, double *fb_sq, hipStream_t st);

@@ -89,6 +89,7 @@ struct ttgpu_handle {
   std::vector<void *> allocs;
   double *fb = nullptr, *fb_sq = nullptr;
   void *select_temp = nullptr;  // storage of the slot-ordered queue selection
+  BdptWork bdpt{};              // bdpt only
   InferSort infer_sort{};       // learned guide: sort of the inference queue by hit point
   bool infer_sorted = false;
   std::vector<uint64_t> pixel_spp;
@@ -776,7 +777,10 @@ void BuildTables(ttgpu_handle *h, const ttgpu_scene &s, double bb_diag) {
 }
 
 void AllocateQueues(ttgpu_handle *h) {
-  const uint32_t N = h->capacity;
+  // bdpt keeps its own workspace instead of the wavefront's path state: of path queues it only
+  // uses the counters.
+  const bool bdpt = h->params.algo == TTGPU_ALGO_BDPT;
+  const uint32_t N = bdpt ? 1u : h->capacity;
   PathQueues &q = h->q;
   q.capacity = (int)N;
   q.org = h->Alloc<float4>(N); q.dir = h->Alloc<float4>(N); q.hit = h->Alloc<float4>(N);
@@ -831,6 +835,19 @@ void AllocateQueues(ttgpu_handle *h) {
     q.rec_pos_w = h->Alloc<float4>(q.rec_capacity);
     q.rec_dir = h->Alloc<float4>(q.rec_capacity);
     h->stats.state_bytes += (size_t)N * (48 * nvtx + 16) + (size_t)q.rec_capacity * 32;
+  }
+  if (bdpt) {
+    // 2^18 samples in flight: four waves per SIMD in the walks, 0.7 GB at depth 8, 1.3 GB at 16.
+    BdptWork &w = h->bdpt;
+    w.max_nodes = h->params.max_ray_depth + 1;
+    w.capacity = 1u << 18;
+    w.verts = (float4 *)h->Alloc<uint8_t>(w.capacity * BdptVertexBytes(w.max_nodes));
+    w.pairs = h->Alloc<uint32_t>(w.capacity * BdptMaxPairs(w.max_nodes));
+    w.info = h->Alloc<uint2>(w.capacity);
+    w.acc = h->Alloc<double>(3 * (size_t)w.capacity);
+    w.count = h->Alloc<uint32_t>(1);
+    Check(hipMemset(w.count, 0, sizeof(uint32_t)), "hipMemset bdpt count");
+    h->stats.state_bytes += w.capacity * (BdptVertexBytes(w.max_nodes) + 4 * BdptMaxPairs(w.max_nodes) + 32);
   }
   q.vt = nullptr;
   q.wtn_r = q.wtn_c = nullptr;
@@ -1308,19 +1325,20 @@ void ResetFramebuffer(ttgpu_handle *h) {
 // the slots of finished paths take the next camera paths, so launches stay full until the pass's
 // last paths drain.  The host runs one iteration ahead of a 16-byte progress read-back.  A stop
 // request ends the issuing of new paths; the paths in flight finish.  Returns false after a stop.
-// bdpt: one thread per camera sample (eye and light subpaths and all their connections), in
-// launches of at most 2^20 samples so that a stop request ends the pass after the launch in flight.
+// bdpt: chunks of as many samples as the workspace holds; a stop request ends the pass after the
+// chunk in flight.
 bool RenderPassBdpt(ttgpu_handle *h, int spp) {
   const uint64_t npix = (uint64_t)h->npix;
   const uint64_t total = npix * (uint64_t)spp;
   const uint32_t spp_base = (uint32_t)h->total_spp;
   hipEvent_t ev0 = h->NextEvent(), ev1 = h->NextEvent();
   Check(hipEventRecord(ev0, h->stream), "hipEventRecord");
-  constexpr uint64_t kChunk = 1ull << 20;
   uint64_t issued = 0;
   while (issued < total && !h->stop.load()) {
-    const uint64_t n = std::min(kChunk, total - issued);
-    h->Timed("bdpt", [&] { LaunchBdpt(h->dsc, issued, n, (uint32_t)npix, spp_base, h->params.seed, h->fb, h->fb_sq, h->q.counters, h->stream); });
+    const uint64_t n = std::min<uint64_t>(h->bdpt.capacity, total - issued);
+    h->Timed("bdpt", [&] {
+      LaunchBdpt(h->dsc, h->bdpt, issued, (uint32_t)n, (uint32_t)npix, spp_base, h->params.seed, h->fb, h->fb_sq, h->q.counters, h->stream);
+    });
     Check(hipGetLastError(), "kernel launch");
     Check(hipStreamSynchronize(h->stream), "hipStreamSynchronize");
     issued += n;

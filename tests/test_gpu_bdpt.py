@@ -106,3 +106,24 @@ def test_gpu_bdpt_rejects_unsupported(gpu_lib):
     s.set_camera([0.0, 1.0, 3.4], [0.0, 1.0, 0.0], [0.0, 1.0, 0.0], 40.0, kind=abi.CAMERA_FISHEYE)
     with pytest.raises(TTGpuError, match="pinhole"):
         GpuRenderer(s, _params(8, 8, 8))
+
+
+@pytest.mark.parametrize("w,h,spp,depth", [(1, 1, 3, 2), (13, 7, 5, 16), (257, 511, 3, 3)])
+def test_gpu_bdpt_chunks_and_wave_edges(gpu_lib, w, h, spp, depth):
+    """One pass (the last size spans two chunks of 2^18 samples and ends inside a wave) equals the sum
+    of 1-spp passes: each sample draws the same numbers wherever it lies in a chunk.  A sample's sum
+    runs over at most 136 connections in another order, in FP64, and is rounded to FP32 once."""
+    scene = configs.cornell_box(w, h)
+
+    def render(passes):
+        with GpuRenderer(scene, _params(w, h, depth)) as r:
+            for n in passes:
+                r.render_spp(n)
+            rgb, _, n = r.framebuffer()
+            return rgb, n, r.stats()["paths_traced"]
+    a, na, pa = render([spp])
+    b, nb, pb = render([1] * spp)
+    assert np.all(na == spp) and np.array_equal(na, nb) and pa == pb == w * h * spp
+    if w > 100:
+        assert a.sum() > 0
+    np.testing.assert_allclose(a, b, rtol=spp * 2.0 ** -23, atol=1e-12)
