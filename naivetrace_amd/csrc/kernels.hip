@@ -50,6 +50,13 @@ __device__ __forceinline__ uint32_t wave_append(uint32_t *counter, bool pred) {
   return base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
 }
 
+// Adds every lane's count with one atomic per wave (called by whole waves).
+__device__ __forceinline__ void wave_stat(uint32_t *counter, uint32_t n) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+  if ((threadIdx.x & 63) == 0 && n) atomicAdd(counter, n);
+}
+
 __device__ __forceinline__ uint32_t grid_stride() { return gridDim.x * blockDim.x; }
 __device__ __forceinline__ uint32_t gtid() { return blockIdx.x * blockDim.x + threadIdx.x; }
 
@@ -980,16 +987,42 @@ __global__ void __launch_bounds__(kTraceBlock, TTGPU_TRACE_WAVES) k_shadow(Devic
 // segment is unoccluded, MIS weight x camera importance (= direction pdf) x light value x
 // wavelength weights / pixel count added to that pixel.  With TTGPU_MIS_REFERENCE the pixel index
 // truncates toward zero as the reference does.
-__global__ void __launch_bounds__(kTraceBlock) k_camera_connect(DeviceScene sc, uint64_t first, uint64_t count, uint32_t npix,
-                                                                 uint32_t spp_base, uint64_t seed, double *fb, double *fb_sq,
-                                                                 uint32_t *stats) {
-  __shared__ int lds_stack[kLdsStack * kTraceBlock];
+//
+// The light's image is a few hundred pixels that every sample hits, so six FP64 atomics per sample
+// on them bound the kernel: 1.88 ms for 4.2 M samples of the 512 x 512 Cornell box (780 pixels), 0.23
+// without them.  Each block sums its samples in an LDS table of kConnectSlots pixels and adds each
+// slot once at its end: 0.32 ms.  A pixel that finds no slot in kConnectProbes goes to memory as
+// before; those are what a small table pays for (512 slots and two probes: 0.82 ms).  LDS holds the
+// table and the traversal stacks, which leaves one block per CU; 1024 threads with 1024 slots took
+// 0.29 ms but cover half the pixels.
+constexpr int kConnectBlock = 512, kConnectBits = 11, kConnectSlots = 1 << kConnectBits, kConnectProbes = 16, kConnectBlocks = 256;
+
+__global__ void __launch_bounds__(kConnectBlock) k_camera_connect(DeviceScene sc, uint64_t first, uint64_t count, uint32_t npix,
+                                                                   uint32_t spp_base, uint64_t seed, double *fb, double *fb_sq,
+                                                                   uint32_t *stats) {
+  static_assert(kConnectBlock % kTraceBlock == 0, "stack columns are laid out per kTraceBlock threads");
+  __shared__ int lds_stack[kLdsStack * kConnectBlock];
+  __shared__ uint32_t s_pixel[kConnectSlots];  // pixel + 1, 0: free
+  __shared__ double s_sum[6][kConnectSlots];
+  int *stack = lds_stack + (threadIdx.x / kTraceBlock) * (kLdsStack * kTraceBlock) + threadIdx.x % kTraceBlock;
+  for (int k = threadIdx.x; k < kConnectSlots; k += kConnectBlock) {
+    s_pixel[k] = 0;
+#pragma unroll
+    for (int j = 0; j < 6; ++j) s_sum[j][k] = 0.;
+  }
+  __syncthreads();
   const bool mis = sc.sample_mode == TTGPU_SAMPLE_BOTH;
   const DevCamera &c = sc.cam;
   uint32_t rays = 0;
-  for (uint64_t g = first + gtid(); g < first + count; g += grid_stride()) {
-    const uint32_t pixel = (uint32_t)(g % npix);
-    const uint64_t sample = spp_base + g / npix;
+  // Pixel and sample of g, advanced by the grid's stride without a division per sample.
+  const uint32_t step_pixel = grid_stride() % npix, step_sample = grid_stride() / npix;
+  uint32_t pixel = (uint32_t)((first + gtid()) % npix);
+  uint64_t sample = spp_base + (first + gtid()) / npix;
+  for (uint64_t g = gtid(); g < count; g += grid_stride(), pixel += step_pixel, sample += step_sample) {
+    if (pixel >= npix) {
+      pixel -= npix;
+      ++sample;
+    }
     Pcg rng;
     rng.seed(seed ^ 0xC2B2AE3D27D4EB4Full, sample * npix + pixel);
     const int main_idx = (int)rng.bounded(kStrata);
@@ -1016,18 +1049,38 @@ __global__ void __launch_bounds__(kTraceBlock) k_camera_connect(DeviceScene sc, 
     r.tmax = ls.len * 0.9999f;
     HitRec hr;
     ++rays;
-    if (traverse<true>(sc.nodes, sc.prims_kz, sc.num_prims, r, lds_stack + threadIdx.x, hr)) continue;
-    const size_t p = (size_t)iy * c.width + (size_t)ix;
-    atomicAdd(fb + 3 * p + 0, (double)crgb.x);
-    atomicAdd(fb + 3 * p + 1, (double)crgb.y);
-    atomicAdd(fb + 3 * p + 2, (double)crgb.z);
-    if (fb_sq) {
-      atomicAdd(fb_sq + 3 * p + 0, (double)crgb.x * crgb.x);
-      atomicAdd(fb_sq + 3 * p + 1, (double)crgb.y * crgb.y);
-      atomicAdd(fb_sq + 3 * p + 2, (double)crgb.z * crgb.z);
+    if (traverse<true>(sc.nodes, sc.prims_kz, sc.num_prims, r, stack, hr)) continue;
+    const uint32_t p = (uint32_t)((size_t)iy * c.width + (size_t)ix);
+    const double v[6] = {(double)crgb.x, (double)crgb.y, (double)crgb.z, (double)crgb.x * crgb.x, (double)crgb.y * crgb.y,
+                         (double)crgb.z * crgb.z};
+    uint32_t slot = (p * 2654435761u) >> (32 - kConnectBits), owner = 0u;
+    for (int probe = 0; probe < kConnectProbes; ++probe) {
+      owner = atomicCAS(&s_pixel[slot], 0u, p + 1u);
+      if (owner == 0u || owner == p + 1u) break;
+      slot = (slot + 1u) & (kConnectSlots - 1);
+    }
+    if (owner == 0u || owner == p + 1u) {
+#pragma unroll
+      for (int j = 0; j < 6; ++j) atomicAdd(&s_sum[j][slot], v[j]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        atomicAdd(fb + 3 * (size_t)p + j, v[j]);
+        if (fb_sq) atomicAdd(fb_sq + 3 * (size_t)p + j, v[3 + j]);
+      }
     }
   }
-  if (rays) atomicAdd(stats + kStatShadow, rays);
+  __syncthreads();
+  for (int k = threadIdx.x; k < kConnectSlots; k += kConnectBlock) {
+    if (s_pixel[k] == 0) continue;
+    const size_t p = s_pixel[k] - 1u;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      atomicAdd(fb + 3 * p + j, s_sum[j][k]);
+      if (fb_sq) atomicAdd(fb_sq + 3 * p + j, s_sum[3 + j][k]);
+    }
+  }
+  wave_stat(stats + kStatShadow, rays);
 }
 
 // ---- media: shade with null-path tracking (pt2.cxx:410-443 with media_integrator.cxx) ------
@@ -2026,7 +2079,8 @@ __global__ void k_guide_pdf_at(DeviceScene sc, int64_t n, const float *pos, cons
 // before it and the summed squares of the strategies that connect earlier on its subpath, so a
 // connection's MIS weight takes a dozen FP64 operations instead of a product per strategy.  As one
 // kernel with private arrays (5.9 KB of scratch per lane, 232 registers, 23 % of the lanes active, 72
-// % of the wave cycles waiting) 262,144 samples of the Cornell box took 4.75 ms.
+// % of the wave cycles waiting) 262,144 samples of the Cornell box took 4.75 ms; these
+// take 0.51 + 0.79 + 0.03 ms.
 enum { kBvCamera = 0, kBvSurf = 1, kBvArea = 2, kBvEnv = 3, kBvPoint = 4 };
 
 struct BdptVertex {
@@ -2224,13 +2278,6 @@ __device__ __forceinline__ float bv_scatter_pdf(const BdptCtx &c, const BdptVert
 }
 
 __device__ __forceinline__ double sq(double x) { return x * x; }
-
-// Adds every lane's count with one atomic per wave (called by whole waves).
-__device__ __forceinline__ void wave_stat(uint32_t *counter, uint32_t n) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
-  if ((threadIdx.x & 63) == 0 && n) atomicAdd(counter, n);
-}
 
 // BdptForwardTrace (:598-646) from `cur`, the subpath's first vertex (index 0, already stored), with
 // the sampled direction `dir`; stores the vertices and returns their number.  Eye subpaths add their
@@ -2689,8 +2736,8 @@ void LaunchBdpt(const DeviceScene &sc, const BdptWork &w, uint64_t first, uint32
 void LaunchCameraConnect(const DeviceScene &sc, uint64_t first, uint64_t count, uint32_t npix, uint32_t spp_base, uint64_t seed,
                          double *fb, double *fb_sq, uint32_t *stats, hipStream_t st) {
   if (count == 0) return;
-  hipLaunchKernelGGL(k_camera_connect, dim3(Blocks(count, kTraceBlock, 16384)), dim3(kTraceBlock), 0, st, sc, first, count, npix,
-                     spp_base, seed, fb, fb_sq, stats);
+  hipLaunchKernelGGL(k_camera_connect, dim3(Blocks(count, kConnectBlock, kConnectBlocks)), dim3(kConnectBlock), 0, st, sc, first, count,
+                     npix, spp_base, seed, fb, fb_sq, stats);
 }
 bool ShadowInTrace(const DeviceScene &sc, const PathQueues &q) { return sc.shadow_in_trace && !q.vt && !sc.has_media; }
 void LaunchShadow(const DeviceScene &sc, const PathQueues &q, uint32_t max_count, double *fb, double *fb_sq, hipStream_t st) {

@@ -97,3 +97,23 @@ def test_gpu_pt_reference_pixel_truncation_quirk(gpu_lib):
 def test_gpu_pt_rejects_media(gpu_lib):
     with pytest.raises(TTGpuError, match="surface scenes"):
         GpuRenderer(fog_furnace_scene(0.5), _params(4, 4, 8, abi.SAMPLE_BOTH, abi.MIS_CONSISTENT))
+
+
+@pytest.mark.parametrize("w,h,spp", [(7, 5, 2), (45, 45, 3), (46, 45, 3), (96, 64, 4)])
+def test_camera_connections_through_the_pixel_table(gpu_lib, w, h, spp):
+    """Light points connected to the camera, with an emitter that fills the view: fewer pixels than the
+    block's table of 2048 slots, about as many, and more (the rest goes to memory).  One pass equals
+    the sum of 1-spp passes up to the order of the FP64 sums (at most 64 terms land on a pixel here
+    many times over: 1e-12), and the squared sums do too."""
+    def render(passes):
+        p = abi.default_params(w, h, max_depth=3, seed=9, algo=abi.ALGO_PT)
+        p.sample_mode = abi.SAMPLE_LIGHTS
+        with GpuRenderer(emitter_wall_scene(2.0), p) as r:
+            for n in passes:
+                r.render_spp(n)
+            return r.framebuffer()
+    a, a2, n = render([spp])
+    b, b2, _ = render([1] * spp)
+    assert np.all(n == spp) and a.sum() > 0
+    np.testing.assert_allclose(a, b, rtol=1e-12, atol=1e-15)
+    np.testing.assert_allclose(a2, b2, rtol=1e-12, atol=1e-15)
