@@ -203,6 +203,7 @@ struct DeviceScene {
   float3 bb_center;                // centre of the scene's bounding box
   int empty_space_medium;          // kVacuum or medium id
   int has_media;
+  int has_atmosphere;              // 1: some medium is an atmosphere (its coefficients vary along a ray)
   uint64_t cam_tracker;            // packed medium tracker at the camera
   DevCamera cam;
   int sample_mode, mis_mode, max_depth;

@@ -171,9 +171,12 @@ TT_HD void atmo_coeffs(const DevMedium &m, double alt, uint32_t bins, float4 &ss
   ss_mie = take(m.mie_sigma_s, bins) * rm;
   sa = take(m.mie_sigma_a, bins) * rm;
 }
+// kAtmo = false: code for scenes whose media are all homogeneous (DeviceScene::has_atmosphere == 0).  The
+// atmosphere's paths cost the shading kernel registers that no such scene uses.
+template <bool kAtmo = true>
 TT_HD void medium_coeffs(const DeviceScene &sc, int mid, D3 pos, uint32_t bins, float4 &ss, float4 &st) {
   const DevMedium &m = sc.media[mid];
-  if (is_atmosphere(m)) {
+  if (kAtmo && is_atmosphere(m)) {
     float4 a, b, c;
     atmo_coeffs(m, atmo_altitude(m, pos), bins, a, b, c);
     ss = a + b;
@@ -183,11 +186,63 @@ TT_HD void medium_coeffs(const DeviceScene &sc, int mid, D3 pos, uint32_t bins, 
   ss = take(m.sigma_s, bins);
   st = take(m.sigma_t, bins);
 }
+// What the transmission loop reads of its medium, loaded once per segment: its iterations depend on
+// each other, and with the look-ups inside (a dozen gathers of the path's bins, the planet's
+// geometry) each of the atmosphere's null collisions waited for memory.  Shadow rays of the
+// 1024 x 512 atmosphere: 1.60 -> 1.42 ms per 8-spp pass.  (The shading kernel, at 248 registers, has no
+// room for it: its tracking loop spilled and the launch took 4.36 ms instead of 3.07.)  Same operations
+// as medium_coeffs; the tabulated atmosphere, whose rows depend on the altitude, still goes through it.
+struct MediumAt {
+  int kind;
+  float4 a, b, c;  // homogeneous: scattering, extinction; atmosphere: Rayleigh, Mie scattering, Mie absorption
+  double cx, cy, cz, radius, inv_h_ray, inv_h_mie, lower_cutoff;
+};
+template <bool kAtmo>
+TT_HD MediumAt load_medium(const DeviceScene &sc, int mid, uint32_t bins) {
+  const DevMedium &m = sc.media[mid];
+  MediumAt v;
+  v.kind = m.kind;
+  v.c = f4(0.f);
+  v.cx = v.cy = v.cz = v.radius = v.inv_h_ray = v.inv_h_mie = v.lower_cutoff = 0.;
+  if (kAtmo && m.kind == TTGPU_MEDIUM_ATMOSPHERE) {
+    v.a = take(m.rayleigh_sigma_s, bins);
+    v.b = take(m.mie_sigma_s, bins);
+    v.c = take(m.mie_sigma_a, bins);
+    v.cx = m.planet_center[0];
+    v.cy = m.planet_center[1];
+    v.cz = m.planet_center[2];
+    v.radius = m.planet_radius;
+    v.inv_h_ray = m.rayleigh_inv_h;
+    v.inv_h_mie = m.mie_inv_h;
+    v.lower_cutoff = m.lower_cutoff;
+  } else {
+    v.a = take(m.sigma_s, bins);
+    v.b = take(m.sigma_t, bins);
+  }
+  return v;
+}
+template <bool kAtmo>
+TT_HD void medium_coeffs(const DeviceScene &sc, int mid, const MediumAt &v, D3 pos, uint32_t bins, float4 &ss, float4 &st) {
+  if (kAtmo && v.kind == TTGPU_MEDIUM_ATMOSPHERE) {
+    const double x = pos.x - v.cx, y = pos.y - v.cy, z = pos.z - v.cz;
+    double alt = sqrt(x * x + y * y + z * z) - v.radius;
+    alt = alt > v.lower_cutoff ? alt : v.lower_cutoff;
+    const float rr = expf((float)(-alt * v.inv_h_ray)), rm = expf((float)(-alt * v.inv_h_mie));
+    ss = v.a * rr + v.b * rm;
+    st = ss + v.c * rm;
+  } else if (kAtmo && v.kind == TTGPU_MEDIUM_ATMOSPHERE_TABULATED) {
+    medium_coeffs(sc, mid, pos, bins, ss, st);
+  } else {
+    ss = v.a;
+    st = v.b;
+  }
+}
 // Majorant over a segment; the atmosphere's is taken at the segment's lowest point
 // (SphereGeometry::ComputeLowestPointAlong, atmosphere.hxx:95-123).
+template <bool kAtmo = true>
 TT_HD float4 medium_majorant(const DeviceScene &sc, int mid, D3 org, float3 dir, double len, uint32_t bins) {
   const DevMedium &m = sc.media[mid];
-  if (is_atmosphere(m)) {
+  if (kAtmo && is_atmosphere(m)) {
     const double ox = org.x - m.planet_center[0], oy = org.y - m.planet_center[1], oz = org.z - m.planet_center[2];
     double tl = -(ox * dir.x + oy * dir.y + oz * dir.z);
     tl = tl > len ? len : (tl < 0. ? 0. : tl);
@@ -263,11 +318,12 @@ TT_HD PhaseMix atmo_phase(const DevMedium &m, D3 pos, uint32_t bins) {
   atmo_coeffs(m, atmo_altitude(m, pos), bins, ss_ray, ss_mie, sa);
   return phase_mix(TTGPU_PHASE_RAYLEIGH, 0.f, ss_ray, TTGPU_PHASE_HENYEY_GREENSTEIN, m.mie_g, ss_mie);
 }
+template <bool kAtmo = true>
 TT_HD Scatter medium_phase_sample(const DeviceScene &sc, int mid, float3 wi, D3 pos, uint32_t bins, Pcg &rng) {
   const DevMedium &m = sc.media[mid];
   Scatter s;
   s.delta = false;
-  if (is_atmosphere(m)) {
+  if (kAtmo && is_atmosphere(m)) {
     phase_mix_sample(atmo_phase(m, pos, bins), wi, rng, s.dir, s.value, s.pdf);
     return s;
   }
@@ -277,9 +333,10 @@ TT_HD Scatter medium_phase_sample(const DeviceScene &sc, int mid, float3 wi, D3 
   s.pdf = val;
   return s;
 }
+template <bool kAtmo = true>
 TT_HD float4 medium_phase_eval(const DeviceScene &sc, int mid, float3 wi, D3 pos, uint32_t bins, float3 wo, float *pdf) {
   const DevMedium &m = sc.media[mid];
-  if (is_atmosphere(m)) return phase_mix_eval(atmo_phase(m, pos, bins), wi, wo, pdf);
+  if (kAtmo && is_atmosphere(m)) return phase_mix_eval(atmo_phase(m, pos, bins), wi, wo, pdf);
   const float v = phase_eval(m.phase_kind, m.phase_g, wi, wo);
   *pdf = v;
   return f4(v);
@@ -336,12 +393,35 @@ TT_HD bool track_medium(const DeviceScene &sc, int mid, D3 org, float3 dir, doub
   return false;
 }
 
+// Tracking through a homogeneous medium: the majorant is the extinction, so the first collision is real.
+TT_HD bool track_homogeneous(const DeviceScene &sc, int mid, double len, uint32_t bins, Pcg &rng, NullMat &w_nulls, NullMat &w_track,
+                             double &t_out) {
+  const float4 st = take(sc.media[mid].sigma_t, bins);
+  const double mfp = 1.0 / (double)st.x;
+  const double v = (double)(-logf(1.f - rng.uniform())) * mfp;
+  const double t = v < kLargeNumber ? v : kLargeNumber;
+  const double seg = t < len ? t : len;
+  const float4 tr = exp_neg(seg, st);
+  t_out = t;
+  if (t >= len) {
+    nm_acc(w_track, tr, tr);
+    nm_acc(w_nulls, tr, tr);
+    return false;
+  }
+  rng.uniform();  // the draw between a real and a null collision
+  nm_acc(w_track, tr * st, tr * st);
+  nm_acc(w_nulls, tr * st, tr);
+  return true;
+}
+
 // nullpath::Transmission(medium, ...) (media_integrator.cxx:288-327): ratio tracking through
 // null collisions only.
+template <bool kAtmo>
 TT_HD void transmit_medium(const DeviceScene &sc, int mid, D3 org, float3 dir, double len, uint32_t bins, Pcg &rng, NullMat &w_nulls,
                            NullMat &w_track) {
-  const float4 maj = medium_majorant(sc, mid, org, dir, len, bins);
+  const float4 maj = medium_majorant<kAtmo>(sc, mid, org, dir, len, bins);
   const double mfp = 1.0 / (double)maj.x;
+  const MediumAt med = load_medium<kAtmo>(sc, mid, bins);
   double t = 0.;
   for (int it = 1; it < kMaxTrackingIterations; ++it) {
     const double v = (double)(-logf(1.f - rng.uniform())) * mfp;
@@ -355,7 +435,7 @@ TT_HD void transmit_medium(const DeviceScene &sc, int mid, D3 org, float3 dir, d
       return;
     }
     float4 ss, st;
-    medium_coeffs(sc, mid, d3_along(org, dir, t), bins, ss, st);
+    medium_coeffs<kAtmo>(sc, mid, med, d3_along(org, dir, t), bins, ss, st);
     const float4 sn = null_coeff(maj, st);
     nm_acc(w_track, tr * sn, tr * sn);
     nm_acc(w_nulls, tr * sn, tr * maj);
@@ -483,6 +563,7 @@ TT_HD void cross_boundaries(const DeviceScene &sc, Tracker &tr, const BoundaryHi
 
 // nullpath::Tracking(scene, ...) (media_integrator.cxx:330-376) along [0, seg_end): returns true
 // on a real collision at distance t_coll with scattering coefficient ss.
+template <bool kAtmo = true>
 TT_HD bool track_scene(const DeviceScene &sc, float3 org, float3 dir, double seg_end, uint32_t bins, Pcg &rng, Tracker &tr,
                        NullMat &nulls, NullMat &track, double &t_coll, float4 &ss, int &coll_medium) {
   double tnear = 0.;
@@ -492,7 +573,10 @@ TT_HD bool track_scene(const DeviceScene &sc, float3 org, float3 dir, double seg
     const double sfar = bh.n ? bh.t : seg_end;
     if ((int)tr.cur != kVacuum) {
       double t;
-      if (track_medium(sc, (int)tr.cur, d3_along(d3(org), dir, tnear), dir, sfar - tnear, bins, rng, nulls, track, t, ss)) {
+      const bool collided =
+          kAtmo ? track_medium(sc, (int)tr.cur, d3_along(d3(org), dir, tnear), dir, sfar - tnear, bins, rng, nulls, track, t, ss)
+                : track_homogeneous(sc, (int)tr.cur, sfar - tnear, bins, rng, nulls, track, t);
+      if (collided) {
         t_coll = tnear + t;
         coll_medium = (int)tr.cur;
         return true;
@@ -507,6 +591,7 @@ TT_HD bool track_scene(const DeviceScene &sc, float3 org, float3 dir, double seg
 
 // nullpath::Transmission(scene, ...) (media_integrator.cxx:379-409) along [0, length) after the
 // caller's occlusion test.
+template <bool kAtmo>
 TT_HD void transmit_scene(const DeviceScene &sc, float3 org, float3 dir, double length, uint32_t bins, Pcg &rng, Tracker &tr,
                           NullMat &nulls, NullMat &track) {
   double tnear = 0.;
@@ -516,7 +601,7 @@ TT_HD void transmit_scene(const DeviceScene &sc, float3 org, float3 dir, double 
     const double sfar = bh.n ? bh.t : length;
     if ((int)tr.cur != kVacuum) {
       NullMat s_n = nm_ones(), s_t = nm_ones();
-      transmit_medium(sc, (int)tr.cur, d3_along(d3(org), dir, tnear), dir, sfar - tnear, bins, rng, s_n, s_t);
+      transmit_medium<kAtmo>(sc, (int)tr.cur, d3_along(d3(org), dir, tnear), dir, sfar - tnear, bins, rng, s_n, s_t);
       nm_acc(nulls, s_n);
       nm_acc(track, s_t);
     }

@@ -744,6 +744,9 @@ void BuildTables(ttgpu_handle *h, const ttgpu_scene &s, double bb_diag) {
   bool any_medium = s.empty_space_medium >= 0;
   for (int i = 0; i < s.num_materials; ++i) any_medium |= s.materials[i].medium >= 0 || s.materials[i].outer_medium >= 0;
   h->dsc.has_media = any_medium ? 1 : 0;
+  h->dsc.has_atmosphere = 0;
+  for (int i = 0; i < s.num_media; ++i)
+    if (s.media[i].kind == TTGPU_MEDIUM_ATMOSPHERE || s.media[i].kind == TTGPU_MEDIUM_ATMOSPHERE_TABULATED) h->dsc.has_atmosphere = 1;
   h->dsc.cam_tracker = CameraTracker(s, h->dsc.empty_space_medium);
   // Camera (src/camera.hxx:43-93, 165-174).
   const auto &c = s.camera;

@@ -89,3 +89,30 @@ def test_gpu_fog_furnace(gpu_lib, variant, mode):
     expected = spectrum_to_rgb(flat(1.0 / (1 - rho)))
     print(variant, mode, mean, "+-", se, "expected", expected, flush=True)
     assert np.all(np.abs(mean - expected) < 4 * se + 2e-3 * np.abs(expected))
+
+
+@pytest.mark.parametrize("build,mode", [(configs.medium_sphere, abi.SAMPLE_BOTH), (configs.fog_box, abi.SAMPLE_BOTH),
+                                        (configs.fog_box, abi.SAMPLE_LIGHTS), (configs.absorber_slab, abi.SAMPLE_BOTH)])
+def test_homogeneous_kernels_match_the_general_ones(gpu_lib, build, mode):
+    """Scenes whose media are all homogeneous run kernels without the atmosphere's code, with a
+    single collision per segment instead of the null-collision loop.  An atmosphere that no material
+    names sends the same scene through the general kernels: every path draws the same random numbers,
+    so pixels agree to FP32 rounding of the separately compiled code (2^-23 per operation, some
+    hundred operations per path), but for paths whose rounding flips a decision."""
+    def render(general):
+        s = build(48, 40)
+        if general:
+            s.add_atmosphere([0.0, -6371.0, 0.0], 6371.0, 100.0, 8.0, 1.2, 0.76, configs.rayleigh_sigma_s_per_km(),
+                             np.full(36, 20e-3), np.full(36, 2.22e-3))
+        p = abi.default_params(48, 40, max_depth=10, seed=21)
+        p.sample_mode = mode
+        with GpuRenderer(s, p) as r:
+            r.render_spp(8)
+            return r.mean_image(), (r.stats()["rays_closest"], r.stats()["rays_shadow"])
+    a, rays_a = render(False)
+    b, rays_b = render(True)
+    assert b.max() > 0
+    off = np.abs(a - b) > 1e-4 * np.abs(b) + 1e-6
+    print(f"{off.mean():.2e} of the values differ; rays {rays_a} {rays_b}", flush=True)
+    assert off.mean() < 2e-3
+    assert abs(rays_a[0] - rays_b[0]) <= 1e-4 * rays_b[0] + 2 and abs(rays_a[1] - rays_b[1]) <= 1e-4 * rays_b[1] + 2
