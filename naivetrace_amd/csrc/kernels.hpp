@@ -62,6 +62,9 @@ void LaunchCameraConnect(const DeviceScene &sc, uint64_t first, uint64_t count, 
 void LaunchShadow(const DeviceScene &sc, const PathQueues &q, uint32_t max_count, double *fb, double *fb_sq, hipStream_t st);
 void LaunchTraceRays(const DeviceScene &sc, int64_t n, const float *org, const float *dir, const float *tmax, float *t, int32_t *prim,
                      float *u, float *v, int32_t *occl, int brute, hipStream_t st);
+// Ray arrays of n <= stride rays from page-locked memory: origins at 0, directions at 12 x stride,
+// tmax at 24 x stride bytes, in both; stride is a multiple of 16.
+void LaunchCopyRays(void *to, const void *from, size_t n, size_t stride, hipStream_t st);
 void LaunchSampleShader(const DevShader &s, float3 wi, float3 ng, float3 ns, uint32_t bins, float rough, uint64_t seed, int64_t n,
                         float *d, float *v, float *p, hipStream_t st);
 void LaunchEvalShader(const DevShader &s, float3 wi, float3 ng, float3 ns, uint32_t bins, float rough, int64_t n, const float *dirs,

@@ -1478,6 +1478,159 @@ bool RenderPass(ttgpu_handle *h, int spp) {
   return complete;
 }
 
+// ---- ray queries through page-locked staging ---------------------------------------------
+// The caller's rays are copied in chunks into page-locked slots; a kernel takes a slot's rays to
+// the device, and the trace writes the results into the slot.  The slots' streams overlap, so the
+// host copies one chunk while the GPU fetches and traces others.  With seven hipMalloc / hipFree
+// pairs and seven copies of pageable arrays per call, a million closest-hit rays took 3.0 ms, of
+// which 0.35 were tracing; now 1.9 ms, bound by the host's copies and the link (occlusion: 1.66 and
+// 1.45 ms).  Chunks of 2^16 or 2^15 rays were slower (launches; 3.75 and 5.3 ms for both queries
+// against 3.65), and tracing straight from the page-locked rays took 5.2 ms.
+constexpr int kStageSlots = 3;
+constexpr size_t kStageRays = 1 << 17;                // of a slot at most: 2048 waves, 5.8 MB
+constexpr size_t kMinStageRays = 1 << 10;
+constexpr size_t kRayBytes = 28;                      // origin, direction, tmax
+constexpr size_t kStageBytesPerRay = kRayBytes + 16;  // and t, prim, u, v (or occluded)
+struct RayStage {
+  unsigned char *host = nullptr, *dev = nullptr;  // slots and their device address
+  unsigned char *rays = nullptr;                  // device memory: a slot's rays each
+  hipStream_t stream[kStageSlots] = {};           // of several slots; a single one uses the handle's
+  hipEvent_t done[kStageSlots] = {}, begin = nullptr;
+  size_t slot_rays = 0;
+  int slots = 0, device = 0;
+  void Free() {
+    for (auto &e : done)
+      if (e) (void)hipEventDestroy(e);
+    if (begin) (void)hipEventDestroy(begin);
+    for (auto &st : stream)
+      if (st) (void)hipStreamDestroy(st);
+    if (host) (void)hipHostFree(host);
+    if (rays) (void)hipFree(rays);
+    *this = RayStage{};
+  }
+};
+// Stages are shared by the process's handles (a query borrows one, so queries of several threads
+// each have their own); at most kMaxIdleStages are kept, and none after the last handle.
+constexpr size_t kMaxIdleStages = 4;
+std::mutex g_stage_mu;
+std::vector<RayStage> g_idle_stages;
+int g_handles = 0;
+
+// A stage for `count` rays: one slot of at least that many, or kStageSlots of kStageRays.
+RayStage BorrowStage(size_t count) {
+  RayStage s;
+  Check(hipGetDevice(&s.device), "hipGetDevice");
+  s.slots = count > kStageRays ? kStageSlots : 1;
+  s.slot_rays = kMinStageRays;
+  while (s.slot_rays < std::min(count, kStageRays)) s.slot_rays *= 2;
+  {
+    std::lock_guard<std::mutex> lock(g_stage_mu);
+    for (size_t k = 0; k < g_idle_stages.size(); ++k) {
+      const RayStage idle = g_idle_stages[k];
+      if (idle.device != s.device || idle.slots < s.slots || idle.slot_rays < s.slot_rays) continue;
+      g_idle_stages.erase(g_idle_stages.begin() + k);
+      return idle;
+    }
+  }
+  try {
+    const size_t rays = s.slots * s.slot_rays;
+    Check(hipHostMalloc((void **)&s.host, rays * kStageBytesPerRay), "hipHostMalloc");
+    Check(hipHostGetDevicePointer((void **)&s.dev, s.host, 0), "hipHostGetDevicePointer");
+    Check(hipMalloc((void **)&s.rays, rays * kRayBytes), "hipMalloc");
+    Check(hipEventCreateWithFlags(&s.begin, hipEventDisableTiming), "hipEventCreate");
+    for (int k = 0; k < s.slots; ++k) {
+      Check(hipEventCreateWithFlags(&s.done[k], hipEventDisableTiming), "hipEventCreate");
+      if (s.slots > 1) Check(hipStreamCreateWithFlags(&s.stream[k], hipStreamNonBlocking), "hipStreamCreate");
+    }
+  } catch (...) {
+    s.Free();
+    throw;
+  }
+  return s;
+}
+void ReturnStage(RayStage s) {
+  {
+    std::lock_guard<std::mutex> lock(g_stage_mu);
+    if (g_handles > 0) {
+      g_idle_stages.push_back(s);
+      if (g_idle_stages.size() <= kMaxIdleStages) return;
+      // The smallest goes.
+      auto small = std::min_element(g_idle_stages.begin(), g_idle_stages.end(), [](const RayStage &a, const RayStage &b) {
+        return a.slots * a.slot_rays < b.slots * b.slot_rays;
+      });
+      s = *small;
+      g_idle_stages.erase(small);
+    }
+  }
+  s.Free();
+}
+void CountHandle(int d) {
+  std::vector<RayStage> drop;
+  {
+    std::lock_guard<std::mutex> lock(g_stage_mu);
+    g_handles += d;
+    if (g_handles == 0) drop.swap(g_idle_stages);
+  }
+  for (auto &s : drop) s.Free();
+}
+
+// Closest hits (t, prim, u, v) or, with `occluded`, occlusion of `count` rays.
+void QueryRays(ttgpu_handle *h, size_t count, const float *org, const float *dir, const float *tmax, float *t, int32_t *prim, float *u,
+               float *v, int32_t *occluded, int brute) {
+  struct Loan {
+    hipStream_t own;
+    RayStage s;
+    ~Loan() {  // no kernel may still use the slots
+      (void)hipStreamSynchronize(own);
+      for (auto &st : s.stream)
+        if (st) (void)hipStreamSynchronize(st);
+      ReturnStage(s);
+    }
+  } loan{h->stream, BorrowStage(count)};
+  RayStage &s = loan.s;
+  const size_t R = s.slot_rays, chunks = (count + R - 1) / R, slots = (size_t)s.slots;
+  // Slot layout: origins (12 R bytes), directions (12 R), tmax (4 R), then four result arrays (4 R each).
+  auto in_slot = [&](unsigned char *base, size_t slot, size_t offset) { return base + slot * R * kStageBytesPerRay + offset * R; };
+  auto collect = [&](size_t chunk) {
+    const size_t slot = chunk % slots, at = chunk * R, n = std::min(R, count - at);
+    Check(hipEventSynchronize(s.done[slot]), "hipEventSynchronize");
+    if (occluded) {
+      std::memcpy(occluded + at, in_slot(s.host, slot, 28), 4 * n);
+      return;
+    }
+    std::memcpy(t + at, in_slot(s.host, slot, 28), 4 * n);
+    std::memcpy(prim + at, in_slot(s.host, slot, 32), 4 * n);
+    std::memcpy(u + at, in_slot(s.host, slot, 36), 4 * n);
+    std::memcpy(v + at, in_slot(s.host, slot, 40), 4 * n);
+  };
+  if (slots > 1) {
+    Check(hipEventRecord(s.begin, h->stream), "hipEventRecord");
+    for (auto &st : s.stream) Check(hipStreamWaitEvent(st, s.begin, 0), "hipStreamWaitEvent");
+  }
+  for (size_t c = 0; c < chunks; ++c) {
+    if (c >= slots) collect(c - slots);
+    const size_t slot = c % slots, at = c * R, n = std::min(R, count - at);
+    std::memcpy(in_slot(s.host, slot, 0), org + 3 * at, 12 * n);
+    std::memcpy(in_slot(s.host, slot, 12), dir + 3 * at, 12 * n);
+    std::memcpy(in_slot(s.host, slot, 24), tmax + at, 4 * n);
+    hipStream_t st = slots > 1 ? s.stream[slot] : h->stream;
+    unsigned char *rays = s.rays + slot * R * kRayBytes;
+    auto ray = [&](size_t offset) { return reinterpret_cast<const float *>(rays + offset * R); };
+    auto out = [&](size_t offset) { return reinterpret_cast<float *>(in_slot(s.dev, slot, offset)); };
+    LaunchCopyRays(rays, in_slot(s.dev, slot, 0), n, R, st);
+    if (occluded)
+      LaunchTraceRays(h->dsc, (int64_t)n, ray(0), ray(12), ray(24), nullptr, nullptr, nullptr, nullptr,
+                      reinterpret_cast<int32_t *>(out(28)), 0, st);
+    else
+      LaunchTraceRays(h->dsc, (int64_t)n, ray(0), ray(12), ray(24), out(28), reinterpret_cast<int32_t *>(out(32)), out(36), out(40),
+                      nullptr, brute, st);
+    Check(hipGetLastError(), "launch");
+    Check(hipEventRecord(s.done[slot], st), "hipEventRecord");
+  }
+  for (size_t c = chunks > slots ? chunks - slots : 0; c < chunks; ++c) collect(c);
+  CheckTraversal(h->stream);  // of every chunk
+}
+
 }  // namespace
 
 extern "C" {
@@ -1577,6 +1730,7 @@ int ttgpu_create(const ttgpu_scene *scene, const ttgpu_params *params, ttgpu_han
     auto t1 = std::chrono::steady_clock::now();
     h->stats.upload_ms = std::chrono::duration<double, std::milli>(t1 - t0).count() - h->stats.bvh_build_ms;
     *out = h;
+    CountHandle(1);
     return TTGPU_OK;
   } catch (const std::invalid_argument &e) {
     g_create_error = e.what();
@@ -1593,7 +1747,11 @@ int ttgpu_create(const ttgpu_scene *scene, const ttgpu_params *params, ttgpu_han
   }
 }
 
-void ttgpu_destroy(ttgpu_handle *h) { delete h; }
+void ttgpu_destroy(ttgpu_handle *h) {
+  if (!h) return;
+  delete h;
+  CountHandle(-1);
+}
 
 const char *ttgpu_last_error(const ttgpu_handle *h) { return h ? h->err.c_str() : g_create_error.c_str(); }
 
@@ -1765,29 +1923,11 @@ static int TraceClosestImpl(ttgpu_handle *h, int64_t count, const float *org, co
   if (!h || count < 0 || (count && (!org || !dir || !tmax || !t || !prim || !u || !v))) return TTGPU_ERR_INVALID_ARGUMENT;
   if (count == 0) return TTGPU_OK;
   TTGPU_GUARD(h, {
-    float *d_org = nullptr, *d_dir = nullptr, *d_tmax = nullptr, *d_t = nullptr, *d_u = nullptr, *d_v = nullptr;
-    int32_t *d_prim = nullptr;
-    size_t n = (size_t)count;
-    Check(hipMalloc(&d_org, 3 * n * 4), "hipMalloc"); Check(hipMalloc(&d_dir, 3 * n * 4), "hipMalloc");
-    Check(hipMalloc(&d_tmax, n * 4), "hipMalloc"); Check(hipMalloc(&d_t, n * 4), "hipMalloc");
-    Check(hipMalloc(&d_u, n * 4), "hipMalloc"); Check(hipMalloc(&d_v, n * 4), "hipMalloc");
-    Check(hipMalloc(&d_prim, n * 4), "hipMalloc");
-    Check(hipMemcpy(d_org, org, 3 * n * 4, hipMemcpyHostToDevice), "H2D");
-    Check(hipMemcpy(d_dir, dir, 3 * n * 4, hipMemcpyHostToDevice), "H2D");
-    Check(hipMemcpy(d_tmax, tmax, n * 4, hipMemcpyHostToDevice), "H2D");
     if (h->dsc.num_prims > 0) {
-      LaunchTraceRays(h->dsc, count, d_org, d_dir, d_tmax, d_t, d_prim, d_u, d_v, nullptr, brute, h->stream);
-      Check(hipGetLastError(), "launch");
-      Check(hipStreamSynchronize(h->stream), "sync");
-      CheckTraversal(h->stream);
-      Check(hipMemcpy(t, d_t, n * 4, hipMemcpyDeviceToHost), "D2H");
-      Check(hipMemcpy(prim, d_prim, n * 4, hipMemcpyDeviceToHost), "D2H");
-      Check(hipMemcpy(u, d_u, n * 4, hipMemcpyDeviceToHost), "D2H");
-      Check(hipMemcpy(v, d_v, n * 4, hipMemcpyDeviceToHost), "D2H");
+      QueryRays(h, (size_t)count, org, dir, tmax, t, prim, u, v, nullptr, brute);
     } else {
-      for (size_t i = 0; i < n; ++i) { t[i] = INFINITY; prim[i] = -1; u[i] = v[i] = 0.f; }
+      for (int64_t i = 0; i < count; ++i) { t[i] = INFINITY; prim[i] = -1; u[i] = v[i] = 0.f; }
     }
-    (void)hipFree(d_org); (void)hipFree(d_dir); (void)hipFree(d_tmax); (void)hipFree(d_t); (void)hipFree(d_u); (void)hipFree(d_v); (void)hipFree(d_prim);
     return TTGPU_OK;
   })
 }
@@ -1916,24 +2056,8 @@ int ttgpu_trace_occluded(ttgpu_handle *h, int64_t count, const float *org, const
   if (!h || count < 0 || (count && (!org || !dir || !tmax || !occluded))) return TTGPU_ERR_INVALID_ARGUMENT;
   if (count == 0) return TTGPU_OK;
   TTGPU_GUARD(h, {
-    size_t n = (size_t)count;
-    float *d_org = nullptr, *d_dir = nullptr, *d_tmax = nullptr;
-    int32_t *d_occ = nullptr;
-    Check(hipMalloc(&d_org, 3 * n * 4), "hipMalloc"); Check(hipMalloc(&d_dir, 3 * n * 4), "hipMalloc");
-    Check(hipMalloc(&d_tmax, n * 4), "hipMalloc"); Check(hipMalloc(&d_occ, n * 4), "hipMalloc");
-    Check(hipMemcpy(d_org, org, 3 * n * 4, hipMemcpyHostToDevice), "H2D");
-    Check(hipMemcpy(d_dir, dir, 3 * n * 4, hipMemcpyHostToDevice), "H2D");
-    Check(hipMemcpy(d_tmax, tmax, n * 4, hipMemcpyHostToDevice), "H2D");
-    if (h->dsc.num_prims > 0) {
-      LaunchTraceRays(h->dsc, count, d_org, d_dir, d_tmax, nullptr, nullptr, nullptr, nullptr, d_occ, 0, h->stream);
-      Check(hipGetLastError(), "launch");
-      Check(hipStreamSynchronize(h->stream), "sync");
-      CheckTraversal(h->stream);
-      Check(hipMemcpy(occluded, d_occ, n * 4, hipMemcpyDeviceToHost), "D2H");
-    } else {
-      for (size_t i = 0; i < n; ++i) occluded[i] = 0;
-    }
-    (void)hipFree(d_org); (void)hipFree(d_dir); (void)hipFree(d_tmax); (void)hipFree(d_occ);
+    if (h->dsc.num_prims > 0) QueryRays(h, (size_t)count, org, dir, tmax, nullptr, nullptr, nullptr, nullptr, occluded, 0);
+    else std::fill(occluded, occluded + count, 0);
     return TTGPU_OK;
   })
 }

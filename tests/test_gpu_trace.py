@@ -129,3 +129,35 @@ def test_full_scale_bvh_matches_bruteforce(gpu_lib):
     assert np.array_equal(occ == 1, hit)
     assert np.all(occ_half[hit] == 0)
     assert np.all(occ_past[hit] == 1)
+
+
+@pytest.mark.parametrize("count", [1, 63, 1024, 1025, 1 << 17, (1 << 17) + 1, 4 * (1 << 17) + 3])
+def test_query_chunks(count):
+    """Queries of one slot and of several, whole and partly filled, against the same rays asked for
+    in other portions (each ray's answer is its own: equal bits) and against brute force."""
+    from concurrent.futures import ThreadPoolExecutor
+    rng = np.random.default_rng(count)
+    pool = 5000
+    org = rng.uniform(-0.3, 0.3, (pool, 3)).astype(np.float32)
+    d = rng.normal(size=(pool, 3))
+    d = (d / np.linalg.norm(d, axis=1, keepdims=True)).astype(np.float32)
+    tmax = np.where(rng.random(pool) < 0.3, 0.4, 1e30).astype(np.float32)
+    pick = rng.integers(0, pool, count)
+    with GpuRenderer(configs.cornell_box(8, 8), abi.default_params(8, 8)) as r:
+        portions = [slice(k, k + 700) for k in range(0, pool, 700)]
+        parts = [r.trace_closest(org[p], d[p], tmax[p]) for p in portions]
+        want = [np.concatenate([p[k] for p in parts]) for k in range(4)]
+        want_occ = np.concatenate([r.trace_occluded(org[p], d[p], tmax[p]) for p in portions])
+        brute = r.trace_closest(org, d, tmax, bruteforce=True)
+        assert np.array_equal(want[0], brute[0])
+        ask = lambda _: (r.trace_closest(org[pick], d[pick], tmax[pick]), r.trace_occluded(org[pick], d[pick], tmax[pick]))
+        got, occ = ask(0)
+        assert all(np.array_equal(g, w[pick]) for g, w in zip(got, want))
+        assert np.array_equal(occ, want_occ[pick])
+    if count == (1 << 17) + 1:  # handles of several threads, each with slots of its own
+        def one(_):
+            with GpuRenderer(configs.cornell_box(8, 8), abi.default_params(8, 8)) as q:
+                return q.trace_closest(org[pick], d[pick], tmax[pick])
+        with ThreadPoolExecutor(3) as ex:
+            for g in ex.map(one, range(3)):
+                assert all(np.array_equal(a, w[pick]) for a, w in zip(g, want))
