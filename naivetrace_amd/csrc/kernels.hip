@@ -1827,10 +1827,11 @@ __global__ void __launch_bounds__(kTraceBlock) k_shadow_guided(DeviceScene sc, P
 // Sort keys of the queued paths for inference: the Morton code of the hit point (from the ray and
 // its hit distance) on a 2^kInferKeyBits grid per axis, so that a sort puts the queries of
 // neighbouring points into the same waves; misses and entries past the queue share the last code and
-// so the sort's end (it is stable: what is past the queue stays last).  The sort takes eight bits a pass: 24 bits cost the three passes of 19 (six bits
-// per axis and one for the misses) and put closer points together.  Keys, sort and inference of a
-// 128 x 128, 1024 spp pass: 19.9 ms with 19 bits, 19.2 with 22, 19.0 with 24; two passes, of 16 bits:
-// 20.6 with five bits per axis, 19.2 - 19.9 with the top 16 of 18.
+// so the sort's end (it is stable: what is past the queue stays last).  The sort takes eight bits a
+// pass: 24 bits cost the three passes of 19 (six bits per axis and one for the misses) and put closer
+// points together.  Keys, sort and inference of a 128 x 128, 1024 spp pass: 19.9 ms with 19 bits, 19.2
+// with 22, 19.0 with 24; two passes, of 16 bits: 20.6 with five bits per axis, 19.2 - 19.9 with the top
+// 16 of 18.
 constexpr int kInferKeyBits = 8;
 constexpr uint32_t kInferMissKey = (1u << (3 * kInferKeyBits)) - 1u;
 __global__ void __launch_bounds__(256) k_infer_keys(PathQueues q, const uint32_t *__restrict__ queue, const uint32_t *__restrict__ count_ptr,
