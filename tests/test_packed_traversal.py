@@ -13,7 +13,7 @@ CSRC = os.path.join(ROOT, "naivetrace_amd", "csrc")
 
 
 @pytest.fixture(scope="module")
-def checker(tmp_path_factory):
+def program(tmp_path_factory):
     from naivetrace_amd import build
     exe = str(tmp_path_factory.mktemp("packed") / "packed_traversal_check")
     subprocess.run([build.hipcc(), "-O2", "-std=c++17", "-x", "hip", f"--offload-arch={build.ARCH}", "-Wno-unused-result",
@@ -22,8 +22,8 @@ def checker(tmp_path_factory):
     return exe
 
 
-def run(checker, *args):
-    r = subprocess.run([checker, *map(str, args)], capture_output=True, text=True, timeout=300)
+def run(program, *args):
+    r = subprocess.run([program, *map(str, args)], capture_output=True, text=True, timeout=300)
     print(r.stdout.strip())
     assert r.returncode == 0, r.stdout + r.stderr
     f = r.stdout.split()
@@ -32,16 +32,16 @@ def run(checker, *args):
 
 @pytest.mark.parametrize("grid,offset,rays", [(1, 0.0, 2000), (2, 0.0, 5000), (7, 0.0, 20000), (60, 0.0, 40000), (80, 5000.0, 40000),
                                               (512, 0.0, 16000)])
-def test_packed_traversal_matches_brute_force(checker, grid, offset, rays):
-    val = run(checker, grid, offset, rays)
+def test_packed_traversal_matches_brute_force(program, grid, offset, rays):
+    val = run(program, grid, offset, rays)
     assert val("box_errors") == 0 and val("layout_errors") == 0
     assert val("hits") > (10 if grid < 7 else 300)
     for k in ("closest_diff", "prim_diff", "anyhit_diff"):
         assert val(k) == 0, k
 
 
-def test_packed_traversal_spills_its_stack(checker):
-    val = run(checker, 400, 0.0, 300, "comb")
+def test_packed_traversal_spills_its_stack(program):
+    val = run(program, 400, 0.0, 300, "comb")
     assert val("max_stack") > val("lds_stack")
     for k in ("closest_diff", "prim_diff", "anyhit_diff"):
         assert val(k) == 0, k
