@@ -840,10 +840,13 @@ void AllocateQueues(ttgpu_handle *h) {
     h->stats.state_bytes += (size_t)N * (48 * nvtx + 16) + (size_t)q.rec_capacity * 32;
   }
   if (bdpt) {
-    // 2^18 samples in flight: four waves per SIMD in the walks, 0.7 GB at depth 8, 1.3 GB at 16.
+    // Samples in flight: 2^18, four waves per SIMD in the walks (0.7 GB at depth 8, 1.4 GB at 16), or
+    // fewer when the caller asks for a smaller wavefront, down to one block of the walk per four CUs
+    // (2^13 samples, 23 MB at depth 8), below which a chunk's launches cost more than its samples.
     BdptWork &w = h->bdpt;
     w.max_nodes = h->params.max_ray_depth + 1;
-    w.capacity = 1u << 18;
+    w.capacity = std::max(1u << 13, std::min(1u << 18, h->capacity));
+    h->stats.wavefront_paths = (int32_t)w.capacity;
     w.verts = (float4 *)h->Alloc<uint8_t>(w.capacity * BdptVertexBytes(w.max_nodes));
     w.pairs = h->Alloc<uint32_t>(w.capacity * BdptMaxPairs(w.max_nodes));
     w.info = h->Alloc<uint2>(w.capacity);

@@ -1,104 +1,49 @@
-// Host-side check of the packed traversal tree (TravNode), running the traversal code of
-// naivetrace_amd/csrc/trace.hpp (compiled for the host, the same source the kernels use):
+// Host-side check of the surface BVH as the device traverses it (TravNode), running the traversal code
+// of naivetrace_amd/csrc/trace.hpp (compiled for the host, the same source the kernels use):
 //   * every packed child box, evaluated in exact (double) arithmetic, contains the child's true box
 //     with room to spare, slots are inner children first, and every primitive is in one leaf;
 //   * closest-hit distance and primitive and the any-hit answer equal a brute-force loop over all
-//     primitives for random, axis-parallel and vertex-aimed rays (a primitive may differ on an
-//     exactly equal distance).
-// Usage: packed_traversal_check <grid> <x offset> <rays> [comb]; prints a summary; exit status 1
-// when a box or the layout is wrong or a stack overflowed.  "comb" as in bvh_quantized_check.cpp.
+//     primitives (every ray when the scene is small, every 16th otherwise) for random, axis-parallel
+//     and vertex-aimed rays (a primitive may differ on an exactly equal distance: ties on shared edges);
+//   * a plain descent of the tree's float planes (check_scene.hpp) is compared the same way.
+// Far from the origin the slab test (plane / dir - org / dir, as in Embree's non-robust mode that the
+// reference uses) cancels and loses some grazing hits; the caller decides what to require there.
+// Usage: packed_traversal_check <grid> <x offset> <rays> [comb | spheres]; prints a summary; exit status
+// 1 when a box or the layout is wrong or a stack overflowed.  "comb": grid x 1000 teeth of
+// check::comb instead of the heightfield; "spheres": grid spheres over the heightfield.
 static long g_overflows = 0;
 #define TTGPU_STACK_OVERFLOW() (++g_overflows)
-#include "../../naivetrace_amd/csrc/bvh_build.hpp"
-#include "../../naivetrace_amd/csrc/device_scene.hpp"
-#include "../../naivetrace_amd/csrc/trace.hpp"
+#include "check_scene.hpp"
 #include <cstdio>
-#include <cmath>
-#include <cstring>
+#include <cstdlib>
 #include <string>
-#include <random>
-#include <vector>
-using namespace ttgpu;
-
-// The traversal's three copies of the records in the packed order (copy k: triangle vertices in the
-// order ((k+1) mod 3, (k+2) mod 3, k), w of the first = leaf-order index), as the library uploads them.
-static std::vector<ttgpu::PrimRecord> per_axis_copies(const std::vector<ttgpu::PrimRecord> &recs, const std::vector<uint32_t> &order) {
-  std::vector<ttgpu::PrimRecord> out(3 * recs.size());
-  for (int k = 0; k < 3; ++k)
-    for (size_t i = 0; i < recs.size(); ++i) {
-      auto perm = [&](float4 v) {
-        const float c[3] = {v.x, v.y, v.z};
-        return make_float4(c[(k + 1) % 3], c[(k + 2) % 3], c[k], v.w);
-      };
-      ttgpu::PrimRecord r = recs[order[i]];
-      const int index = (int)order[i];
-      std::memcpy(&r.a.w, &index, 4);
-      r.a = perm(r.a); r.b = perm(r.b); r.c = perm(r.c);
-      out[k * recs.size() + i] = r;
-    }
-  return out;
-}
-
+using namespace check;
 
 int main(int argc, char **argv) {
   const int grid = argc > 1 ? atoi(argv[1]) : 100;
   const float off = argc > 2 ? (float)atof(argv[2]) : 0.f;
   const int rays = argc > 3 ? atoi(argv[3]) : 50000;
-  const bool comb = argc > 4 && std::string(argv[4]) == "comb";
+  const std::string kind = argc > 4 ? argv[4] : "";
+  const bool teeth = kind == "comb";
   std::mt19937 rng(7);
   std::uniform_real_distribution<float> U(0.f, 1.f);
-  // A bumpy heightfield of grid x grid cells plus small random triangles floating above it.
-  std::vector<float3> v0, v1, v2;
-  std::vector<float> h((grid + 1) * (grid + 1));
-  if (comb) {
-    // Tooth k at x = off + 0.01 (g^k - 1) / (g - 1) (spacing growing geometrically, e^4 over the
-    // comb, so the binned SAH splits unevenly and the tree is deep): (y, z) corners (1, -1), (1, 1),
-    // (-0.8, 1), each turned by a small random angle about x; the axis (y = z = 0) passes beside
-    // every tooth, inside its box.
-    const int nt = grid * 1000;
-    const double g = 1.0 + 4.0 / nt;
-    for (int k = 0; k < nt; ++k) {
-      const float a = 0.2f * (U(rng) - 0.5f), ca = cosf(a), sa = sinf(a);
-      const float x = off + (float)(0.01 * (std::pow(g, (double)k) - 1.0) / (g - 1.0));
-      auto yz = [&](float y, float z) { return mk(x + 0.004f * (y + 1.f), ca * y - sa * z, sa * y + ca * z); };
-      v0.push_back(yz(1.f, -1.f)); v1.push_back(yz(1.f, 1.f)); v2.push_back(yz(-0.8f, 1.f));
-    }
-  }
-  for (int i = 0; i <= grid && !comb; ++i)
-    for (int j = 0; j <= grid; ++j) h[i * (grid + 1) + j] = 3.f * sinf(i * 0.13f) * cosf(j * 0.07f) + 0.3f * U(rng);
-  for (int i = 0; i < grid && !comb; ++i)
-    for (int j = 0; j < grid; ++j) {
-      const float3 a = mk(i + off, h[i * (grid + 1) + j], j), b = mk(i + 1 + off, h[(i + 1) * (grid + 1) + j], j);
-      const float3 c = mk(i + off, h[i * (grid + 1) + j + 1], j + 1), d = mk(i + 1 + off, h[(i + 1) * (grid + 1) + j + 1], j + 1);
-      v0.push_back(a); v1.push_back(b); v2.push_back(c);
-      v0.push_back(b); v1.push_back(d); v2.push_back(c);
-    }
-  for (int k = 0; k < (comb ? 0 : grid * grid / 2); ++k) {
-    const float3 c = mk(U(rng) * grid + off, 4 + 10 * U(rng), U(rng) * grid);
-    v0.push_back(c); v1.push_back(c + mk(U(rng), U(rng), 0)); v2.push_back(c + mk(0, U(rng), U(rng)));
-  }
-  const int n = (int)v0.size();
+  std::vector<Prim> prims = teeth ? comb(grid * 1000, off, rng) : heightfield(grid, off, rng);
+  const int ground = teeth ? 0 : 2 * grid * grid;
+  if (kind == "spheres") add_spheres(prims, grid, grid, off, rng);
+  const int n = (int)prims.size();
   float comb_end = off;
-  for (const float3 &p : v0) comb_end = std::max(comb_end, p.x + 0.01f);
-  std::vector<BuildPrim> bp(n);
-  for (int i = 0; i < n; ++i)
-    for (int k = 0; k < 3; ++k) {
-      const float a = comp3(v0[i], k), b = comp3(v1[i], k), c = comp3(v2[i], k);
-      bp[i].lo[k] = std::min(a, std::min(b, c));
-      bp[i].hi[k] = std::max(a, std::max(b, c));
-    }
-  const BuiltBvh b2 = BuildBvh(bp, 4, 0);
-  const BuiltBvh4 b4 = CollapseToBvh4(b2);
-  const PackedBvh pk = PackTraversal(b4);
-  const TravNode *qn = (const TravNode *)pk.nodes.data();
-  long bad_box = 0, bad_layout = pk.num_nodes != b4.num_nodes;
+  for (const Prim &p : prims) comb_end = std::max(comb_end, p.v[0].x + 0.01f);
+  const Tree tree = build(prims);
+  const PackedBvh &pk = tree.packed;
+  const TravNode *qn = tree.nodes();
+  long bad_box = 0, bad_layout = pk.num_nodes != tree.b4.num_nodes;
   std::vector<int> seen(n, 0);
   // Walk both trees together.
   std::vector<std::pair<int, int>> todo{{0, 0}};
   while (!todo.empty()) {
     const auto [i, j] = todo.back();
     todo.pop_back();
-    const float *f = &b4.nodes[32 * (size_t)i];
+    const float *f = &tree.b4.nodes[32 * (size_t)i];
     int child[4], count[4], slot[4], num = 0, inner = 0;
     std::memcpy(child, f + 24, 16);
     std::memcpy(count, f + 28, 16);
@@ -132,25 +77,22 @@ int main(int argc, char **argv) {
     }
   }
   for (int k = 0; k < n; ++k) bad_layout += seen[k] != 1;
-  std::vector<PrimRecord> recs(n);
-  for (int k = 0; k < n; ++k) {
-    const int p = (int)b2.order[k];
-    recs[k].a = make_float4(v0[p].x, v0[p].y, v0[p].z, 0.f);
-    recs[k].b = make_float4(v1[p].x, v1[p].y, v1[p].z, 0.f);
-    recs[k].c = make_float4(v2[p].x, v2[p].y, v2[p].z, 0.f);
-  }
-  const std::vector<PrimRecord> kzrecs = per_axis_copies(recs, pk.prims);
   std::vector<int> stack(kLdsStack * kTraceBlock);
-  long diff = 0, any_diff = 0, prim_diff = 0, checked = 0, hits = 0;
+  long diff = 0, any_diff = 0, prim_diff = 0, full_diff = 0, checked = 0, hits = 0, sphere_hits = 0;
   int max_sp = 0;
-  const int every = (n <= 2000 || comb) ? 1 : 16;
+  const int every = (n <= 2000 || teeth) ? 1 : 16;
   for (int r = 0; r < rays; ++r) {
     Ray ray;
-    ray.org = mk(U(rng) * grid + off, 2 + 15 * U(rng), U(rng) * grid);
-    float3 d = mk(U(rng) - 0.5f, U(rng) - 0.7f, U(rng) - 0.5f);
+    ray.org.x = U(rng) * grid + off;
+    ray.org.y = 2 + 15 * U(rng);
+    ray.org.z = U(rng) * grid;
+    float3 d;
+    d.x = U(rng) - 0.5f;
+    d.y = U(rng) - 0.7f;
+    d.z = U(rng) - 0.5f;
     if (r % 7 == 0) d = mk(1.f, 0.f, 0.f);
     if (r % 11 == 0) d = mk(0.f, -1.f, 0.f);
-    if (comb) {
+    if (teeth) {
       // Along the axis from before the first tooth (every fourth ray exactly on it, the others
       // up to 0.02 off, some of those tilted enough to hit a tooth further on), or backwards.
       const bool on_axis = r % 4 == 0;
@@ -160,10 +102,8 @@ int main(int argc, char **argv) {
         ray.org.x = comb_end + 1.f;
         d.x = -1.f;
       }
-    }
-    if (!comb && r % 5 == 0) {  // at a vertex shared by several triangles, from above
-      const float3 v = v0[(size_t)(U(rng) * 2 * grid * grid)];
-      d = v - ray.org;
+    } else if (r % 5 == 0) {  // at a vertex shared by several triangles, from above
+      d = prims[(size_t)(U(rng) * ground)].v[0] - ray.org;
     }
     ray.dir = normalize(d);
     ray.tmax = 3e38f;
@@ -175,30 +115,28 @@ int main(int argc, char **argv) {
       Trav t;
       trav_init(t, ray, n, false, stack.data());
       while (t.active()) {
-        trav_advance(t, qn, kzrecs.data(), stack.data(), spill);
+        trav_advance(t, qn, tree.per_axis.data(), stack.data(), spill);
         max_sp = std::max(max_sp, t.sp / kTraceBlock);
       }
       hq = t.hit;
     }
-    const bool oq = traverse<true>(qn, kzrecs.data(), n, ray, stack.data(), aq);
-    const RayPre pp = precompute(ray);
-    float best = 3e38f;
-    int bi = -1;
-    for (int k = 0; k < n; ++k) {
-      float th, u, v;
-      if (intersect_prim(recs[k], pp, ray, best, th, u, v)) { best = th; bi = k; }
-    }
+    const bool oq = traverse<true>(qn, tree.per_axis.data(), n, ray, stack.data(), aq);
+    float best, full;
+    const int bi = brute_force(tree, ray, best), fi = float_planes(tree, ray, full);
     checked++;
     hits += bi >= 0;
+    sphere_hits += bi >= 0 && as_int(tree.recs[bi].b.w) != 0;
     diff += (hq.prim >= 0) != (bi >= 0) || (bi >= 0 && hq.t != best);
+    full_diff += (fi >= 0) != (bi >= 0) || (bi >= 0 && full != best);
     if (bi >= 0 && hq.prim >= 0 && hq.prim != bi) {  // only on an exactly equal distance
       float th, u, v;
-      prim_diff += !(intersect_prim(recs[hq.prim], pp, ray, 3e38f, th, u, v) && th == best);
+      prim_diff += !(intersect_prim(tree.recs[hq.prim], precompute(ray), ray, 3e38f, th, u, v) && th == best);
     }
     any_diff += oq != (bi >= 0);
   }
-  printf("prims %d nodes %d depth %d box_errors %ld layout_errors %ld rays %ld hits %ld closest_diff %ld prim_diff %ld anyhit_diff %ld "
-         "max_stack %d lds_stack %d overflows %ld\n",
-         n, b4.num_nodes, b4.max_depth, bad_box, bad_layout, checked, hits, diff, prim_diff, any_diff, max_sp, kLdsStack, g_overflows);
+  printf("prims %d nodes %d depth %d box_errors %ld layout_errors %ld rays %ld hits %ld sphere_hits %ld closest_diff %ld prim_diff %ld "
+         "anyhit_diff %ld full_closest_diff %ld max_stack %d lds_stack %d overflows %ld\n",
+         n, pk.num_nodes, tree.b4.max_depth, bad_box, bad_layout, checked, hits, sphere_hits, diff, prim_diff, any_diff, full_diff, max_sp,
+         kLdsStack, g_overflows);
   return (bad_box || bad_layout || g_overflows) ? 1 : 0;
 }

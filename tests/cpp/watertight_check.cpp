@@ -1,64 +1,49 @@
 // Host replay of rays aimed at the shared edges and vertices of a closed mesh through the traversal
 // source of the kernels (naivetrace_amd/csrc/trace.hpp, built for the host with the same
-// multiply-add contraction as the device code): every ray must hit, in the quantized BVH4, the
-// full-precision BVH4 and a brute-force loop over the triangles.
+// multiply-add contraction as the device code): every ray must hit, as a closest-hit and as an any-hit
+// query of the packed tree and in a brute-force loop over the triangles, and the closest hit's distance
+// is the loop's.
 // Usage: watertight_check <file>; the file holds int32 nv, nt, nr, then float32 vertices (3 nv),
 // int32 triangles (3 nt), float32 origins (3 nr) and directions (3 nr).  Prints the miss counts.
-#include "../../naivetrace_amd/csrc/bvh_build.hpp"
-#include "../../naivetrace_amd/csrc/device_scene.hpp"
-#include "../../naivetrace_amd/csrc/trace.hpp"
+#include "check_scene.hpp"
 #include <cstdio>
-#include <vector>
 #include <fstream>
-using namespace ttgpu;
-
-// The traversal's three copies of the records (copy k: triangle vertices in the order
-// ((k+1) mod 3, (k+2) mod 3, k)), as the library uploads them.
-static std::vector<ttgpu::PrimRecord> per_axis_copies(const std::vector<ttgpu::PrimRecord> &recs) {
-  std::vector<ttgpu::PrimRecord> out(3 * recs.size());
-  for (int k = 0; k < 3; ++k)
-    for (size_t i = 0; i < recs.size(); ++i) {
-      auto perm = [&](float4 v) {
-        const float c[3] = {v.x, v.y, v.z};
-        return make_float4(c[(k + 1) % 3], c[(k + 2) % 3], c[k], v.w);
-      };
-      ttgpu::PrimRecord r = recs[i];
-      r.a = perm(r.a); r.b = perm(r.b); r.c = perm(r.c);
-      out[k * recs.size() + i] = r;
-    }
-  return out;
-}
+using namespace check;
 
 int main(int argc, char **argv) {
-  // raw binary: nv, nt, nr, then v (nv*3 f32), f (nt*3 i32), org (nr*3 f32), d (nr*3 f32)
+  if (argc < 2) return 2;
   std::ifstream in(argv[1], std::ios::binary);
-  int nv, nt, nr; in.read((char*)&nv, 4); in.read((char*)&nt, 4); in.read((char*)&nr, 4);
-  std::vector<float> v(nv*3), org(nr*3), d(nr*3); std::vector<int> f(nt*3);
-  in.read((char*)v.data(), nv*12); in.read((char*)f.data(), nt*12); in.read((char*)org.data(), nr*12); in.read((char*)d.data(), nr*12);
-  auto V = [&](int i){ return mk(v[3*i], v[3*i+1], v[3*i+2]); };
-  std::vector<BuildPrim> bp(nt);
-  for (int i = 0; i < nt; ++i) for (int k = 0; k < 3; ++k) {
-    float a = comp3(V(f[3*i]),k), b = comp3(V(f[3*i+1]),k), c = comp3(V(f[3*i+2]),k);
-    bp[i].lo[k] = std::min(a, std::min(b,c)); bp[i].hi[k] = std::max(a, std::max(b,c)); }
-  const BuiltBvh b2 = BuildBvh(bp, 4, 0);
-  const BuiltBvh4 b4 = CollapseToBvh4(b2);
-  const std::vector<uint32_t> q = QuantizeBvh4(b4);
-  const QBvh4Node *qn = (const QBvh4Node *)q.data();
-  const Bvh4Node *fn = (const Bvh4Node *)b4.nodes.data();
-  std::vector<PrimRecord> recs(nt);
-  for (int k = 0; k < nt; ++k) { int p = (int)b2.order[k];
-    recs[k].a = make_float4(v[3*f[3*p]], v[3*f[3*p]+1], v[3*f[3*p]+2], 0.f);
-    recs[k].b = make_float4(v[3*f[3*p+1]], v[3*f[3*p+1]+1], v[3*f[3*p+1]+2], 0.f);
-    recs[k].c = make_float4(v[3*f[3*p+2]], v[3*f[3*p+2]+1], v[3*f[3*p+2]+2], 0.f); }
-  const std::vector<PrimRecord> kzrecs = per_axis_copies(recs);
+  int nv, nt, nr;
+  in.read((char *)&nv, 4);
+  in.read((char *)&nt, 4);
+  in.read((char *)&nr, 4);
+  std::vector<float> v(nv * 3), org(nr * 3), d(nr * 3);
+  std::vector<int> f(nt * 3);
+  in.read((char *)v.data(), nv * 12);
+  in.read((char *)f.data(), nt * 12);
+  in.read((char *)org.data(), nr * 12);
+  in.read((char *)d.data(), nr * 12);
+  if (!in) return 2;
+  std::vector<Prim> prims(nt);
+  for (int i = 0; i < nt; ++i)
+    for (int c = 0; c < 3; ++c) prims[i].v[c] = mk(v[3 * f[3 * i + c]], v[3 * f[3 * i + c] + 1], v[3 * f[3 * i + c] + 2]);
+  const Tree tree = build(prims);
   std::vector<int> stack(kLdsStack * kTraceBlock);
-  int qmiss = 0, fmiss = 0, bmiss = 0;
+  int miss = 0, any_miss = 0, brute_miss = 0, diff = 0;
   for (int r = 0; r < nr; ++r) {
-    Ray ray; ray.org = mk(org[3*r], org[3*r+1], org[3*r+2]); ray.dir = mk(d[3*r], d[3*r+1], d[3*r+2]); ray.tmax = 1e30f;
-    HitRec hq, hf; traverse<false>(qn, kzrecs.data(), nt, ray, stack.data(), hq); traverse<false>(fn, kzrecs.data(), nt, ray, stack.data(), hf);
-    const RayPre pp = precompute(ray); float best = 1e30f; int bi = -1;
-    for (int k = 0; k < nt; ++k) { float th,u,w; if (intersect_prim(recs[k], pp, ray, best, th, u, w)) { best = th; bi = k; } }
-    qmiss += hq.prim < 0; fmiss += hf.prim < 0; bmiss += bi < 0;
+    Ray ray;
+    ray.org = mk(org[3 * r], org[3 * r + 1], org[3 * r + 2]);
+    ray.dir = mk(d[3 * r], d[3 * r + 1], d[3 * r + 2]);
+    ray.tmax = 1e30f;
+    HitRec h, a;
+    traverse<false>(tree.nodes(), tree.per_axis.data(), nt, ray, stack.data(), h);
+    const bool any = traverse<true>(tree.nodes(), tree.per_axis.data(), nt, ray, stack.data(), a);
+    float best;
+    const int bi = brute_force(tree, ray, best);
+    miss += h.prim < 0;
+    any_miss += !any;
+    brute_miss += bi < 0;
+    diff += h.prim >= 0 && h.t != best;
   }
-  printf("rays %d quantized misses %d full misses %d brute misses %d\n", nr, qmiss, fmiss, bmiss);
+  printf("rays %d packed misses %d anyhit misses %d brute misses %d distance differences %d\n", nr, miss, any_miss, brute_miss, diff);
 }

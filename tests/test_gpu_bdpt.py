@@ -127,3 +127,25 @@ def test_gpu_bdpt_chunks_and_wave_edges(gpu_lib, w, h, spp, depth):
     if w > 100:
         assert a.sum() > 0
     np.testing.assert_allclose(a, b, rtol=spp * 2.0 ** -23, atol=1e-12)
+
+
+@pytest.mark.parametrize("wavefront,expected", [(0, 1 << 18), (1 << 20, 1 << 18), (20001, 20001), (1, 1 << 13)])
+def test_gpu_bdpt_wavefront_paths_bound_the_workspace(gpu_lib, wavefront, expected):
+    """The caller's wavefront size bounds the samples in flight, and with them the memory of a handle
+    (vertices of 96 B, three per path vertex, and the connections); the image does not depend on it.
+    A sample's FP64 sum is rounded to FP32 once, in whatever order its connections arrive."""
+    w, h, spp, depth = 97, 65, 5, 8
+
+    def render(paths):
+        p = _params(w, h, depth)
+        p.wavefront_paths = paths
+        with GpuRenderer(configs.cornell_box(w, h), p) as r:
+            r.render_spp(spp)
+            rgb, _, n = r.framebuffer()
+            assert np.all(n == spp)
+            return rgb, r.stats()
+    rgb, st = render(wavefront)
+    assert st["wavefront_paths"] == expected
+    assert st["state_bytes"] < expected * (3 * 96 * (depth + 1) + 4 * depth * (depth + 1) // 2 + 32) + 4096
+    ref, _ = render(0)
+    np.testing.assert_allclose(rgb, ref, rtol=spp * 2.0 ** -23, atol=1e-12)
