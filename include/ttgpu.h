@@ -239,7 +239,8 @@ typedef struct ttgpu_params {
   int32_t num_wavelengths;      /* wavelengths per path; 4 on the GPU */
   uint64_t seed;                /* PCG32 initial state; stream = global sample index */
   int64_t wavefront_paths;      /* paths in flight per wavefront; 0 = automatic.  TTGPU_ALGO_BDPT: samples
-                                   in flight, from 2^13 to 2^18 (2.8 KB each at depth 8, 5.5 KB at 16) */
+                                   in flight, from 2^13 to 2^20 (2.8 KB each at depth 8, 5.5 KB at 16) or
+                                   as many as 1.4 GB hold */
   int32_t linear_output;        /* --linear-out for GenerateImage */
   int32_t num_threads;          /* CPU threads (oracle / host side) */
   /* guiding (ptg) */

@@ -840,12 +840,17 @@ void AllocateQueues(ttgpu_handle *h) {
     h->stats.state_bytes += (size_t)N * (48 * nvtx + 16) + (size_t)q.rec_capacity * 32;
   }
   if (bdpt) {
-    // Samples in flight: 2^18, four waves per SIMD in the walks (0.7 GB at depth 8, 1.4 GB at 16), or
-    // fewer when the caller asks for a smaller wavefront, down to one block of the walk per four CUs
-    // (2^13 samples, 23 MB at depth 8), below which a chunk's launches cost more than its samples.
+    // Samples in flight: at every depth the memory that 2^18 samples of the deepest paths take (1.4 GB),
+    // up to 2^20 (the connection list's sample field).  Each chunk ends in a drained launch of each
+    // kernel and a host wait: with 2^18 samples 1024 x 1024 x 16 spp of the Cornell box took 31.1 ms
+    // at depth 2, 42.9 at 3 and 91.1 at 8, with this rule 25.2, 33.1 and 85.8.  Fewer when the caller
+    // asks for a smaller wavefront, down to one block of the walk per four CUs (2^13 samples), below
+    // which a chunk's launches cost more than its samples.
     BdptWork &w = h->bdpt;
     w.max_nodes = h->params.max_ray_depth + 1;
-    w.capacity = std::max(1u << 13, std::min(1u << 18, h->capacity));
+    auto sample_bytes = [](int nodes) { return BdptVertexBytes(nodes) + 4 * BdptMaxPairs(nodes) + 32; };
+    const size_t fit = ((size_t)sample_bytes(kBdptMaxVertices) << 18) / sample_bytes(w.max_nodes);
+    w.capacity = std::max(1u << 13, std::min((uint32_t)std::min<size_t>(fit, 1u << 20), h->capacity));
     h->stats.wavefront_paths = (int32_t)w.capacity;
     w.verts = (float4 *)h->Alloc<uint8_t>(w.capacity * BdptVertexBytes(w.max_nodes));
     w.pairs = h->Alloc<uint32_t>(w.capacity * BdptMaxPairs(w.max_nodes));
@@ -853,7 +858,7 @@ void AllocateQueues(ttgpu_handle *h) {
     w.acc = h->Alloc<double>(3 * (size_t)w.capacity);
     w.count = h->Alloc<uint32_t>(1);
     Check(hipMemset(w.count, 0, sizeof(uint32_t)), "hipMemset bdpt count");
-    h->stats.state_bytes += w.capacity * (BdptVertexBytes(w.max_nodes) + 4 * BdptMaxPairs(w.max_nodes) + 32);
+    h->stats.state_bytes += w.capacity * sample_bytes(w.max_nodes);
   }
   q.vt = nullptr;
   q.wtn_r = q.wtn_c = nullptr;

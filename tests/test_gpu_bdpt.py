@@ -108,9 +108,9 @@ def test_gpu_bdpt_rejects_unsupported(gpu_lib):
         GpuRenderer(s, _params(8, 8, 8))
 
 
-@pytest.mark.parametrize("w,h,spp,depth", [(1, 1, 3, 2), (13, 7, 5, 16), (257, 511, 3, 3)])
+@pytest.mark.parametrize("w,h,spp,depth", [(1, 1, 3, 2), (13, 7, 5, 16), (257, 511, 3, 16), (641, 421, 4, 3)])
 def test_gpu_bdpt_chunks_and_wave_edges(gpu_lib, w, h, spp, depth):
-    """One pass (the last size spans two chunks of 2^18 samples and ends inside a wave) equals the sum
+    """One pass (the last two span two chunks, of 2^18 and 2^20 samples, and end inside a wave) equals the sum
     of 1-spp passes: each sample draws the same numbers wherever it lies in a chunk.  A sample's sum
     runs over at most 136 connections in another order, in FP64, and is rounded to FP32 once."""
     scene = configs.cornell_box(w, h)
@@ -129,12 +129,19 @@ def test_gpu_bdpt_chunks_and_wave_edges(gpu_lib, w, h, spp, depth):
     np.testing.assert_allclose(a, b, rtol=spp * 2.0 ** -23, atol=1e-12)
 
 
-@pytest.mark.parametrize("wavefront,expected", [(0, 1 << 18), (1 << 20, 1 << 18), (20001, 20001), (1, 1 << 13)])
-def test_gpu_bdpt_wavefront_paths_bound_the_workspace(gpu_lib, wavefront, expected):
-    """The caller's wavefront size bounds the samples in flight, and with them the memory of a handle
-    (vertices of 96 B, three per path vertex, and the connections); the image does not depend on it.
-    A sample's FP64 sum is rounded to FP32 once, in whatever order its connections arrive."""
-    w, h, spp, depth = 97, 65, 5, 8
+def _sample_bytes(depth):
+    """Workspace of a sample: three vertices of 96 B per path vertex, its connections, its sums."""
+    return 3 * 96 * (depth + 1) + 4 * depth * (depth + 1) // 2 + 32
+
+
+@pytest.mark.parametrize("depth,wavefront,expected", [
+    (16, 0, 1 << 18), (8, 0, (_sample_bytes(16) << 18) // _sample_bytes(8)), (2, 0, 1 << 20), (2, 1 << 21, 1 << 20),
+    (8, 20001, 20001), (8, 1, 1 << 13)])
+def test_gpu_bdpt_wavefront_paths_bound_the_workspace(gpu_lib, depth, wavefront, expected):
+    """The samples in flight: what 2^18 take at depth 16, up to 2^20, or the caller's wavefront size,
+    which bounds a handle's memory; the image does not depend on it.  A sample's FP64 sum is rounded to
+    FP32 once, in whatever order its connections arrive."""
+    w, h, spp = 97, 65, 5
 
     def render(paths):
         p = _params(w, h, depth)
@@ -146,6 +153,6 @@ def test_gpu_bdpt_wavefront_paths_bound_the_workspace(gpu_lib, wavefront, expect
             return rgb, r.stats()
     rgb, st = render(wavefront)
     assert st["wavefront_paths"] == expected
-    assert st["state_bytes"] < expected * (3 * 96 * (depth + 1) + 4 * depth * (depth + 1) // 2 + 32) + 4096
+    assert st["state_bytes"] < expected * _sample_bytes(depth) + 4096
     ref, _ = render(0)
     np.testing.assert_allclose(rgb, ref, rtol=spp * 2.0 ** -23, atol=1e-12)
