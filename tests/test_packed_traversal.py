@@ -45,3 +45,12 @@ def test_packed_traversal_spills_its_stack(program):
     assert val("max_stack") > val("lds_stack")
     for k in ("closest_diff", "prim_diff", "anyhit_diff"):
         assert val(k) == 0, k
+
+
+def test_packed_traversal_with_spheres(program):
+    """Sphere records (stored unpermuted, hit distances in FP64) among the triangles."""
+    val = run(program, 60, 0.0, 40000, "spheres")
+    assert val("box_errors") == 0 and val("layout_errors") == 0
+    assert val("sphere_hits") > 50
+    for k in ("closest_diff", "prim_diff", "anyhit_diff"):
+        assert val(k) == 0, k
