@@ -2097,7 +2097,10 @@ __global__ void k_guide_pdf_at(DeviceScene sc, int64_t n, const float *pos, cons
 // connection's MIS weight takes a dozen FP64 operations instead of a product per strategy.  As one
 // kernel with private arrays (5.9 KB of scratch per lane, 232 registers, 23 % of the lanes active, 72
 // % of the wave cycles waiting) 262,144 samples of the Cornell box took 4.75 ms; these
-// take 0.51 + 0.79 + 0.03 ms.
+// take 0.55 + 0.63 + 0.01 ms (0.54 + 0.78 + 0.03 with the connections listed sample by sample, the camera
+// vertex and each subpath's last one kept in memory and a thread and six atomics per sample at the end,
+// which made frames of short paths slower than the one kernel: 1 M samples of a lit wall 0.77 ms against
+// 0.55, now 0.47).
 enum { kBvCamera = 0, kBvSurf = 1, kBvArea = 2, kBvEnv = 3, kBvPoint = 4 };
 
 struct BdptVertex {
@@ -2141,6 +2144,16 @@ __device__ __forceinline__ void bdpt_store(const BdptWork &w, int kind, int k, u
   }
   r[4] = v.beta;
   r[5] = pack_doubles(v.prod, v.sum);
+}
+// The eye subpath's first vertex is the same for every sample, and not kept in memory.
+__device__ __forceinline__ BdptVertex bdpt_camera(const DeviceScene &sc) {
+  BdptVertex v{};
+  v.type = kBvCamera;
+  v.h.pos = sc.cam.pos;
+  v.beta = f4((float)kStrata);
+  v.pdf_walk = 1.f;
+  v.prod = 1.;
+  return v;
 }
 __device__ __forceinline__ void bdpt_unpack_geometry(const float4 *r, BdptVertex &v) {
   const float4 a = r[0], b = r[1];
@@ -2361,7 +2374,7 @@ __device__ int bv_walk(const BdptCtx &c, const BdptWork &w, uint32_t s, BdptVert
       v.sum = kLight && !light_delta && !cur.delta ? 1. : 0.;
     }
     v.prod = cur.prod * v.pdf_walk;
-    if (v.type == kBvSurf) bdpt_store(w, kKind, n, s, v);
+    if (v.type == kBvSurf && n + 1 < w.max_nodes) bdpt_store(w, kKind, n, s, v);  // the last vertex connects to nothing
     if constexpr (!kLight) {
       float4 Le = f4(0.f);
       float p_start = 0.f, p_emit = 0.f;
@@ -2432,13 +2445,7 @@ __global__ void __launch_bounds__(kTraceBlock) k_bdpt_walk(DeviceScene sc, BdptW
     float4 acc = f4(0.f);
     // eye subpath
     {
-      BdptVertex v{};
-      v.type = kBvCamera;
-      v.h.pos = sc.cam.pos;
-      v.beta = f4((float)kStrata);
-      v.pdf_walk = 1.f;
-      v.prod = 1.;
-      bdpt_store(w, kBdptEye, 0, s, v);
+      const BdptVertex v = bdpt_camera(sc);
       const int px = pixel % sc.cam.width, py = pixel / sc.cam.width;
       const float r0 = rng.uniform(), r1 = rng.uniform();
       float3 dir;
@@ -2508,23 +2515,27 @@ __global__ void __launch_bounds__(kTraceBlock) k_bdpt_walk(DeviceScene sc, BdptW
     w.acc[3 * (size_t)s + 1] = rgb.y;
     w.acc[3 * (size_t)s + 2] = rgb.z;
   }
-  // The wave's connections, listed with one atomic.
-  uint32_t at = num;
-  const int lane = (int)(threadIdx.x & 63);
+  // The wave's connections, listed with one atomic and by strategy, so that the lanes of a connection wave
+  // load neighbouring samples' vertices and mostly agree in what they evaluate.
+  uint32_t total = num, longest = (uint32_t)ne;
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t x = __shfl_up(at, o);
-    at += lane >= o ? x : 0u;
+  for (int o = 32; o > 0; o >>= 1) {
+    total += __shfl_xor(total, o);
+    longest = max(longest, (uint32_t)__shfl_xor(longest, o));
   }
-  uint32_t base = 0;
-  if (lane == 63 && at) base = atomicAdd(w.count, at);
-  at = __shfl(base, 63) + at - num;
-  if (s < count) {
-    for (int e = 0; e < ne && e + 1 < w.max_nodes; ++e) {
-      if ((directs >> e) & 1u) w.pairs[at++] = s | ((uint32_t)e << 20) | 0u;
-      const int lmax = min(nl, w.max_nodes - e - 1);
-      for (int l = 1; l < lmax; ++l) w.pairs[at++] = s | ((uint32_t)e << 20) | ((uint32_t)l << 25);
-    }
+  if (total) {
+    const int lane = (int)(threadIdx.x & 63);
+    uint32_t at = 0;
+    if (lane == 0) at = atomicAdd(w.count, total);
+    at = __shfl(at, 0);
+    const uint64_t below = (1ull << lane) - 1ull;
+    for (int e = 0; e < (int)longest && e + 1 < w.max_nodes; ++e)
+      for (int l = 0; l < w.max_nodes - e - 1; ++l) {
+        const bool mine = l == 0 ? ((directs >> e) & 1u) != 0 : e < ne && l < nl;
+        const uint64_t lanes = __ballot(mine);
+        if (mine) w.pairs[at + (uint32_t)__popcll(lanes & below)] = s | ((uint32_t)e << 20) | ((uint32_t)l << 25);
+        at += (uint32_t)__popcll(lanes);
+      }
   }
   wave_stat(stats + kStatClosest, rays);
 }
@@ -2541,7 +2552,8 @@ __global__ void __launch_bounds__(kTraceBlock) k_bdpt_connect(DeviceScene sc, Bd
     const uint2 info = w.info[s];
     const BdptCtx c{sc, info.x, as_float((int)info.y), false, 1.f / (float)npix};
     BdptVertex a, b;
-    bdpt_load(w, kBdptEye, e, s, a);
+    if (e == 0) a = bdpt_camera(sc);
+    else bdpt_load(w, kBdptEye, e, s, a);
     if (l == 0) bdpt_load(w, kBdptDirect, e, s, b);
     else bdpt_load(w, kBdptLight, l, s, b);
     float3 org, dir;
@@ -2591,11 +2603,11 @@ __global__ void __launch_bounds__(kTraceBlock) k_bdpt_connect(DeviceScene sc, Bd
     const double mine = sq((e >= 1 ? inv : 1.) * a.prod * b.prod);
     double den = mine;
     if (e >= 1) {
-      BdptVertex p;
-      const float4 *row = bdpt_row(w, kBdptEye, e - 1, s);
-      bdpt_unpack_geometry(row, p);
-      const float4 m = row[5];
+      BdptVertex p = bdpt_camera(sc);
       if (e >= 2) {
+        const float4 *row = bdpt_row(w, kBdptEye, e - 1, s);
+        bdpt_unpack_geometry(row, p);
+        p.prod = unpack_double(row[5].x, row[5].y);
         // a.sum is zero for e < 2: no strategy connects before the first scatter vertex.
         pa_rev = bv_scatter_pdf(c, a, dir, -a.wi, false);
         float3 o2, d2;
@@ -2603,7 +2615,7 @@ __global__ void __launch_bounds__(kTraceBlock) k_bdpt_connect(DeviceScene sc, Bd
         bv_segment(c, a, p, o2, d2, l2);
         den += a.sum * sq((double)pa_rev * bv_conv(a, p, d2, l2) * pl_a * b.prod);
       }
-      if (!p.delta) den += sq((e >= 2 ? inv : 1.) * unpack_double(m.x, m.y) * pl_a * b.prod);
+      if (!p.delta) den += sq((e >= 2 ? inv : 1.) * p.prod * pl_a * b.prod);
     }
     if (l >= 1) {
       BdptVertex p;
@@ -2638,16 +2650,32 @@ __global__ void __launch_bounds__(kTraceBlock) k_bdpt_connect(DeviceScene sc, Bd
   wave_stat(stats + kStatClosest, rays);
 }
 
+// Adds the samples to their pixels: with kPerPixel one thread per pixel of the chunk, without atomics,
+// else one thread per sample.
+template <bool kPerPixel>
 __global__ void __launch_bounds__(256) k_bdpt_finish(BdptWork w, uint64_t first, uint32_t count, uint32_t npix, double *fb, double *fb_sq) {
-  const uint32_t s = gtid();
-  if (s == 0) *w.count = 0;
-  if (s >= count) return;
-  const uint32_t pixel = (uint32_t)((first + s) % npix);
+  const uint32_t k = gtid();
+  if (k == 0) *w.count = 0;
+  if (k >= min(count, kPerPixel ? npix : count)) return;
+  const size_t pixel = (size_t)((first + k) % npix);
+  double sum[3] = {0., 0., 0.}, sum_sq[3] = {0., 0., 0.};
+  for (uint32_t s = k; s < count; s += kPerPixel ? npix : count) {
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const double v = (double)(float)w.acc[3 * (size_t)s + k];
-    atomicAdd(fb + 3 * (size_t)pixel + k, v);
-    if (fb_sq) atomicAdd(fb_sq + 3 * (size_t)pixel + k, v * v);
+    for (int c = 0; c < 3; ++c) {
+      const double v = (double)(float)w.acc[3 * (size_t)s + c];
+      sum[c] += v;
+      sum_sq[c] += v * v;
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    if (kPerPixel) {
+      fb[3 * pixel + c] += sum[c];
+      if (fb_sq) fb_sq[3 * pixel + c] += sum_sq[c];
+    } else {
+      atomicAdd(fb + 3 * pixel + c, sum[c]);
+      if (fb_sq) atomicAdd(fb_sq + 3 * pixel + c, sum_sq[c]);
+    }
   }
 }
 
@@ -2748,7 +2776,13 @@ void LaunchBdpt(const DeviceScene &sc, const BdptWork &w, uint64_t first, uint32
   hipLaunchKernelGGL(k_bdpt_walk, dim3((count + kTraceBlock - 1) / kTraceBlock), dim3(kTraceBlock), 0, st, sc, w, first, count, npix, spp_base,
                      seed, stats);
   hipLaunchKernelGGL(k_bdpt_connect, dim3(Blocks((uint64_t)count * 8, kTraceBlock, 16384)), dim3(kTraceBlock), 0, st, sc, w, npix, fb, stats);
-  hipLaunchKernelGGL(k_bdpt_finish, dim3((count + 255) / 256), dim3(256), 0, st, w, first, count, npix, fb, fb_sq);
+  // A pixel's samples one after the other (0.5 us each) against atomics on rows that others add to as well
+  // (0.1 us per thousand samples): equal near 5000 pixels, whatever the chunk.  2^20 samples on 512 x
+  // 512 pixels 11 / 107 us, 128 x 128: 35 / 110, 64 x 64: 131 / 117, 16 x 16: 1853 / 271.
+  const bool per_pixel = npix >= (1u << 13);
+  const uint32_t threads = per_pixel ? std::min(count, npix) : count;
+  hipLaunchKernelGGL(per_pixel ? k_bdpt_finish<true> : k_bdpt_finish<false>, dim3((threads + 255) / 256), dim3(256), 0, st, w, first, count,
+                     npix, fb, fb_sq);
 }
 void LaunchCameraConnect(const DeviceScene &sc, uint64_t first, uint64_t count, uint32_t npix, uint32_t spp_base, uint64_t seed,
                          double *fb, double *fb_sq, uint32_t *stats, hipStream_t st) {

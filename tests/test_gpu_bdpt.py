@@ -108,10 +108,12 @@ def test_gpu_bdpt_rejects_unsupported(gpu_lib):
         GpuRenderer(s, _params(8, 8, 8))
 
 
-@pytest.mark.parametrize("w,h,spp,depth", [(1, 1, 3, 2), (13, 7, 5, 16), (257, 511, 3, 16), (641, 421, 4, 3)])
+@pytest.mark.parametrize("w,h,spp,depth", [(1, 1, 3, 2), (13, 7, 5, 16), (91, 90, 4, 3), (128, 64, 4, 3), (257, 511, 3, 16),
+                                              (641, 421, 4, 3)])
 def test_gpu_bdpt_chunks_and_wave_edges(gpu_lib, w, h, spp, depth):
-    """One pass (the last two span two chunks, of 2^18 and 2^20 samples, and end inside a wave) equals the sum
-    of 1-spp passes: each sample draws the same numbers wherever it lies in a chunk.  A sample's sum
+    """One pass (the last two span two chunks, of 2^18 and 2^20 samples, and end inside a wave) equals
+    the sum of 1-spp passes: each sample draws the same numbers wherever it lies in a chunk.  Frames of
+    8190 pixels take their samples by atomics, of 8192 and more by a thread per pixel.  A sample's sum
     runs over at most 136 connections in another order, in FP64, and is rounded to FP32 once."""
     scene = configs.cornell_box(w, h)
 
@@ -119,14 +121,15 @@ def test_gpu_bdpt_chunks_and_wave_edges(gpu_lib, w, h, spp, depth):
         with GpuRenderer(scene, _params(w, h, depth)) as r:
             for n in passes:
                 r.render_spp(n)
-            rgb, _, n = r.framebuffer()
-            return rgb, n, r.stats()["paths_traced"]
-    a, na, pa = render([spp])
-    b, nb, pb = render([1] * spp)
+            rgb, sq, n = r.framebuffer()
+            return rgb, sq, n, r.stats()["paths_traced"]
+    a, a2, na, pa = render([spp])
+    b, b2, nb, pb = render([1] * spp)
     assert np.all(na == spp) and np.array_equal(na, nb) and pa == pb == w * h * spp
     if w > 100:
         assert a.sum() > 0
     np.testing.assert_allclose(a, b, rtol=spp * 2.0 ** -23, atol=1e-12)
+    np.testing.assert_allclose(a2, b2, rtol=spp * 2.0 ** -22, atol=1e-12)
 
 
 def _sample_bytes(depth):
