@@ -297,11 +297,6 @@ struct SlotPlan {
   unsigned long long sample0;
   uint32_t pixel0, refill;
 };
-// Progress record of an iteration, written by the device into page-locked host memory: camera
-// paths issued, work queued for the next iteration, and the iteration's number (written last).
-struct PassProgress {
-  unsigned long long issued, queued, seq;
-};
 // End of a pass, written by the device into page-locked host memory.
 struct PassReport {
   uint32_t counters[kNumCounters];

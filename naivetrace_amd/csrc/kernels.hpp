@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include "device_scene.hpp"
 #include "nn.hpp"
+#include "pass_progress.hpp"
 
 namespace ttgpu {
 

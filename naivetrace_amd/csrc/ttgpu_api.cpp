@@ -15,6 +15,7 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/ttgpu.h"
@@ -115,6 +116,7 @@ struct ttgpu_handle {
     PassProgress poll[2];
     PassReport report;
   } *pinned = nullptr, *pinned_dev = nullptr;
+  ProgressRecords progress;
   int npix = 0;
   uint32_t capacity = 0;
   // host copies needed later
@@ -810,9 +812,11 @@ void AllocateQueues(ttgpu_handle *h) {
   }
   q.progress = h->Alloc<unsigned long long>(2);
   Check(hipMemset(q.progress, 0, 2 * sizeof(unsigned long long)), "hipMemset progress");
-  Check(hipHostMalloc((void **)&h->pinned, sizeof(*h->pinned)), "hipHostMalloc");
+  // Coherent: the host reads the progress while the device runs.
+  Check(hipHostMalloc((void **)&h->pinned, sizeof(*h->pinned), hipHostMallocMapped | hipHostMallocCoherent), "hipHostMalloc");
   Check(hipHostGetDevicePointer((void **)&h->pinned_dev, h->pinned, 0), "hipHostGetDevicePointer");
   *h->pinned = {};
+  h->progress.Attach(h->pinned->poll, h->pinned_dev->poll);
   q.shadow_in = q.shadow_out = q.counters + kCountShadow;
   if (h->dsc.has_media) {
     q.wt_r = h->Alloc<float4>(N);
@@ -1311,18 +1315,24 @@ void CheckReport(const ttgpu_handle *h) {
 }
 
 // Waits until iteration `seq` has reported its progress.  The stream's state bounds the wait: once
-// it has run dry (or failed) no report is on its way.
-const PassProgress &WaitProgress(ttgpu_handle *h, int slot, unsigned long long seq) {
-  const PassProgress &r = h->pinned->poll[slot];
-  for (unsigned spins = 1; __atomic_load_n(&r.seq, __ATOMIC_ACQUIRE) != seq; ++spins) {
-    __builtin_ia32_pause();
-    if (spins % 8192 != 0) continue;
+// it has run dry (or failed) no report is on its way.  Short iterations are polled; one that takes longer
+// leaves the core to others, 20 us at a time, while the iteration queued behind it keeps the GPU busy.
+const PassProgress &WaitProgress(ttgpu_handle *h, unsigned long long seq) {
+  constexpr unsigned kSpins = 8192;  // 0.1 to 0.4 ms, by the processor
+  for (unsigned spins = 1; !h->progress.Arrived(seq); ++spins) {
+    if (spins < kSpins) {
+      __builtin_ia32_pause();
+      continue;
+    }
     const hipError_t e = hipStreamQuery(h->stream);
-    if (e == hipErrorNotReady) continue;
-    Check(e, "hipStreamQuery");
-    if (__atomic_load_n(&r.seq, __ATOMIC_ACQUIRE) != seq) throw std::runtime_error("no progress report from the device (internal error)");
+    if (e != hipErrorNotReady) {
+      Check(e, "hipStreamQuery");
+      if (!h->progress.Arrived(seq)) throw std::runtime_error("no progress report from the device (internal error)");
+      break;
+    }
+    std::this_thread::sleep_for(std::chrono::microseconds(20));
   }
-  return r;
+  return h->progress.Record(seq);
 }
 
 void ResetFramebuffer(ttgpu_handle *h) {
@@ -1405,10 +1415,10 @@ bool RenderPass(ttgpu_handle *h, int spp) {
   const bool shadow_in_trace = ShadowInTrace(h->dsc, q);
   const bool slot_order = q.alive != nullptr;
   if (!slot_order) shadow_in = shadow_out;
-  h->pinned->poll[0] = h->pinned->poll[1] = PassProgress{n0, n0, 0};
   // Every queue holds at most the pass's n0 slots; once all paths are issued, at most the work
   // the last known iteration left (the launches' grids; their kernels stride over any count).
   uint32_t bound = n0;
+  uint64_t issued = n0;  // as of the last iteration that has reported
   for (uint64_t it = 0;; ++it) {
     if (it > max_iter) throw std::runtime_error("path regeneration did not drain (internal error)");
     if (!stopped && h->stop.load()) {
@@ -1430,10 +1440,10 @@ bool RenderPass(ttgpu_handle *h, int spp) {
     }
     h->Timed("shade", [&] { LaunchShade(h->dsc, q, cur_q, cur_c, nxt_q, nxt_c, bound, h->fb, h->fb_sq, h->stream); });
     if (!shadow_in_trace) h->Timed("shadow", [&] { LaunchShadow(h->dsc, q, bound, h->fb, h->fb_sq, h->stream); });
-    const int slot = (int)(it & 1);
+    const unsigned long long seq = h->progress.Next();
     h->Timed("raygen", [&] {
       LaunchRegen(h->dsc, q,
-                  RegenArgs{nxt_q, nxt_c, n0, limit, (uint32_t)npix, spp_base, h->params.seed, shadow_in_trace, &h->pinned_dev->poll[slot], it + 1,
+                  RegenArgs{nxt_q, nxt_c, n0, limit, (uint32_t)npix, spp_base, h->params.seed, shadow_in_trace, h->progress.Device(seq), seq,
                             h->select_temp},
                   h->stream);
     });
@@ -1448,12 +1458,12 @@ bool RenderPass(ttgpu_handle *h, int spp) {
     // Wait for the previous iteration (this one is already queued behind it): an empty queue after
     // regeneration means every issued path has finished and none is left to issue.
     if (it > 0) {
-      const PassProgress &r = WaitProgress(h, 1 - slot, it);
+      const PassProgress &r = WaitProgress(h, seq - 1);
+      issued = r.issued;
       if (r.queued == 0) break;
       if (r.issued >= limit) bound = (uint32_t)std::min<uint64_t>(n0, r.queued);
     }
   }
-  const uint64_t issued = std::max(h->pinned->poll[0].issued, h->pinned->poll[1].issued);
   const bool complete = issued == total;
   // pt: the light connection at the camera node of every issued camera sample.
   if (h->dsc.algo_pt && h->dsc.sample_mode != TTGPU_SAMPLE_BSDF && h->dsc.cam.kind == TTGPU_CAMERA_PINHOLE)
