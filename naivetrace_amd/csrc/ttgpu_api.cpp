@@ -23,6 +23,7 @@
 #include "device_scene.hpp"
 #include "guide_fit.hpp"
 #include "guiding.hpp"
+#include "idle_stages.hpp"
 #include "kernels.hpp"
 #include "media.hpp"
 #include "scene_file.hpp"
@@ -1500,10 +1501,12 @@ bool RenderPass(ttgpu_handle *h, int spp) {
 // The caller's rays are copied in chunks into page-locked slots; a kernel takes a slot's rays to
 // the device, and the trace writes the results into the slot.  The slots' streams overlap, so the
 // host copies one chunk while the GPU fetches and traces others.  With seven hipMalloc / hipFree
-// pairs and seven copies of pageable arrays per call, a million closest-hit rays took 3.0 ms, of
-// which 0.35 were tracing; now 1.9 ms, bound by the host's copies and the link (occlusion: 1.66 and
-// 1.45 ms).  Chunks of 2^16 or 2^15 rays were slower (launches; 3.75 and 5.3 ms for both queries
-// against 3.65), and tracing straight from the page-locked rays took 5.2 ms.
+// pairs and seven copies of pageable arrays per call, a million closest-hit rays of the 1 M triangle
+// terrain took 2.6 ms, of which 0.35 were tracing; now 1.9 ms, bound by the host's copies and the link
+// (occlusion: 1.6 and 1.5 ms), and 200,000 took 0.66 ms, now 0.50.  Six slots of 2^16 rays, which take the
+// same memory: 1.79 and 1.51 ms for a million, but 0.52 (occlusion 0.45 against 0.40) for 200,000; four
+// of 2^16: 2.0 and 1.76 ms; twelve of 2^15: 2.2 and 2.0.  Tracing straight from the page-locked rays took
+// 5.2 ms for both queries instead of 3.65.
 constexpr int kStageSlots = 3;
 constexpr size_t kStageRays = 1 << 17;                // of a slot at most: 2048 waves, 5.8 MB
 constexpr size_t kMinStageRays = 1 << 10;
@@ -1528,10 +1531,10 @@ struct RayStage {
   }
 };
 // Stages are shared by the process's handles (a query borrows one, so queries of several threads
-// each have their own); at most kMaxIdleStages are kept, and none after the last handle.
-constexpr size_t kMaxIdleStages = 4;
+// each have their own; small ones leave the stages of several slots to the large); at most kMaxIdleStages are kept, and none after the last handle.
+constexpr int kMaxIdleStages = 4;
 std::mutex g_stage_mu;
-std::vector<RayStage> g_idle_stages;
+IdleStages<RayStage, kMaxIdleStages> g_idle_stages;
 int g_handles = 0;
 
 // A stage for `count` rays: one slot of at least that many, or kStageSlots of kStageRays.
@@ -1543,12 +1546,8 @@ RayStage BorrowStage(size_t count) {
   while (s.slot_rays < std::min(count, kStageRays)) s.slot_rays *= 2;
   {
     std::lock_guard<std::mutex> lock(g_stage_mu);
-    for (size_t k = 0; k < g_idle_stages.size(); ++k) {
-      const RayStage idle = g_idle_stages[k];
-      if (idle.device != s.device || idle.slots < s.slots || idle.slot_rays < s.slot_rays) continue;
-      g_idle_stages.erase(g_idle_stages.begin() + k);
-      return idle;
-    }
+    const RayStage idle = g_idle_stages.Take(s);
+    if (idle.slots) return idle;
   }
   try {
     const size_t rays = s.slots * s.slot_rays;
@@ -1566,30 +1565,21 @@ RayStage BorrowStage(size_t count) {
   }
   return s;
 }
-void ReturnStage(RayStage s) {
+void ReturnStage(RayStage s) noexcept {
   {
     std::lock_guard<std::mutex> lock(g_stage_mu);
-    if (g_handles > 0) {
-      g_idle_stages.push_back(s);
-      if (g_idle_stages.size() <= kMaxIdleStages) return;
-      // The smallest goes.
-      auto small = std::min_element(g_idle_stages.begin(), g_idle_stages.end(), [](const RayStage &a, const RayStage &b) {
-        return a.slots * a.slot_rays < b.slots * b.slot_rays;
-      });
-      s = *small;
-      g_idle_stages.erase(small);
-    }
+    if (g_handles > 0) s = g_idle_stages.Put(s);
   }
-  s.Free();
+  if (s.slots) s.Free();
 }
-void CountHandle(int d) {
-  std::vector<RayStage> drop;
+void CountHandle(int d) noexcept {
+  IdleStages<RayStage, kMaxIdleStages> drop;
   {
     std::lock_guard<std::mutex> lock(g_stage_mu);
     g_handles += d;
-    if (g_handles == 0) drop.swap(g_idle_stages);
+    if (g_handles == 0) std::swap(drop, g_idle_stages);
   }
-  for (auto &s : drop) s.Free();
+  for (RayStage s = drop.Drop(); s.slots; s = drop.Drop()) s.Free();
 }
 
 // Closest hits (t, prim, u, v) or, with `occluded`, occlusion of `count` rays.
