@@ -146,19 +146,18 @@ def test_cornell_parity_sorted_shade(gpu_lib, monkeypatch):
                                                                             sky=(256, 128)))
 
 
-@pytest.mark.parametrize("persistent,shadow_in_trace,slot_order", [("1", "1", "1"), ("1", "0", "1"), ("0", "0", "1"), ("0", "1", "0")])
-def test_traversal_modes_render_the_same_image(gpu_lib, monkeypatch, persistent, shadow_in_trace, slot_order):
-    """Persistent traversal, separate shadow launches and queues appended per block instead of
-    selected in slot order give the default mode's image (one ray per thread, shadow rays in the
-    next closest-hit launch, slot-ordered queues) up to the order of the FP64 framebuffer sums:
-    every path draws the same random numbers whichever kernel traces it, in whatever order."""
+@pytest.mark.parametrize("shadow_in_trace,slot_order", [("0", "1"), ("1", "0"), ("0", "0")])
+def test_traversal_modes_render_the_same_image(gpu_lib, monkeypatch, shadow_in_trace, slot_order):
+    """Separate shadow launches and queues appended per block instead of selected in slot order give
+    the default mode's image (shadow rays in the next closest-hit launch, slot-ordered queues) up to
+    the order of the FP64 framebuffer sums: every path draws the same random numbers whichever kernel
+    traces it, in whatever order."""
     def render():
         s = configs.terrain_instances(48, 32, cells=32, n_spheres=24, freq=3, sky=(256, 128))
         with GpuRenderer(s, abi.default_params(48, 32, spp=16, max_depth=8, seed=5)) as r:
             r.run()
             return r.mean_image()
     base = render()
-    monkeypatch.setenv("TTGPU_PERSISTENT_TRAVERSAL", persistent)
     monkeypatch.setenv("TTGPU_SHADOW_IN_TRACE", shadow_in_trace)
     monkeypatch.setenv("TTGPU_SLOT_ORDER", slot_order)
     other = render()
