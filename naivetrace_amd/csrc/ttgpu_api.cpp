@@ -799,12 +799,14 @@ void AllocateQueues(ttgpu_handle *h) {
   q.queue_a = h->Alloc<uint32_t>(N); q.queue_b = h->Alloc<uint32_t>(N); q.shadow_queue = h->Alloc<uint32_t>(N);
   q.counters = h->Alloc<uint32_t>(kNumCounters);
   Check(hipMemset(q.counters, 0, kNumCounters * sizeof(uint32_t)), "hipMemset counters");
-  q.free_slots = h->Alloc<uint32_t>(N);
   // Slot-ordered queues (the next queue selected from per-slot alive flags, in ascending slot
   // order) unless TTGPU_SLOT_ORDER=0 (continuing paths appended per block).
   const char *so = std::getenv("TTGPU_SLOT_ORDER");
   q.alive = q.freed = nullptr;
-  if (!(so && so[0] == '0')) {
+  q.free_slots = nullptr;
+  if (so && so[0] == '0') {
+    q.free_slots = h->Alloc<uint32_t>(N);
+  } else {
     q.alive = h->Alloc<uint8_t>(N);
     q.freed = h->Alloc<uint8_t>(N);
     Check(hipMemset(q.alive, 0, N), "hipMemset alive flags");
