@@ -23,22 +23,17 @@ struct BuiltBvh {
 // SAH with 32 bins per axis, leaves of at most `max_leaf` primitives.
 BuiltBvh BuildBvh(const std::vector<BuildPrim> &prims, int max_leaf = 4, int num_threads = 0);
 
-// 4-wide BVH collapsed from a BVH2 (device layout Bvh4Node, 32 words per node): every node takes
-// its BVH2 node's two children and then opens the inner child of largest surface area until it has
-// four.  Leaves keep the BVH2's primitive ranges (same leaf order).
+// 4-wide BVH collapsed from a BVH2: every node takes its BVH2 node's two children and then opens the
+// inner child of largest surface area until it has four.  Leaves keep the BVH2's primitive ranges (same
+// leaf order).  32 words per node: rows of four (one word per child) of lo.x, hi.x, lo.y, hi.y, lo.z,
+// hi.z, then the children (>= 0 inner node, < 0 leaf ~first primitive) and their leaves' primitive
+// counts (0 with a leaf: empty slot, planes at infinity).
 struct BuiltBvh4 {
   std::vector<float> nodes;      // 32 * num_nodes
   int num_nodes = 0;
   int max_depth = 0;             // depth of the deepest node (root = 0)
 };
 BuiltBvh4 CollapseToBvh4(const BuiltBvh &b2);
-
-// The same tree with 8-bit child planes (device layout QBvh4Node, 16 words per node): per node and
-// axis a grid origin (the lowest child plane) and a power-of-two step chosen so that 255 steps span
-// the children; lower planes round down and upper planes up, each checked after the decode the
-// device performs, so every decoded child box contains the true one.  Empty slots (leaf, count 0)
-// get q = 0.  Throws if a leaf holds more than 255 primitives or an extent exceeds 255 x 2^127.
-std::vector<uint32_t> QuantizeBvh4(const BuiltBvh4 &b4);
 
 // The tree as the device traverses it (device layout TravNode, 16 words per node): inner children of
 // a node consecutive and in its first slots, the primitives of its leaves consecutive.  Planes are

@@ -28,32 +28,8 @@ struct alignas(16) BvhNode {
   int4 ch;      // left, right: >= 0 inner node, < 0 leaf ~first_prim; z/w: prim counts of leaves
 };
 
-// BVH4 node of the surface BVH, 128 bytes: the bounds of all four children in the parent
-// (structure of arrays, one float4 row per bound), so one fetch decides all four.  Empty slots
-// have bounds at +infinity.
-struct alignas(16) Bvh4Node {
-  float4 lox, hix, loy, hiy, loz, hiz;
-  int4 child;   // >= 0: inner node; < 0: leaf ~first primitive
-  int4 count;   // primitives of a leaf child
-};
-
-// Quantized BVH4 node, 64 bytes (two per 128-byte cache line).  The children's planes are
-// 8-bit offsets on a per-node grid: plane = origin_k + q * 2^(e_k - 127), q in [0, 255], with
-// the host choosing q so that every decoded box contains its child's true box (the product
-// q * 2^e is exact, so the decode rounds once, identically on host and device).
-//   origin : xyz = grid origin (lo corner of the union of the children), w = exponent bytes e_x, e_y, e_z
-//   qxy    : lo.x, hi.x, lo.y, hi.y rows, byte c = child c
-//   qz     : lo.z, hi.z rows, then the four leaf counts (byte c = child c), then 0
-//   child  : >= 0 inner node; < 0 leaf ~first primitive (count 0: empty slot)
-struct alignas(64) QBvh4Node {
-  float4 origin;
-  uint4 qxy;
-  uint4 qz;
-  int4 child;
-};
-
-// Traversal node of the surface BVH, 64 bytes: the quantized BVH4 laid out for few instructions per
-// visit.  A node's inner children are consecutive nodes and take its first slots, so that child
+// Traversal node of the surface BVH, 64 bytes (two per 128-byte cache line): four children whose boxes
+// have 8-bit planes on a per-node grid, laid out for few instructions per visit.  A node's inner children are consecutive nodes and take its first slots, so that child
 // slot c is node child_base + c; the primitives of its leaves are consecutive too, so that the
 // leaves a ray enters are one bit mask.
 //   origin : xyz = grid origin, w = the grid steps' exponents (signed bytes x, y, z)
@@ -69,7 +45,6 @@ struct alignas(64) TravNode {
   int child_base, prim_base;
   uint4 leaf;
 };
-using SurfNode = TravNode;
 
 constexpr int kStackEntries = 96;                   // traversal stack entries per lane
 // A BVH4 node pushes at most three children, so a tree of depth D needs 3 (D + 1) entries.
@@ -171,7 +146,7 @@ struct QuadCell {
 };
 
 struct DeviceScene {
-  const SurfNode *nodes;           // surface BVH
+  const TravNode *nodes;           // surface BVH
   const PrimRecord *prims;         // leaf order
   // Three copies of prims for traversal, in the order of the nodes' primitive ranges: copy k holds
   // each triangle's vertex coordinates in the order ((k+1) mod 3, (k+2) mod 3, k), the frame of the

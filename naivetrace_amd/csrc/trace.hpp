@@ -204,236 +204,8 @@ TT_HD void box2(const BvhNode &n, const RayPre &p, float tmax, float &tl, float 
   tr = rmin <= rmax ? rmin : as_float(0x7f800000);
 }
 
-// ---- BVH4 traversal of the intermediate layouts (run on the host by the checks of the BVH build) --
-// A ray's traversal state; one step is one node visit or one primitive test, so the loop below
-// and the persistent kernels with dynamic ray fetch (Aila & Laine 2009) share the same code.
-// `cur` holds the node to visit next and `rec` the primitive to test next, both already fetched:
-// each step issues the fetch its successor step needs, so memory latency overlaps the tests.
-template <class Node>
-struct TravT {
-  RayPre p;
-  float3 org, dir;
-  float tmax;
-  HitRec hit;
-  int sp;
-  Node cur;             // next node to visit, already fetched (valid when has_node)
-  bool has_node;
-  int leaf_first;       // primitive to test next (valid while leaf_left > 0)
-  int leaf_left;        // primitives left in the current leaf
-  int pend[3];          // further leaves of the same node: first << 3 | count
-  int npend;
-  PrimRecord rec;       // the record of leaf_first, already fetched
-  int kofs;             // p.kz x the number of primitives: this ray's copy of the records
-  bool any;             // any-hit query: finished at the first hit
-};
-
-template <class Node>
-TT_HD void trav_init(TravT<Node> &t, const Ray &r, const Node *__restrict__ nodes, int num_prims, bool any_hit = false) {
-  t.any = any_hit;
-  t.p = precompute(r);
-  t.kofs = t.p.kz * num_prims;
-  t.org = r.org;
-  t.dir = r.dir;
-  t.tmax = r.tmax;
-  t.hit.prim = -1;
-  t.sp = 0;
-  t.cur = nodes[0];
-  t.has_node = true;
-  t.leaf_left = 0;
-  t.npend = 0;
-}
-
-// Slab test of the four children; entry distances, +inf when missed.  The planes the ray enters
-// and leaves by are picked per axis by the direction's sign, once per node.
-TT_HD void box4(const Bvh4Node &n, const RayPre &p, float tmax, float t[4]) {
-  const float4 nx4 = p.negx ? n.hix : n.lox, fx4 = p.negx ? n.lox : n.hix;
-  const float4 ny4 = p.negy ? n.hiy : n.loy, fy4 = p.negy ? n.loy : n.hiy;
-  const float4 nz4 = p.negz ? n.hiz : n.loz, fz4 = p.negz ? n.loz : n.hiz;
-  const float nx[4] = {nx4.x, nx4.y, nx4.z, nx4.w}, fx[4] = {fx4.x, fx4.y, fx4.z, fx4.w};
-  const float ny[4] = {ny4.x, ny4.y, ny4.z, ny4.w}, fy[4] = {fy4.x, fy4.y, fy4.z, fy4.w};
-  const float nz[4] = {nz4.x, nz4.y, nz4.z, nz4.w}, fz[4] = {fz4.x, fz4.y, fz4.z, fz4.w};
-  // Conservative far bound (1 + 2 gamma(3)) so grazing hits are not lost (Ize 2013).
-  const float pad = 1.0000004f;
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const float tn = fmaxf(fmaxf(nx[c] * p.inv.x - p.onear.x, ny[c] * p.inv.y - p.onear.y), fmaxf(nz[c] * p.inv.z - p.onear.z, 0.f));
-    const float tf = fminf(fminf(fx[c] * p.inv.x - p.ofar.x, fy[c] * p.inv.y - p.ofar.y), fminf(fz[c] * p.inv.z - p.ofar.z, tmax)) * pad;
-    t[c] = tn <= tf ? tn : as_float(0x7f800000);
-  }
-}
-
-TT_HD void node_counts(const Bvh4Node &n, int count[4]) {
-  count[0] = n.count.x; count[1] = n.count.y; count[2] = n.count.z; count[3] = n.count.w;
-}
-
-// Quantized node: each plane decodes as fma(q, 2^(e - 127), origin) -- exact product, one
-// rounding, the value the host checked to enclose the child -- and then enters the same slab test
-// as a full-precision plane.
-TT_HD float qplane(uint32_t row, int c, float scale, float origin) {
-  return fmaf((float)((row >> (8 * c)) & 0xffu), scale, origin);
-}
-
-TT_HD void box4(const QBvh4Node &n, const RayPre &p, float tmax, float t[4]) {
-  const uint32_t e = as_uint(n.origin.w);
-  const float sx = as_float((e & 0xffu) << 23), sy = as_float(((e >> 8) & 0xffu) << 23), sz = as_float(((e >> 16) & 0xffu) << 23);
-  // Rows of the planes the ray enters and leaves by, per axis.
-  const uint32_t nx = p.negx ? n.qxy.y : n.qxy.x, fx = p.negx ? n.qxy.x : n.qxy.y;
-  const uint32_t ny = p.negy ? n.qxy.w : n.qxy.z, fy = p.negy ? n.qxy.z : n.qxy.w;
-  const uint32_t nz = p.negz ? n.qz.y : n.qz.x, fz = p.negz ? n.qz.x : n.qz.y;
-  const float pad = 1.0000004f;
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const float tn = fmaxf(fmaxf(qplane(nx, c, sx, n.origin.x) * p.inv.x - p.onear.x, qplane(ny, c, sy, n.origin.y) * p.inv.y - p.onear.y),
-                           fmaxf(qplane(nz, c, sz, n.origin.z) * p.inv.z - p.onear.z, 0.f));
-    const float tf = fminf(fminf(qplane(fx, c, sx, n.origin.x) * p.inv.x - p.ofar.x, qplane(fy, c, sy, n.origin.y) * p.inv.y - p.ofar.y),
-                           fminf(qplane(fz, c, sz, n.origin.z) * p.inv.z - p.ofar.z, tmax)) * pad;
-    t[c] = tn <= tf ? tn : as_float(0x7f800000);
-  }
-}
-
-TT_HD void node_counts(const QBvh4Node &n, int count[4]) {
-#pragma unroll
-  for (int c = 0; c < 4; ++c) count[c] = (int)((n.qz.z >> (8 * c)) & 0xffu);
-}
-
-// One iteration of a ray's traversal: either one node step or one primitive test, so the lanes of
-// a wave that are testing primitives and those that are visiting nodes advance together instead of
-// the whole wave waiting for the lane with the most primitives in its node's leaves.
-//   node step: slab test of the four children of the (prefetched) node; inner children ordered by
-//     entry distance with a five-comparator network, the nearest visited next and the others pushed
-//     far to near; the successor's fetch is issued; the leaves the ray enters are queued (the first
-//     one's record fetched) to be tested one primitive per iteration.
-//   primitive step: tests the fetched record and fetches the next one of the queued leaves.
-// Returns false when the traversal is finished (no queued primitive and no node left, or an
-// occluder found for any-hit queries: kAnyHit, or the state's `any` flag).  Queued leaves are not culled against a hit found after
-// they were queued: the primitive test rejects what lies beyond it.  `stack` is this lane's LDS
-// column (stride kTraceBlock), `spill` its private overflow; the host bounds the tree depth so
-// that the kStackEntries entries always suffice (a push that finds the stack full is dropped and
-// reported through TTGPU_STACK_OVERFLOW); leaves hold at most 7 primitives (the host
-// builds leaves of at most 4) and primitive indices stay below 2^28.
-template <bool kAnyHit, class Node>
-TT_HD bool trav_step(TravT<Node> &t, const Node *nodes, const PrimRecord *prims, int *stack, int *spill) {
-  if (t.leaf_left > 0) {
-    const PrimRecord cur = t.rec;
-    const int cur_id = t.leaf_first;
-    ++t.leaf_first;
-    --t.leaf_left;
-    {
-      // Next queued leaf when this one is done (selects, not branches).
-      const bool adv = t.leaf_left == 0 && t.npend > 0;
-      const int e = t.pend[0];
-      t.pend[0] = adv ? t.pend[1] : t.pend[0];
-      t.pend[1] = adv ? t.pend[2] : t.pend[1];
-      t.npend -= adv ? 1 : 0;
-      t.leaf_first = adv ? e >> 3 : t.leaf_first;
-      t.leaf_left = adv ? e & 7 : t.leaf_left;
-    }
-    if (t.leaf_left > 0) t.rec = prims[t.kofs + t.leaf_first];
-#if defined(__HIP_DEVICE_COMPILE__)
-    // Keeps the compiler from sinking the fetch below the test it should overlap.
-    asm volatile("" ::: "memory");
-#endif
-    Ray r;
-    r.org = t.org;
-    r.dir = t.dir;
-    float th, u, v;
-    if (intersect_prim_k(cur, t.p, r, t.tmax, th, u, v)) {
-      t.tmax = th;
-      t.hit.t = th; t.hit.u = u; t.hit.v = v; t.hit.prim = cur_id;
-      if (kAnyHit || t.any) return false;
-    }
-    return t.leaf_left > 0 || t.has_node;
-  }
-  if (!t.has_node) return false;
-  float tc[4];
-  box4(t.cur, t.p, t.tmax, tc);
-  const int child[4] = {t.cur.child.x, t.cur.child.y, t.cur.child.z, t.cur.child.w};
-  int count[4];
-  node_counts(t.cur, count);
-  float key[4];
-  int id[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const bool inner = child[c] >= 0 && tc[c] <= t.tmax;
-    key[c] = inner ? tc[c] : as_float(0x7f800000);
-    id[c] = inner ? child[c] : -1;
-  }
-  // Sort the (at most four) inner children by entry distance: five compare-exchanges.
-#define TT_CSWAP(a, b)                                                                  \
-  if (key[b] < key[a]) {                                                               \
-    const float kt = key[a]; key[a] = key[b]; key[b] = kt;                             \
-    const int it = id[a]; id[a] = id[b]; id[b] = it;                                   \
-  }
-  TT_CSWAP(0, 1) TT_CSWAP(2, 3) TT_CSWAP(0, 2) TT_CSWAP(1, 3) TT_CSWAP(1, 2)
-#undef TT_CSWAP
-  // The inner children are id[0 .. n-1] (the misses sort last, with key +inf); id[0] is visited
-  // next and id[n-1] .. id[1] are pushed.
-  int next = id[0];
-  if (t.sp + 3 <= kLdsStack) {
-    // All three writes land in the LDS part: each writes at the top and only a child moves it, so
-    // an absent child's write is overwritten or left above the top.
-#pragma unroll
-    for (int c = 3; c >= 1; --c) {
-      stack[t.sp * kTraceBlock] = id[c];
-      t.sp += id[c] >= 0 ? 1 : 0;
-    }
-  } else {
-#pragma unroll
-    for (int c = 3; c >= 1; --c) {
-      if (id[c] < 0) continue;
-      if (t.sp < kLdsStack) stack[t.sp * kTraceBlock] = id[c];
-      else if (t.sp < kStackEntries) spill[t.sp - kLdsStack] = id[c];
-      if (t.sp < kStackEntries) ++t.sp;
-      else TTGPU_STACK_OVERFLOW();
-    }
-  }
-  if (next < 0 && t.sp > 0) {
-    --t.sp;
-    // An LDS read (the top's entry, or the last LDS entry when the top lies in the spill part)
-    // rather than one generic load through a selected address space.
-    next = stack[min(t.sp, kLdsStack - 1) * kTraceBlock];
-    if (t.sp >= kLdsStack) next = spill[t.sp - kLdsStack];
-  }
-  // Queue the leaves the ray enters, in child order: each entered leaf, from the last child to
-  // the first, is put in front of the list L0..L3 (entries first << 3 | count, all positive).
-  int L0 = 0, L1 = 0, L2 = 0, L3 = 0, nl = 0;
-#pragma unroll
-  for (int c = 3; c >= 0; --c) {
-    const bool ok = child[c] < 0 && count[c] != 0 && tc[c] <= t.tmax;
-    const int e = (int)(((uint32_t)~child[c] << 3) | (uint32_t)count[c]);
-    L3 = ok ? L2 : L3;
-    L2 = ok ? L1 : L2;
-    L1 = ok ? L0 : L1;
-    L0 = ok ? e : L0;
-    nl += ok ? 1 : 0;
-  }
-  // The node step runs with no leaf left, so leaf_left stays 0 when no leaf is entered.
-  t.leaf_first = L0 >> 3;
-  t.leaf_left = L0 & 7;
-  t.pend[0] = L1;
-  t.pend[1] = L2;
-  t.pend[2] = L3;
-  t.npend = nl > 1 ? nl - 1 : 0;
-  if (nl > 0) t.rec = prims[t.kofs + t.leaf_first];
-  t.has_node = next >= 0;
-  t.cur = nodes[next < 0 ? 0 : next];
-  return t.has_node || t.leaf_left > 0;
-}
-
-// Whole traversal of one ray (closest hit, or any hit with kAnyHit); true if something was hit.
-template <bool kAnyHit, class Node>
-TT_HD bool traverse(const Node *__restrict__ nodes, const PrimRecord *__restrict__ prims, int num_prims, const Ray &r,
-                    int *stack, HitRec &hit) {
-  int spill[kSpillStack];
-  TravT<Node> t;
-  trav_init(t, r, nodes, num_prims);
-  while (trav_step<kAnyHit>(t, nodes, prims, stack, spill)) {}
-  hit = t.hit;
-  return t.hit.prim >= 0;
-}
-
 // ---- traversal of the packed nodes ------------------------------------------------------------
-// Issue-bound as one ray per lane with the intermediate layout (VALU work in 95-100 % of SIMD cycles,
+// Issue-bound as one ray per lane with nodes of decoded 8-bit planes (VALU work in 95-100 % of SIMD cycles,
 // 5.4e8 instructions per launch of the 1080p benchmark): what counted was instructions per step times
 // the steps a wave makes, which its busiest lanes set.  Now 2.9e8 instructions, VALU busy 78 % and the
 // vector-memory return path 80 % (a scattered 16-byte load of 32 lanes takes 30 cycles of it, so a
@@ -443,7 +215,7 @@ TT_HD bool traverse(const Node *__restrict__ nodes, const PrimRecord *__restrict
 //    per-node constants); entry distances carry the slot in their low two bits, so sorting the four
 //    is five integer min / max pairs and a child's index one addition; entered leaves are bits of
 //    one mask.  A node step is 173 VALU instructions, with the decoded planes, compare-and-swap pairs
-//    and leaf list of the intermediate layout it was 233.
+//    and leaf list of such nodes it was 233.
 //  * one kind of step per iteration.  Lanes with primitives to test and lanes with a node to visit
 //    do not advance together: the wave takes the kind of step that more of its lanes wait for, and
 //    the others wait (their fetch is on its way meanwhile).  A model of 64-lane waves over the
