@@ -1,6 +1,7 @@
 """The two-launch slot selection (chunk counts scanned by the last block, queue and regeneration in
 one scatter) against the appended queues, at wavefront sizes around its chunk (1024 slots, 16 flags
-per lane) and block (16 chunks) edges and with passes that refill the slots several times."""
+per lane) and block (16 chunks) edges, above 2^20 slots, where each thread of the last block scans
+several chunks (two and three here), and with passes that refill the slots."""
 import numpy as np
 import pytest
 
@@ -10,9 +11,10 @@ from naivetrace_amd.renderer import GpuRenderer
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("wavefront", [1, 15, 16, 17, 1023, 1024, 1025, 16383, 16384, 16385, 33001])
+@pytest.mark.parametrize("wavefront", [1, 15, 16, 17, 1023, 1024, 1025, 16383, 16384, 16385, 33001, (1 << 20) + 1,
+                                       (1 << 21) + 1025])
 def test_slot_selection_renders_the_appended_queues_image(gpu_lib, monkeypatch, wavefront):
-    w, h = (5, 3) if wavefront < 1000 else (97, 61)
+    w, h = (5, 3) if wavefront < 1000 else (97, 61) if wavefront < 1 << 20 else (640, 512)
     spp = 3 if wavefront < 1000 else 8
 
     def render():
