@@ -988,23 +988,29 @@ __global__ void __launch_bounds__(kTraceBlock, TTGPU_TRACE_WAVES) k_shadow(Devic
 // wavelength weights / pixel count added to that pixel.  With TTGPU_MIS_REFERENCE the pixel index
 // truncates toward zero as the reference does.
 //
-// The light's image is a few hundred pixels that every sample hits, so six FP64 atomics per sample
-// on them bound the kernel: 1.88 ms for 4.2 M samples of the 512 x 512 Cornell box (780 pixels), 0.23
+// Every sample hits the light's image, a few hundred to a few thousand pixels, so six FP64 atomics per
+// sample on them bound the kernel: 1.88 ms for 4.2 M samples of the 512 x 512 Cornell box (780 pixels), 0.23
 // without them.  Each block sums its samples in an LDS table of kConnectSlots pixels and adds each
-// slot once at its end: 0.32 ms.  A pixel that finds no slot in kConnectProbes goes to memory as
-// before; those are what a small table pays for (512 slots and two probes: 0.82 ms).  LDS holds the
-// table and the traversal stacks, which leaves one block per CU; 1024 threads with 1024 slots took
-// 0.29 ms but cover half the pixels.
-constexpr int kConnectBlock = 512, kConnectBits = 11, kConnectSlots = 1 << kConnectBits, kConnectProbes = 16, kConnectBlocks = 256;
+// slot once at its end: 0.27 ms.  A pixel that finds no slot in kConnectProbes goes to memory as
+// before; those are what a small table pays for (512 slots and two probes: 0.82 ms; with 1024 slots
+// instead of 2048 images of 1750 and 3100 pixels, 768^2 and 1024^2 x 4 spp: 0.55 and 1.35 ms instead of
+// 0.28 and 0.78; larger images gain little, 2048^2 x 4 spp 4.9 ms against 5.3 without a table).  In a
+// large scene the traversal bounds the kernel, and one block per CU, which is what LDS admits, has to
+// hold all the waves that the registers allow: 1024 threads, whose stacks keep 13 entries in LDS and
+// the rest in private memory.  With 512 threads and 24 entries a light over the 1 M triangle terrain
+// (960 x 540 x 8 spp) took 0.81 ms, now 0.58 (0.53 without the table).  More than 256 blocks only add
+// tables to sum: Cornell box 0.36 ms with 512.
+constexpr int kConnectBlock = 1024, kConnectBits = 11, kConnectSlots = 1 << kConnectBits, kConnectProbes = 16, kConnectBlocks = 256;
+constexpr int kConnectStack = 13;  // traversal stack entries in LDS
 
 __global__ void __launch_bounds__(kConnectBlock) k_camera_connect(DeviceScene sc, uint64_t first, uint64_t count, uint32_t npix,
                                                                    uint32_t spp_base, uint64_t seed, double *fb, double *fb_sq,
                                                                    uint32_t *stats) {
   static_assert(kConnectBlock % kTraceBlock == 0, "stack columns are laid out per kTraceBlock threads");
-  __shared__ int lds_stack[kLdsStack * kConnectBlock];
+  __shared__ int lds_stack[kConnectStack * kConnectBlock];
   __shared__ uint32_t s_pixel[kConnectSlots];  // pixel + 1, 0: free
   __shared__ double s_sum[6][kConnectSlots];
-  int *stack = lds_stack + (threadIdx.x / kTraceBlock) * (kLdsStack * kTraceBlock) + threadIdx.x % kTraceBlock;
+  int *stack = lds_stack + (threadIdx.x / kTraceBlock) * (kConnectStack * kTraceBlock) + threadIdx.x % kTraceBlock;
   for (int k = threadIdx.x; k < kConnectSlots; k += kConnectBlock) {
     s_pixel[k] = 0;
 #pragma unroll
@@ -1049,7 +1055,7 @@ __global__ void __launch_bounds__(kConnectBlock) k_camera_connect(DeviceScene sc
     r.tmax = ls.len * 0.9999f;
     HitRec hr;
     ++rays;
-    if (traverse<true>(sc.nodes, sc.prims_kz, sc.num_prims, r, stack, hr)) continue;
+    if (traverse<true, kConnectStack>(sc.nodes, sc.prims_kz, sc.num_prims, r, stack, hr)) continue;
     const uint32_t p = (uint32_t)((size_t)iy * c.width + (size_t)ix);
     const double v[6] = {(double)crgb.x, (double)crgb.y, (double)crgb.z, (double)crgb.x * crgb.x, (double)crgb.y * crgb.y,
                          (double)crgb.z * crgb.z};

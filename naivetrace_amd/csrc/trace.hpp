@@ -289,7 +289,9 @@ TT_HD void trav_prim(Trav &t, const PrimRecord *prims) {
 }
 
 // Node step: slab test of the four children; inner children sorted by entry distance, the nearest
-// visited next and the others pushed far to near; the mask of the entered leaves' primitives.
+// visited next and the others pushed far to near; the mask of the entered leaves' primitives.  The first
+// kLds stack entries are in LDS.
+template <int kLds>
 TT_HD void trav_node(Trav &t, const TravNode *nodes, int *stack, int *spill) {
   const TravNode n = nodes[t.node];
   const uint32_t e = as_uint(n.origin.w);
@@ -323,7 +325,7 @@ TT_HD void trav_node(Trav &t, const TravNode *nodes, int *stack, int *spill) {
   sort2(key[1], key[3]);
   sort2(key[1], key[2]);
   const int base = n.child_base;
-  if (t.sp + 3 * kTraceBlock <= kLdsStack * kTraceBlock) {
+  if (t.sp + 3 * kTraceBlock <= kLds * kTraceBlock) {
     // All three writes land in the LDS part: each writes at the top and only a child moves it, so
     // an absent child's write is overwritten or left above the top.
 #pragma unroll
@@ -336,8 +338,8 @@ TT_HD void trav_node(Trav &t, const TravNode *nodes, int *stack, int *spill) {
     for (int c = 3; c >= 1; --c) {
       if ((int)key[c] < 0) continue;
       const int id = base + (int)(key[c] & 3u), k = t.sp / kTraceBlock;
-      if (k < kLdsStack) stack[t.sp] = id;
-      else if (k < kStackEntries) spill[k - kLdsStack] = id;
+      if (k < kLds) stack[t.sp] = id;
+      else if (k < kStackEntries) spill[k - kLds] = id;
       if (k < kStackEntries) t.sp += kTraceBlock;
       else TTGPU_STACK_OVERFLOW();
     }
@@ -348,8 +350,8 @@ TT_HD void trav_node(Trav &t, const TravNode *nodes, int *stack, int *spill) {
     // An LDS read (the top's entry, or the last LDS entry when the top lies in the spill part)
     // rather than one generic load through a selected address space.
     const int top = t.sp;
-    next = stack[top < (kLdsStack - 1) * kTraceBlock ? top : (kLdsStack - 1) * kTraceBlock];
-    if (top >= kLdsStack * kTraceBlock) next = spill[top / kTraceBlock - kLdsStack];
+    next = stack[top < (kLds - 1) * kTraceBlock ? top : (kLds - 1) * kTraceBlock];
+    if (top >= kLds * kTraceBlock) next = spill[top / kTraceBlock - kLds];
   }
   t.pmask = mask & 0x7fffffffu;
   t.pbase = t.kofs + n.prim_base;
@@ -357,6 +359,7 @@ TT_HD void trav_node(Trav &t, const TravNode *nodes, int *stack, int *spill) {
 }
 
 // One iteration of the wave: the kind of step more of its lanes wait for.
+template <int kLds = kLdsStack>
 TT_HD void trav_advance(Trav &t, const TravNode *nodes, const PrimRecord *prims, int *stack, int *spill) {
   const bool wp = t.wants_prim(), wn = t.wants_node();
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -365,20 +368,20 @@ TT_HD void trav_advance(Trav &t, const TravNode *nodes, const PrimRecord *prims,
   const bool take_node = wn;
 #endif
   if (take_node) {
-    if (wn) trav_node(t, nodes, stack, spill);
+    if (wn) trav_node<kLds>(t, nodes, stack, spill);
   } else {
     if (wp) trav_prim(t, prims);
   }
 }
 
 // Whole traversal of one ray (closest hit, or any hit with kAnyHit); true if something was hit.
-template <bool kAnyHit>
+template <bool kAnyHit, int kLds = kLdsStack>
 TT_HD bool traverse(const TravNode *__restrict__ nodes, const PrimRecord *__restrict__ prims, int num_prims, const Ray &r, int *stack,
                     HitRec &hit) {
-  int spill[kSpillStack];
+  int spill[kStackEntries - kLds];
   Trav t;
   trav_init(t, r, num_prims, kAnyHit, stack);
-  while (t.active()) trav_advance(t, nodes, prims, stack, spill);
+  while (t.active()) trav_advance<kLds>(t, nodes, prims, stack, spill);
   hit = t.hit;
   return t.hit.prim >= 0;
 }

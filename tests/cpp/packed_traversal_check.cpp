@@ -78,7 +78,7 @@ int main(int argc, char **argv) {
   }
   for (int k = 0; k < n; ++k) bad_layout += seen[k] != 1;
   std::vector<int> stack(kLdsStack * kTraceBlock);
-  long diff = 0, any_diff = 0, prim_diff = 0, full_diff = 0, checked = 0, hits = 0, sphere_hits = 0;
+  long diff = 0, any_diff = 0, prim_diff = 0, full_diff = 0, short_diff = 0, checked = 0, hits = 0, sphere_hits = 0;
   int max_sp = 0;
   const int every = (n <= 2000 || teeth) ? 1 : 16;
   for (int r = 0; r < rays; ++r) {
@@ -121,6 +121,11 @@ int main(int argc, char **argv) {
       hq = t.hit;
     }
     const bool oq = traverse<true>(qn, tree.per_axis.data(), n, ray, stack.data(), aq);
+    // The camera connections keep fewer stack entries in LDS.
+    HitRec hs, as;
+    traverse<false, 13>(qn, tree.per_axis.data(), n, ray, stack.data(), hs);
+    const bool os = traverse<true, 13>(qn, tree.per_axis.data(), n, ray, stack.data(), as);
+    short_diff += hs.prim != hq.prim || (hq.prim >= 0 && hs.t != hq.t) || os != oq;
     float best, full;
     const int bi = brute_force(tree, ray, best), fi = float_planes(tree, ray, full);
     checked++;
@@ -135,8 +140,8 @@ int main(int argc, char **argv) {
     any_diff += oq != (bi >= 0);
   }
   printf("prims %d nodes %d depth %d box_errors %ld layout_errors %ld rays %ld hits %ld sphere_hits %ld closest_diff %ld prim_diff %ld "
-         "anyhit_diff %ld full_closest_diff %ld max_stack %d lds_stack %d overflows %ld\n",
-         n, pk.num_nodes, tree.b4.max_depth, bad_box, bad_layout, checked, hits, sphere_hits, diff, prim_diff, any_diff, full_diff, max_sp,
-         kLdsStack, g_overflows);
+         "anyhit_diff %ld full_closest_diff %ld short_stack_diff %ld max_stack %d lds_stack %d overflows %ld\n",
+         n, pk.num_nodes, tree.b4.max_depth, bad_box, bad_layout, checked, hits, sphere_hits, diff, prim_diff, any_diff, full_diff, short_diff,
+         max_sp, kLdsStack, g_overflows);
   return (bad_box || bad_layout || g_overflows) ? 1 : 0;
 }

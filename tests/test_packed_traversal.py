@@ -36,14 +36,14 @@ def test_packed_traversal_matches_brute_force(program, grid, offset, rays):
     val = run(program, grid, offset, rays)
     assert val("box_errors") == 0 and val("layout_errors") == 0
     assert val("hits") > (10 if grid < 7 else 300)
-    for k in ("closest_diff", "prim_diff", "anyhit_diff"):
+    for k in ("closest_diff", "prim_diff", "anyhit_diff", "short_stack_diff"):
         assert val(k) == 0, k
 
 
 def test_packed_traversal_spills_its_stack(program):
     val = run(program, 400, 0.0, 300, "comb")
     assert val("max_stack") > val("lds_stack")
-    for k in ("closest_diff", "prim_diff", "anyhit_diff"):
+    for k in ("closest_diff", "prim_diff", "anyhit_diff", "short_stack_diff"):
         assert val(k) == 0, k
 
 
@@ -52,5 +52,5 @@ def test_packed_traversal_with_spheres(program):
     val = run(program, 60, 0.0, 40000, "spheres")
     assert val("box_errors") == 0 and val("layout_errors") == 0
     assert val("sphere_hits") > 50
-    for k in ("closest_diff", "prim_diff", "anyhit_diff"):
+    for k in ("closest_diff", "prim_diff", "anyhit_diff", "short_stack_diff"):
         assert val(k) == 0, k
