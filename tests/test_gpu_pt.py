@@ -99,12 +99,12 @@ def test_gpu_pt_rejects_media(gpu_lib):
         GpuRenderer(fog_furnace_scene(0.5), _params(4, 4, 8, abi.SAMPLE_BOTH, abi.MIS_CONSISTENT))
 
 
-@pytest.mark.parametrize("w,h,spp", [(7, 5, 2), (45, 45, 3), (46, 45, 3), (96, 64, 4), (31, 29, 300), (97, 65, 512)])
+@pytest.mark.parametrize("w,h,spp", [(7, 5, 2), (45, 45, 3), (46, 45, 3), (96, 64, 4), (31, 29, 600), (97, 65, 512)])
 def test_camera_connections_through_the_pixel_table(gpu_lib, w, h, spp):
     """Light points connected to the camera, with an emitter that fills the view.  One pass equals the sum
     of 1-spp passes up to the order of the FP64 sums (at most a thousand positive terms on a pixel:
-    1e-12), and the squared sums do too.  A 1-spp pass gives each block at most 512 samples, one per
-    thread, so its table of 2048 slots never fills.  In one pass the last two sizes give a block 1.1 and
+    1e-12), and the squared sums do too.  A 1-spp pass gives each block at most 1024 samples, one per
+    thread, so its table of 2048 slots never fills.  In one pass the last two sizes give a block 2.1 and
     12.6 thousand samples: several per thread (pixel and sample advanced by the grid's stride, which
     neither frame's size divides), and, of 6305 pixels, three times what the table holds, so that most
     samples find no slot and go to memory."""
