@@ -1318,22 +1318,27 @@ void CheckReport(const ttgpu_handle *h) {
 }
 
 // Waits until iteration `seq` has reported its progress.  The stream's state bounds the wait: once
-// it has run dry (or failed) no report is on its way.  Short iterations are polled; one that takes longer
-// leaves the core to others, 20 us at a time, while the iteration queued behind it keeps the GPU busy.
-const PassProgress &WaitProgress(ttgpu_handle *h, unsigned long long seq) {
+// it has run dry (or failed) no report is on its way.  The wait polls, but where the one before was long
+// too (`was_long`, kept over a pass), so that the iteration queued behind this one keeps the GPU busy, it
+// leaves the core to others 20 us at a time.  (A wait may be long only because of the work queued before
+// the pass: sleeping in it left the GPU idle, 0.4 ms per training sweep of the quadtree guide.)
+const PassProgress &WaitProgress(ttgpu_handle *h, unsigned long long seq, bool &was_long) {
   constexpr unsigned kSpins = 8192;  // 0.1 to 0.4 ms, by the processor
+  const bool sleep = was_long;
+  was_long = false;
   for (unsigned spins = 1; !h->progress.Arrived(seq); ++spins) {
-    if (spins < kSpins) {
+    if (spins % kSpins != 0 && !(sleep && was_long)) {
       __builtin_ia32_pause();
       continue;
     }
+    was_long = true;
     const hipError_t e = hipStreamQuery(h->stream);
     if (e != hipErrorNotReady) {
       Check(e, "hipStreamQuery");
       if (!h->progress.Arrived(seq)) throw std::runtime_error("no progress report from the device (internal error)");
       break;
     }
-    std::this_thread::sleep_for(std::chrono::microseconds(20));
+    if (sleep) std::this_thread::sleep_for(std::chrono::microseconds(20));
   }
   return h->progress.Record(seq);
 }
@@ -1422,6 +1427,7 @@ bool RenderPass(ttgpu_handle *h, int spp) {
   // the last known iteration left (the launches' grids; their kernels stride over any count).
   uint32_t bound = n0;
   uint64_t issued = n0;  // as of the last iteration that has reported
+  bool was_long = false;
   for (uint64_t it = 0;; ++it) {
     if (it > max_iter) throw std::runtime_error("path regeneration did not drain (internal error)");
     if (!stopped && h->stop.load()) {
@@ -1461,7 +1467,7 @@ bool RenderPass(ttgpu_handle *h, int spp) {
     // Wait for the previous iteration (this one is already queued behind it): an empty queue after
     // regeneration means every issued path has finished and none is left to issue.
     if (it > 0) {
-      const PassProgress &r = WaitProgress(h, seq - 1);
+      const PassProgress &r = WaitProgress(h, seq - 1, was_long);
       issued = r.issued;
       if (r.queued == 0) break;
       if (r.issued >= limit) bound = (uint32_t)std::min<uint64_t>(n0, r.queued);
