@@ -208,7 +208,7 @@ TT_HD void box2(const BvhNode &n, const RayPre &p, float tmax, float &tl, float 
 // Issue-bound as one ray per lane with nodes of decoded 8-bit planes (VALU work in 95-100 % of SIMD cycles,
 // 5.4e8 instructions per launch of the 1080p benchmark): what counted was instructions per step times
 // the steps a wave makes, which its busiest lanes set.  Now 2.9e8 instructions, VALU busy 78 % and the
-// vector-memory return path 80 % (a scattered 16-byte load of 32 lanes takes 30 cycles of it, so a
+// vector-memory return path 84 % (a scattered 16-byte load of 32 lanes takes 30 cycles of it, so a
 // node step's four take 120 of the 173 x 4 its arithmetic takes on each of the four SIMDs).  Three
 // things keep both low:
 //  * the packed layout.  Child boxes take two instructions per plane (byte to float, fma onto
